@@ -123,6 +123,8 @@ bool router_takes_lookup(uint32_t hidden, uint32_t experts, uint32_t batch, cons
 hipError_t launch_fill_u32(hipStream_t s, uint32_t *p, uint32_t n, uint32_t value);
 // Per-token counters of the fused router selection (zero between launches).
 constexpr uint32_t kRouterTickets = 4096;
+// Words of the fp16 matvec's K-split meeting places (4 MiB).
+constexpr uint32_t kQmvMeetWords = 512 * 1024;
 hipError_t launch_rms_norm(hipStream_t s, const float *in, uint32_t batch, uint32_t n,
                            const float *weight, float eps, float *out);
 hipError_t launch_silu_mul(hipStream_t s, const float *gate, const float *up, size_t n, float *out);

@@ -1,19 +1,21 @@
-// kernels_qmv.hip -- MFMA quantized matvec for gfx950 (decode, batch 1..16).
+// kernels_qmv.hip -- fp16-MFMA quantized matvec for gfx950 (decode, the
+// batches of up to 16 tokens the int8 kernels do not take).
 //
 // y[b][r] = sum_c W[r][c] * x[b][c] for Q4_K / Q6_K rows (src/cpu.rs:345-399
 // semantics, fp32 accumulation).
 //
 // Operands of v_mfma_f32_16x16x32_f16, all exact:
-//  * B (weights): 16 rows x 32 columns per step.  Each weight enters as the
-//    fp16 integer sc*q (Q4_K: 0..945) or sc*(q-32) (Q6_K: |.| <= 1984 when
-//    |sc| <= 62), built from the packed bits with the "1024 + q" exponent
-//    trick and one packed fp16 FMA (exact: the result is representable and
-//    the FMA rounds once).  The super-block scale d (and dmin) multiply the
-//    fp32 block result afterwards.  Q6_K blocks with a larger |sc| split the
-//    scale into 8*sh + sl and run two exact MFMAs.
-//  * A (activations): 16 rows = 8 tokens x {hi, lo}.  Each token is scaled
-//    by a power of two so |x| < 2^15, then x = hi + lo with hi, lo fp16
-//    (22 significant bits).  Products are exact; MFMA accumulates in fp32.
+//  * B (weights): 16 rows x 32 columns per step.  A Q4_K weight enters as the
+//    fp16 integer sc*q (0..945), built from the packed bits with the
+//    "1024 + q" exponent trick and one packed fp16 FMA (exact: the result is
+//    representable and the FMA rounds once).  Q6_K's sc*(q-32) needs up to 13
+//    bits: the scale is split into 8*sh + sl and sh*(q-32) and sl*(q-32),
+//    both exact, go to an MFMA each.  The super-block scale d (and dmin)
+//    multiply the fp32 block result afterwards.
+//  * A (activations): 16 rows = 8 tokens x {hi, lo}.  Each 256-value block of
+//    a token is scaled by a power of two so |x| < 2^15, then x = hi + lo with
+//    hi, lo fp16 (22 significant bits).  Products are exact; MFMA accumulates
+//    in fp32, and the block's result is multiplied back by 2^e.
 //  * Q4_K's "- dmin * m * x" term is a ninth MFMA step per block whose B
 //    column carries 64*m and whose A row carries the sub-block sums of x
 //    (scaled by 2^-6, hi/lo), accumulated separately and scaled by dmin.
@@ -23,14 +25,7 @@
 // the lane supplies.  C[m][n] sits in lane n + 16*(m/4), element m%4, so
 // lane (n, g4) accumulates tokens 2*g4 and 2*g4+1 of row n.
 //
-// Data movement: a wave stages G = 2 consecutive blocks of each of its row
-// tiles in its own LDS area with contiguous 16-byte loads (out-of-range rows
-// read zero), the next group in flight while the current one is computed,
-// and every lane takes its pieces from there.  For batch 1-2 the activation
-// fragments of the whole row are staged once per workgroup in LDS and read
-// with ds_read_b128; for larger batches they come from L2, the next block's
-// while a block is computed.  Short matrices split K over up to 8 waves of a
-// workgroup.
+// Data movement: see qmv_kernel.
 #include "dm_device.h"
 #include "dm_qmv.h"
 
@@ -78,25 +73,9 @@ __device__ __forceinline__ half8 frag(uint32_t a, uint32_t b, uint32_t c, uint32
     return __builtin_bit_cast(half8, v);
 }
 
-// Steps of 32 columns per 256-column block, including Q4_K's min step.
-template <uint32_t TYPE> struct Steps;
-template <> struct Steps<kQ4_K> { static constexpr uint32_t value = 9; };
-template <> struct Steps<kQ6_K> { static constexpr uint32_t value = 8; };
-
-// Column (0..255) of a block that fragment position j of lane-group kg
-// carries at step t (t < 8).
-template <uint32_t TYPE>
-__device__ __forceinline__ uint32_t fragment_column(uint32_t kg, uint32_t t, uint32_t j) {
-    const uint32_t perm = (j & 3u) == 1 ? 2u : ((j & 3u) == 2 ? 1u : (j & 3u));
-    if (TYPE == kQ4_K) return 64 * kg + 32 * (j >> 2) + 4 * t + perm;
-    // Q6_K: kg = 2h + c; k = t >> 1; dw = 2 * (t & 1) + (j >> 2).
-    const uint32_t h = kg >> 1, c = kg & 1u, k = t >> 1, dw = 2 * (t & 1u) + (j >> 2);
-    return 128 * h + 32 * k + 16 * c + 4 * dw + perm;
-}
-
 // Power-of-two exponent e with max|x| * 2^-e in [2^14, 2^15) (0 for an
-// all-zero or non-finite row, whose result is then non-finite anyway).
-__device__ __forceinline__ int token_exponent(float mx) {
+// all-zero or non-finite block, whose result is then non-finite anyway).
+__device__ __forceinline__ int block_exponent(float mx) {
     int e = 0;
     if (mx > 0.0f && __builtin_isfinite(mx)) {
         int ex;
@@ -108,137 +87,62 @@ __device__ __forceinline__ int token_exponent(float mx) {
     return e;
 }
 
-// The hi/lo fp16 halves of fragment (blk, t, kg) of one token row `xt`
-// scaled by `down` (a power of two).
+// How a wave holds one block of 8 tokens' activations as loaded: value j of
+// load (u, r) (token group u of 4, round r) of lane 16 i + 4 kg + c is column
+// round_column(kg, r) + 4 c + j of token 4 u + i, so a load reads runs of 64
+// bytes.  (One 16-byte piece per lane in fragment order reads 64 lines with
+// one load: 16 waves of them took 3 us of a 6.4 us kernel.)  The quad (r, c)
+// of lane group kg belongs to step quad_step(r, c), half quad_half(r, c) of
+// the lane's 8 values.
 template <uint32_t TYPE>
-__device__ __forceinline__ void build_fragment(const float *xt, uint32_t blk, uint32_t t, uint32_t kg,
-                                               float down, half8 &hi, half8 &lo) {
-    const float *xb = xt + (size_t)blk * 256;
-    // the halves are gathered in scalars and the vectors built once (element
-    // inserts across the branch put the vectors in private memory)
-    _Float16 h[8], l[8];
-    if (TYPE == kQ4_K && t == 8) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const float *sb = xb + 32 * (2 * kg + j);
-            float q[32];
-#pragma unroll
-            for (int i = 0; i < 32; i++) q[i] = sb[i];  // every read issued before the sum
-            float s = 0.0f;
-#pragma unroll
-            for (int i = 0; i < 32; i++) s += q[i] * down;
-            s = s * 0.015625f;  // 2^-6 keeps |sum| inside fp16
-            h[j] = (_Float16)s;
-            l[j] = (_Float16)(s - (float)h[j]);
-        }
-#pragma unroll
-        for (int j = 2; j < 8; j++) h[j] = l[j] = (_Float16)0.0f;
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float v = xb[fragment_column<TYPE>(kg, t, j)] * down;
-            h[j] = (_Float16)v;
-            l[j] = (_Float16)(v - (float)h[j]);
-        }
-    }
-    hi = half8{h[0], h[1], h[2], h[3], h[4], h[5], h[6], h[7]};
-    lo = half8{l[0], l[1], l[2], l[3], l[4], l[5], l[6], l[7]};
+__device__ __forceinline__ constexpr uint32_t round_bytes() { return TYPE == kQ4_K ? 64 : 128; }  // between rounds
+template <uint32_t TYPE>
+__device__ __forceinline__ uint32_t round_column(uint32_t kg) {  // of round 0
+    return TYPE == kQ4_K ? 64 * kg : 128 * (kg >> 1) + 16 * (kg & 1u);
+}
+template <uint32_t TYPE> constexpr uint32_t quad_step(uint32_t r, uint32_t c) {
+    return TYPE == kQ4_K ? 4 * (r & 1u) + c : 2 * r + (c >> 1);
+}
+template <uint32_t TYPE> constexpr uint32_t quad_half(uint32_t r, uint32_t c) {
+    return TYPE == kQ4_K ? r >> 1 : c & 1u;
+}
+
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // x may be 4-byte aligned
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+// DPP controls.  (After the exchanges by 1 and 2 the mirrors of 8 and 16
+// lanes act as exchanges by 4 and 8.)
+constexpr int kXor1 = 0xb1, kXor2 = 0x4e, kHalfMirror = 0x141, kMirror = 0x140;
+
+__device__ __forceinline__ float row_max(float v) {  // over rows of 16 lanes
+    v = fmaxf(v, dpp<kXor1>(v));
+    v = fmaxf(v, dpp<kXor2>(v));
+    v = fmaxf(v, dpp<kHalfMirror>(v));
+    return fmaxf(v, dpp<kMirror>(v));
+}
+__device__ __forceinline__ float quad_sum(float v) {  // over groups of 4 lanes
+    v += dpp<kXor1>(v);
+    return v + dpp<kXor2>(v);
+}
+__device__ __forceinline__ float row_sum(float v) {
+    v = quad_sum(v);
+    v += dpp<kHalfMirror>(v);
+    return v + dpp<kMirror>(v);
+}
+
+// (v0, v1) as fp16 hi + lo: 22 significant bits.
+__device__ __forceinline__ void split_pair(float v0, float v1, uint32_t &hi, uint32_t &lo) {
+    const half2_t h = __builtin_convertvector(floatx2{v0, v1}, half2_t);
+    const half2_t l = __builtin_convertvector(floatx2{v0 - (float)h[0], v1 - (float)h[1]}, half2_t);
+    hi = as_u(h);
+    lo = as_u(l);
 }
 
 }  // namespace
-
-// ---------------------------------------------------------------------------
-// Activation preparation: per token a power-of-two scale 2^-e with
-// max|x| * 2^-e in [2^14, 2^15), the hi/lo fp16 fragments in step order,
-// and (Q4_K) the 32-column sums.  yscale[t] = 2^e (times the RMSNorm factor
-// when `normalize`).  Grid: (blocks of fragments, tokens).
-// ---------------------------------------------------------------------------
-// With STAGED the token row is copied into LDS (columns <= kPrepareLdsColumns)
-// and the fragments are built from there; the row is read from global memory
-// once, every load of a thread in flight at once (16-byte loads when the row
-// is 16-byte aligned).  The 32-column sums of Q4_K issue all their LDS reads
-// before the sequential sum (measured at C3, 4 tokens: 48.5 -> 46.3 us per
-// layer against one read in flight at a time).
-constexpr uint32_t kPrepareLdsColumns = 16384;
-
-template <uint32_t TYPE, bool STAGED>
-__global__ void __launch_bounds__(256) qmv_prepare_kernel(const float *__restrict__ x,
-                                                          uint32_t columns, uint32_t batch,
-                                                          int normalize, float epsilon,
-                                                          _Float16 *__restrict__ xp,
-                                                          float *__restrict__ yscale) {
-    constexpr uint32_t SPB = Steps<TYPE>::value;
-    constexpr uint32_t U = 16;
-    extern __shared__ float s_row[];
-    __shared__ float red_max[4], red_ss[4];
-    const uint32_t token = blockIdx.y;
-    const float *xt = x + (size_t)token * columns;
-    float mx = 0.0f, ss = 0.0f;
-    if (STAGED && ((uintptr_t)xt & 15u) == 0) {
-        // 16-byte loads, every one in flight at once (columns <= 16384 is 16 per thread)
-        const uint32_t n4 = columns / 4;
-        floatx4 v[U];
-#pragma unroll
-        for (uint32_t j = 0; j < U; j++) {
-            const uint32_t i = 256 * j + threadIdx.x;
-            v[j] = i < n4 ? ((const floatx4 *)xt)[i] : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < U; j++) {
-            const uint32_t i = 256 * j + threadIdx.x;
-            if (i < n4) ((floatx4 *)s_row)[i] = v[j];
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                mx = fmaxf(mx, fabsf(v[j][e]));
-                ss = __builtin_fmaf(v[j][e], v[j][e], ss);
-            }
-        }
-    } else
-    for (uint32_t i0 = 0; i0 < columns; i0 += 256 * U) {
-        float v[U];
-#pragma unroll
-        for (uint32_t j = 0; j < U; j++) {
-            const uint32_t i = i0 + 256 * j + threadIdx.x;
-            v[j] = i < columns ? xt[i] : 0.0f;
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < U; j++) {
-            const uint32_t i = i0 + 256 * j + threadIdx.x;
-            if (STAGED && i < columns) s_row[i] = v[j];
-            mx = fmaxf(mx, fabsf(v[j]));
-            ss = __builtin_fmaf(v[j], v[j], ss);
-        }
-    }
-    mx = wave_max(mx);
-    ss = wave_sum(ss);
-    if ((threadIdx.x & 63u) == 0) {
-        red_max[threadIdx.x >> 6] = mx;
-        red_ss[threadIdx.x >> 6] = ss;
-    }
-    __syncthreads();
-    mx = fmaxf(fmaxf(red_max[0], red_max[1]), fmaxf(red_max[2], red_max[3]));
-    ss = red_ss[0] + red_ss[1] + red_ss[2] + red_ss[3];
-    const int e = token_exponent(mx);
-    const float down = ldexpf(1.0f, -e);
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        float up = ldexpf(1.0f, e);
-        if (normalize) up = up * (1.0f / __builtin_sqrtf(ss / (float)columns + epsilon));
-        yscale[token] = up;
-    }
-    // One fragment (8 halves) per thread: fragment f = ((blk*SPB + t)*4 + kg).
-    const uint32_t blocks = columns / 256;
-    const uint32_t m2 = 2 * batch;
-    const uint32_t fragments = blocks * SPB * 4;
-    half8 *dst = (half8 *)xp;
-    for (uint32_t f = blockIdx.x * blockDim.x + threadIdx.x; f < fragments;
-         f += gridDim.x * blockDim.x) {
-        const uint32_t kg = f & 3u, t = (f >> 2) % SPB, blk = (f >> 2) / SPB;
-        half8 hi, lo;
-        build_fragment<TYPE>(STAGED ? s_row : xt, blk, t, kg, down, hi, lo);
-        dst[(size_t)f * m2 + 2 * token] = hi;
-        dst[(size_t)f * m2 + 2 * token + 1] = lo;
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Raw bytes of one block of one row as a lane holds them, and the block's
@@ -249,37 +153,43 @@ template <> struct Raw<kQ4_K> {
     u32x4 hdr, q0, q1;  // d|dmin|scales, then qs bytes [32kg, 32kg+32)
 };
 template <> struct Raw<kQ6_K> {
-    u32x4 a1, a2, a3, a4;          // aligned dwords under ql/ql+32/qh/scales
-    uint32_t e1, e2, e3, e4, e4b;  // the dword after each (for the byte shift)
+    u32x4 a1, a2, a3;                  // aligned dwords under ql/ql+32/qh
+    u32x2 a4;                          // and under the lane's half of the scales
+    uint32_t e1, e2, e3, e4, e4b, e5;  // the dword after each (for the byte shift); e4, e4b hold d
     uint32_t s;                    // block start mod 4
 };
 
+// (a & mask) | b: one instruction when mask and b are in registers, as the
+// callers arrange (as literals they would make it two).
+__device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t mask, uint32_t b) { return (a & mask) | b; }
+
+// The block's contribution to acc[g][j] (tokens 8 g + 2 kg + j), up[g][j] the
+// 2^e of the tokens' scaled activations.
 template <int NT>
-__device__ __forceinline__ void block_dot(const Raw<kQ4_K> &raw, const half8 (&a)[9][NT], uint32_t kg,
+__device__ __forceinline__ void block_dot(const Raw<kQ4_K> &raw, const half8 (&a)[8][NT],
+                                          const uint32_t (&amin)[NT], uint32_t kg, const float (&up)[NT][2],
                                           float (&acc)[NT][2]) {
     const u32x4 hdr = raw.hdr;
     const float dscale = f16_lo(hdr[0]);
     const float mscale = f16_lo(hdr[0] >> 16);
-    // (scale, min) of sub-blocks 2kg and 2kg+1 (src/cpu.rs:607-616): for
+    // (scale, min) bytes of sub-blocks 2kg and 2kg+1 (src/cpu.rs:607-616): for
     // sub-block j < 4 the low 6 bits of scales[j], scales[j+4]; for j >= 4
     // nibbles of scales[j+4] with the top bits of scales[j-4], scales[j].
-    const bool high_half = kg >= 2;
-    uint32_t sc[2], mn[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const uint32_t sh = 8 * ((2 * kg + j) & 3u);
-        const uint32_t b1 = hdr[1] >> sh, b2 = hdr[2] >> sh, b3 = hdr[3] >> sh;
-        const uint32_t sc_lo = b1 & 63u, mn_lo = b2 & 63u;
-        const uint32_t sc_hi = (b3 & 15u) | ((b1 >> 2) & 0x30u);
-        const uint32_t mn_hi = ((b3 >> 4) & 15u) | ((b2 >> 2) & 0x30u);
-        sc[j] = high_half ? sc_hi : sc_lo;
-        mn[j] = high_half ? mn_hi : mn_lo;
-    }
-    const half2_t sl = h2_int((int)sc[0]);
-    const half2_t bl = sl * h2_splat(-1024.0f);
-    const half2_t shi = h2_int((int)sc[1]);
+    const uint32_t sh16 = 16 * (kg & 1u);
+    const uint32_t m_low = kg < 2 ? 0x3f3fu : 0u, m_nib = kg < 2 ? 0u : 0x0f0fu, m_top = kg < 2 ? 0u : 0x3030u;
+    const uint32_t b1 = hdr[1] >> sh16, b2 = hdr[2] >> sh16, b3 = hdr[3] >> sh16;
+    const uint32_t sc = and_or(b1 >> 2, m_top, and_or(b3, m_nib, b1 & m_low));
+    const uint32_t mn = and_or(b2 >> 2, m_top, and_or(b3 >> 4, m_nib, b2 & m_low));
+    // bytes as fp16: 1024 + byte under the exponent of 1024, less 1024
+    const half2_t minus = h2_splat(-1024.0f);
+    const half2_t sl = as_h2(__builtin_amdgcn_perm(kBiasBytes, sc, 0x04000400u)) + minus;
+    const half2_t shi = as_h2(__builtin_amdgcn_perm(kBiasBytes, sc, 0x04010401u)) + minus;
+    const half2_t bl = sl * minus;
     const half2_t sh = shi * h2_splat(0.0625f);
     const half2_t bh = shi * h2_splat(-64.0f);
+    uint32_t bias = kBias16, mask_lo = 0x000f000fu, mask_hi = 0x00f000f0u;
+    asm("" : "+v"(bias));
+    asm("" : "+s"(mask_lo), "+s"(mask_hi));
     floatx4 cm[NT];
 #pragma unroll
     for (int g = 0; g < NT; g++) cm[g] = floatx4{0, 0, 0, 0};
@@ -287,134 +197,133 @@ __device__ __forceinline__ void block_dot(const Raw<kQ4_K> &raw, const half8 (&a
     for (int t = 0; t < 8; t++) {
         const uint32_t d = t < 4 ? raw.q0[t] : raw.q1[t - 4];
         const uint32_t d8 = d >> 8;
-        const uint32_t p0 = as_u(h2_fma(as_h2((d & 0x000f000fu) | kBias16), sl, bl));
-        const uint32_t p1 = as_u(h2_fma(as_h2((d8 & 0x000f000fu) | kBias16), sl, bl));
-        const uint32_t p2 = as_u(h2_fma(as_h2((d & 0x00f000f0u) | kBias16), sh, bh));
-        const uint32_t p3 = as_u(h2_fma(as_h2((d8 & 0x00f000f0u) | kBias16), sh, bh));
+        const uint32_t p0 = as_u(h2_fma(as_h2(and_or(d, mask_lo, bias)), sl, bl));
+        const uint32_t p1 = as_u(h2_fma(as_h2(and_or(d8, mask_lo, bias)), sl, bl));
+        const uint32_t p2 = as_u(h2_fma(as_h2(and_or(d, mask_hi, bias)), sh, bh));
+        const uint32_t p3 = as_u(h2_fma(as_h2(and_or(d8, mask_hi, bias)), sh, bh));
         const half8 b = frag(p0, p1, p2, p3);
 #pragma unroll
         for (int g = 0; g < NT; g++) cm[g] = mfma(a[t][g], b, cm[g]);
     }
     // min step: B = (64 m_lo, 64 m_hi, 0...), A = sub-block sums * 2^-6.
-    const uint32_t mm = (as_u(h2_int((int)(64 * mn[0]))) & 0xffffu) |
-                        (as_u(h2_int((int)(64 * mn[1]))) << 16);
-    const half8 bmin = frag(mm, 0u, 0u, 0u);
+    const half2_t m64 = (as_h2(__builtin_amdgcn_perm(kBiasBytes, mn, 0x04010400u)) + minus) * h2_splat(64.0f);
+    const half8 bmin = frag(as_u(m64), 0u, 0u, 0u);
 #pragma unroll
     for (int g = 0; g < NT; g++) {
-        const floatx4 cmin = mfma(a[8][g], bmin, floatx4{0, 0, 0, 0});
-        acc[g][0] = __builtin_fmaf(dscale, cm[g][0] + cm[g][1], acc[g][0]);
-        acc[g][0] = __builtin_fmaf(-mscale, cmin[0] + cmin[1], acc[g][0]);
-        acc[g][1] = __builtin_fmaf(dscale, cm[g][2] + cm[g][3], acc[g][1]);
-        acc[g][1] = __builtin_fmaf(-mscale, cmin[2] + cmin[3], acc[g][1]);
+        const floatx4 cmin = mfma(frag(amin[g], 0u, 0u, 0u), bmin, floatx4{0, 0, 0, 0});
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            float v = dscale * (cm[g][2 * j] + cm[g][2 * j + 1]);
+            v = __builtin_fmaf(-mscale, cmin[2 * j] + cmin[2 * j + 1], v);
+            acc[g][j] = __builtin_fmaf(up[g][j], v, acc[g][j]);
+        }
     }
 }
 
 template <int NT>
-__device__ __forceinline__ void block_dot(const Raw<kQ6_K> &raw, const half8 (&a)[8][NT], uint32_t kg,
+__device__ __forceinline__ void block_dot(const Raw<kQ6_K> &raw, const half8 (&a)[8][NT],
+                                          const uint32_t (&amin)[NT], uint32_t kg, const float (&up)[NT][2],
                                           float (&acc)[NT][2]) {
     const uint32_t s = raw.s;
     uint32_t L1[4], L2[4], H[4], T[5];
-    if (__builtin_amdgcn_ballot_w64(s != 0) == 0) {
-        // every row of the tile starts this block on a dword boundary
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            L1[i] = raw.a1[i];
-            L2[i] = raw.a2[i];
-            H[i] = raw.a3[i];
-            T[i] = raw.a4[i];
-        }
-        T[4] = raw.e4;
-    } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            L1[i] = funnel(raw.a1[i], i < 3 ? raw.a1[i + 1] : raw.e1, s);
-            L2[i] = funnel(raw.a2[i], i < 3 ? raw.a2[i + 1] : raw.e2, s);
-            H[i] = funnel(raw.a3[i], i < 3 ? raw.a3[i + 1] : raw.e3, s);
-            T[i] = funnel(raw.a4[i], i < 3 ? raw.a4[i + 1] : raw.e4, s);
-        }
-        T[4] = funnel(raw.e4, raw.e4b, s);
+    for (int i = 0; i < 4; i++) {
+        L1[i] = funnel(raw.a1[i], i < 3 ? raw.a1[i + 1] : raw.e1, s);
+        L2[i] = funnel(raw.a2[i], i < 3 ? raw.a2[i + 1] : raw.e2, s);
+        H[i] = funnel(raw.a3[i], i < 3 ? raw.a3[i + 1] : raw.e3, s);
     }
-    const float dscale = f16_lo(T[4]);
+    const float dscale = f16_lo(funnel(raw.e4, raw.e4b, s));
     // int8 scales sc[8h + 2k + c], k = 0..3: bytes c and c+2 of scale words
-    // 2h (k = 0, 1) and 2h+1 (k = 2, 3).
-    const uint32_t h = kg >> 1, c = kg & 1u;
-    const uint32_t w01 = h ? T[2] : T[0], w23 = h ? T[3] : T[1];
-    int sck[4];
-    sck[0] = (int)(int8_t)(w01 >> (8 * c));
-    sck[1] = (int)(int8_t)(w01 >> (8 * c + 16));
-    sck[2] = (int)(int8_t)(w23 >> (8 * c));
-    sck[3] = (int)(int8_t)(w23 >> (8 * c + 16));
-    bool fast = true;
+    // 2h (k = 0, 1) and 2h+1 (k = 2, 3).  sc = 8 sh + sl, sl in 0..7.
+    const uint32_t c = kg & 1u;
+    const uint32_t w01 = funnel(raw.a4[0], raw.a4[1], s) >> (8 * c), w23 = funnel(raw.a4[1], raw.e5, s) >> (8 * c);
+    floatx4 ch[NT], cl[NT];
 #pragma unroll
-    for (int k = 0; k < 4; k++) fast = fast && sck[k] <= 62 && sck[k] >= -62;
-    const bool all_fast = __builtin_amdgcn_ballot_w64(!fast) == 0;
-    floatx4 cm[NT];
+    for (int g = 0; g < NT; g++) ch[g] = cl[g] = floatx4{0, 0, 0, 0};
+    const half2_t off = h2_splat(-1056.0f);
+    uint32_t nib = 0x0f0f0f0fu, top = 0x30303030u, bytes = kBiasBytes;
+    asm("" : "+s"(nib), "+s"(top));
+    asm("" : "+v"(bytes));
 #pragma unroll
-    for (int g = 0; g < NT; g++) cm[g] = floatx4{0, 0, 0, 0};
+    for (int k = 0; k < 4; k++) {
+        const int sck = (int)(int8_t)((k < 2 ? w01 : w23) >> (16 * (k & 1)));
+        const half2_t f_hi = h2_int(sck >> 3), f_lo = h2_int(sck & 7);
+        const half2_t o_hi = f_hi * off, o_lo = f_lo * off;
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-        const int k = t >> 1;
-        uint32_t pr[4];
+        for (int t = 2 * k; t < 2 * k + 2; t++) {
+            uint32_t hi[4], lo[4];
 #pragma unroll
-        for (int half_dw = 0; half_dw < 2; half_dw++) {
-            const int dw = 2 * (t & 1) + half_dw;
-            const uint32_t src = (k & 1) ? L2[dw] : L1[dw];
-            const uint32_t nib = (k & 2) ? (src >> 4) : src;
-            // bits 2k..2k+1 of each qh byte moved to bits 4..5
-            const uint32_t hsh = k == 0 ? H[dw] << 4 : (k == 1 ? H[dw] << 2 : (k == 2 ? H[dw] : H[dw] >> 2));
-            const uint32_t q4 = (nib & 0x0f0f0f0fu) | (hsh & 0x30303030u);  // four 6-bit q
-            // fp16 pairs (1024 + q) of bytes (0, 2) and (1, 3)
-            pr[2 * half_dw] = __builtin_amdgcn_perm(q4, kBiasBytes, 0x00060004u);
-            pr[2 * half_dw + 1] = __builtin_amdgcn_perm(q4, kBiasBytes, 0x00070005u);
-        }
-        if (all_fast) {
-            const half2_t scl = h2_int(sck[k]);
-            const half2_t bias = scl * h2_splat(-1056.0f);
-            const half8 b = frag(as_u(h2_fma(as_h2(pr[0]), scl, bias)), as_u(h2_fma(as_h2(pr[1]), scl, bias)),
-                                 as_u(h2_fma(as_h2(pr[2]), scl, bias)), as_u(h2_fma(as_h2(pr[3]), scl, bias)));
-#pragma unroll
-            for (int g = 0; g < NT; g++) cm[g] = mfma(a[t][g], b, cm[g]);
-        } else {
-            // sc = 8*sh + sl, sl in 0..7: both products exact in fp16.
-            const int shi = sck[k] >> 3, slo = sck[k] & 7;
-            const half2_t off = h2_splat(-1056.0f);
-            const half2_t one = h2_splat(1.0f);
-            const half2_t f_hi = h2_int(8 * shi);
-            const half2_t f_lo = h2_int(slo);
-            half2_t qm[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) qm[i] = h2_fma(as_h2(pr[i]), one, off);  // q - 32
-            const half8 b_hi = frag(as_u(qm[0] * f_hi), as_u(qm[1] * f_hi), as_u(qm[2] * f_hi),
-                                    as_u(qm[3] * f_hi));
-            const half8 b_lo = frag(as_u(qm[0] * f_lo), as_u(qm[1] * f_lo), as_u(qm[2] * f_lo),
-                                    as_u(qm[3] * f_lo));
+            for (int half_dw = 0; half_dw < 2; half_dw++) {
+                const int dw = 2 * (t & 1) + half_dw;
+                const uint32_t src = (k & 1) ? L2[dw] : L1[dw];
+                // bits 2k..2k+1 of each qh byte moved to bits 4..5
+                const uint32_t hsh = k == 0 ? H[dw] << 4 : (k == 1 ? H[dw] << 2 : (k == 2 ? H[dw] : H[dw] >> 2));
+                const uint32_t q4 = and_or((k & 2) ? (src >> 4) : src, nib, hsh & top);  // four 6-bit q
+                // fp16 pairs (1024 + q) of bytes (0, 2) and (1, 3)
+                const half2_t p0 = as_h2(__builtin_amdgcn_perm(q4, bytes, 0x00060004u));
+                const half2_t p1 = as_h2(__builtin_amdgcn_perm(q4, bytes, 0x00070005u));
+                hi[2 * half_dw] = as_u(h2_fma(p0, f_hi, o_hi));
+                hi[2 * half_dw + 1] = as_u(h2_fma(p1, f_hi, o_hi));
+                lo[2 * half_dw] = as_u(h2_fma(p0, f_lo, o_lo));
+                lo[2 * half_dw + 1] = as_u(h2_fma(p1, f_lo, o_lo));
+            }
+            const half8 b_hi = frag(hi[0], hi[1], hi[2], hi[3]), b_lo = frag(lo[0], lo[1], lo[2], lo[3]);
 #pragma unroll
             for (int g = 0; g < NT; g++) {
-                cm[g] = mfma(a[t][g], b_hi, cm[g]);
-                cm[g] = mfma(a[t][g], b_lo, cm[g]);
+                ch[g] = mfma(a[t][g], b_hi, ch[g]);
+                cl[g] = mfma(a[t][g], b_lo, cl[g]);
             }
         }
     }
 #pragma unroll
-    for (int g = 0; g < NT; g++) {
-        acc[g][0] = __builtin_fmaf(dscale, cm[g][0] + cm[g][1], acc[g][0]);
-        acc[g][1] = __builtin_fmaf(dscale, cm[g][2] + cm[g][3], acc[g][1]);
-    }
+    for (int g = 0; g < NT; g++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float v = __builtin_fmaf(8.0f, ch[g][2 * j] + ch[g][2 * j + 1], cl[g][2 * j] + cl[g][2 * j + 1]);
+            acc[g][j] = __builtin_fmaf(up[g][j], dscale * v, acc[g][j]);
+        }
 }
 
 // ---------------------------------------------------------------------------
-// Weight staging.  A wave fetches G consecutive blocks of each of its 16-row
-// tiles as whole 16-byte chunks (row r of the tile: `chunks` chunks from the
-// dword at or below its first block; Q4_K runs start 16-aligned), consecutive
-// lanes on consecutive chunks of a row, and parks them in its own LDS area;
-// each lane then takes its operand pieces from there.  Every load
-// instruction covers a few long runs of rows instead of 16 rows' separate
-// 16-byte pieces.
+// Weight staging.  A wave fetches one block of each row of a 16-row tile as
+// whole 16-byte chunks (row r of the tile: `chunks` chunks from the dword at
+// or below the block; Q4_K blocks start 16-aligned), consecutive lanes on
+// consecutive chunks of a row; each lane then takes its operand pieces from
+// there.
 // ---------------------------------------------------------------------------
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));  // 16-byte aligned (LDS)
 
-template <uint32_t TYPE, uint32_t G> struct StageQ {
-    static constexpr uint32_t chunks = TYPE == kQ4_K ? 9 * G : (210 * G + 2 + 15) / 16;
+// One block of each row of a tile, straight from memory to the wave's LDS
+// ring: `loads` buffer loads of 64 (the last: the remaining) lanes whose
+// 16-byte results go to consecutive places from m0 on.  Written as
+// instructions: as builtins the compiler would make every LDS read wait for
+// all of them.  The caller counts them (s_waitcnt vmcnt).  All 64 lanes of
+// the wave are active.
+#define DM_SLOT4(m, o0, o1, o2, rs)                                                                          \
+    "s_mov_b32 m0, " m "\n\ts_nop 0\n\tbuffer_load_dwordx4 " o0 ", " rs ", 0 offen lds\n\t"                    \
+    "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 " o1 ", " rs ", 0 offen lds\n\t"              \
+    "s_add_u32 m0, m0, 0x400\n\ts_mov_b64 exec, 0xffff\n\tbuffer_load_dwordx4 " o2 ", " rs ", 0 offen lds\n\t" \
+    "s_mov_b64 exec, -1\n\t"
+#define DM_SLOT6(m, o0, o1, o2, o3, rs)                                                                      \
+    "s_mov_b32 m0, " m "\n\ts_nop 0\n\tbuffer_load_dwordx4 " o0 ", " rs ", 0 offen lds\n\t"                    \
+    "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 " o1 ", " rs ", 0 offen lds\n\t"              \
+    "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\tbuffer_load_dwordx4 " o2 ", " rs ", 0 offen lds\n\t"              \
+    "s_add_u32 m0, m0, 0x400\n\ts_mov_b32 exec_hi, 0\n\tbuffer_load_dwordx4 " o3 ", " rs ", 0 offen lds\n\t" \
+    "s_mov_b64 exec, -1\n\t"
+
+__device__ __forceinline__ void load_slot(uint32_t lds, const uint32_t (&o)[3], v4u rs) {
+    asm volatile(DM_SLOT4("%0", "%1", "%2", "%3", "%4")::"s"(lds), "v"(o[0]), "v"(o[1]), "v"(o[2]), "s"(rs)
+                 : "memory", "scc");
+}
+__device__ __forceinline__ void load_slot(uint32_t lds, const uint32_t (&o)[4], v4u rs) {
+    asm volatile(DM_SLOT6("%0", "%1", "%2", "%3", "%4", "%5")::"s"(lds), "v"(o[0]), "v"(o[1]), "v"(o[2]),
+                 "v"(o[3]), "s"(rs)
+                 : "memory", "scc");
+}
+
+template <uint32_t TYPE> struct StageQ {
+    static constexpr uint32_t bytes = TYPE == kQ4_K ? 144 : 210;  // of one block
+    static constexpr uint32_t chunks = TYPE == kQ4_K ? 9 : (210 + 2 + 15) / 16;
     static constexpr uint32_t items = 16 * chunks;        // chunks of one tile
     static constexpr uint32_t loads = (items + 63) / 64;  // 16-byte loads per lane
 };
@@ -438,7 +347,8 @@ __device__ __forceinline__ void take_raw(const v4u *stage, uint32_t ch, uint32_t
     raw.a1 = u32x4{sw[o1], sw[o1 + 1], sw[o1 + 2], sw[o1 + 3]};
     raw.a2 = u32x4{sw[o2], sw[o2 + 1], sw[o2 + 2], sw[o2 + 3]};
     raw.a3 = u32x4{sw[o3], sw[o3 + 1], sw[o3 + 2], sw[o3 + 3]};
-    raw.a4 = u32x4{sw[48], sw[49], sw[50], sw[51]};
+    raw.a4 = u32x2{sw[48 + 2 * h], sw[49 + 2 * h]};
+    raw.e5 = sw[50 + 2 * h];
     raw.e1 = sw[o1 + 4];
     raw.e2 = sw[o2 + 4];
     raw.e3 = sw[o3 + 4];
@@ -446,292 +356,509 @@ __device__ __forceinline__ void take_raw(const v4u *stage, uint32_t ch, uint32_t
     raw.e4b = sw[53];
 }
 
-// ---------------------------------------------------------------------------
-// Main kernel.  A workgroup has 4 waves; S waves split one group of R row
-// tiles along K, so a workgroup covers (4/S)*R tiles of 16 rows.
-// MB > 0: the activation fragments (MB = 2*batch rows) live in LDS.
-// MODE 0: y = W x.  MODE 1: also a per-wave argmax candidate.  MODE 2:
-// gate/up pair, act = silu(gate) * up.
-// ---------------------------------------------------------------------------
-template <uint32_t TYPE, int NT, int R, int S, int MODE, int MB, uint32_t G>
-__global__ void __launch_bounds__(64 * (S > 4 ? S : 4)) qmv_kernel(
-    const uint8_t *__restrict__ w, const uint8_t *__restrict__ w2, uint32_t rows,
-    uint32_t columns, uint32_t row_bytes, uint32_t total_bytes, const float *__restrict__ x,
-    int normalize, float epsilon, const _Float16 *__restrict__ xp,
-    const float *__restrict__ yscale_global, uint32_t batch, float *__restrict__ y,
-    ArgmaxPartial *__restrict__ partials) {
-    constexpr uint32_t SPB = Steps<TYPE>::value;
-    constexpr uint32_t BB = TYPE == kQ4_K ? 144u : 210u;
-    constexpr int RR = MODE == 2 ? 2 * R : R;  // gate/up: R tiles of each matrix
-    constexpr uint32_t WAVES = S > 4 ? S : 4;
-    __shared__ float partial[S > 1 ? WAVES * RR * NT * 64 * 2 : 1];
-    __shared__ float token_scale[2][4];
-    extern __shared__ half8 lds_a[];
+namespace {
 
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+// Workgroup barrier ordering LDS only: the waves' weight loads in flight are
+// not waited for, as __syncthreads() would.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+constexpr uint64_t kMeetEmpty = ~0ull;  // no published pair (two NaNs publish() never writes)
+
+struct QmvArgs {
+    const uint8_t *w, *w2;  // w2: the up matrix (MODE 2)
+    const float *x;
+    float *y;
+    uint64_t *meet;  // K-split meeting places, kMeetEmpty between launches
+    uint32_t rows, columns, row_bytes, batch;
+    uint32_t wave_k;      // waves of a workgroup that split K (1 to 16)
+    uint32_t k_parts;     // workgroups that split K (1, 2, 4 or 8)
+    uint32_t row_groups;  // workgroups that split the row tiles
+    uint32_t phases;      // fragment sets a wave goes through per pass (PHASED)
+    int normalize;
+    float epsilon;
+};
+
+// Two tokens' sums of one row as one word; a NaN becomes the canonical one,
+// so no published pair equals kMeetEmpty.
+__device__ __forceinline__ uint64_t pack_pair(float a, float b) {
+    const uint32_t ua = a == a ? __float_as_uint(a) : 0x7fc00000u, ub = b == b ? __float_as_uint(b) : 0x7fc00000u;
+    return (uint64_t)ub << 32 | ua;
+}
+
+// Tiles of a wave group between two cross-wave sums, whose LDS (red) leaves
+// room for the ring.
+template <int MODE, bool PHASED> constexpr uint32_t pass_tiles() { return (MODE == 2 ? 2 : 4) / (PHASED ? 2 : 1); }
+template <int NT, int MODE, uint32_t W, bool PHASED> constexpr uint32_t red_floats() {
+    return W * pass_tiles<MODE, PHASED>() * (MODE == 2 ? 2 : 1) * NT * 2 * 64;
+}
+// Slots of a wave's ring (one being read, the others in flight): what the
+// 160 KiB of LDS hold, at most 5 or 4 (first_loads).
+template <uint32_t TYPE, int NT, int MODE, uint32_t W, bool PHASED> constexpr uint32_t ring_depth() {
+    constexpr uint32_t fit = (156 * 1024 - red_floats<NT, MODE, W, PHASED>() * 4 - (PHASED ? W * 2048 : 0)) /
+                             (W * StageQ<TYPE>::items * 16);
+    constexpr uint32_t most = TYPE == kQ4_K ? 5 : 4;
+    return fit < most ? fit : most;
+}
+
+// The prologue's loads, in one block with their wait: the wave's first
+// activations (8 loads from the bytes xo0 and xo1 of x on; for XB = 2 also
+// those of the next block), then the first SLOTS slots of its ring, then the
+// wait for the activations alone.  Offsets and descriptors are per slot.
+#define DM_X(a, v, off) "buffer_load_dwordx4 %[" a "], %[" v "], %[xr], 0 offen offset:" off "\n\t"
+#define DM_XQ4                                                                                            \
+    DM_X("a0", "v0", "0") DM_X("a1", "v0", "64") DM_X("a2", "v0", "128") DM_X("a3", "v0", "192")          \
+    DM_X("a4", "v1", "0") DM_X("a5", "v1", "64") DM_X("a6", "v1", "128") DM_X("a7", "v1", "192")
+#define DM_XQ6                                                                                            \
+    DM_X("a0", "v0", "0") DM_X("a1", "v0", "128") DM_X("a2", "v0", "256") DM_X("a3", "v0", "384")         \
+    DM_X("a4", "v1", "0") DM_X("a5", "v1", "128") DM_X("a6", "v1", "256") DM_X("a7", "v1", "384")
+#define DM_XQ4B                                                                                           \
+    DM_X("b0", "v0", "1024") DM_X("b1", "v0", "1088") DM_X("b2", "v0", "1152") DM_X("b3", "v0", "1216")   \
+    DM_X("b4", "v1", "1024") DM_X("b5", "v1", "1088") DM_X("b6", "v1", "1152") DM_X("b7", "v1", "1216")
+#define DM_XQ6B                                                                                           \
+    DM_X("b0", "v0", "1024") DM_X("b1", "v0", "1152") DM_X("b2", "v0", "1280") DM_X("b3", "v0", "1408")   \
+    DM_X("b4", "v1", "1024") DM_X("b5", "v1", "1152") DM_X("b6", "v1", "1280") DM_X("b7", "v1", "1408")
+#define DM_OUT(c, q)                                                                              \
+    [c##0] "=&v"(x[q][0]), [c##1] "=&v"(x[q][1]), [c##2] "=&v"(x[q][2]), [c##3] "=&v"(x[q][3]),   \
+        [c##4] "=&v"(x[q][4]), [c##5] "=&v"(x[q][5]), [c##6] "=&v"(x[q][6]), [c##7] "=&v"(x[q][7])
+#define DM_Q4(d) DM_SLOT4("%[l]", "%[o" #d "0]", "%[o" #d "1]", "%[o" #d "2]", "%[r" #d "]")
+#define DM_Q6(d) DM_SLOT6("%[l]", "%[o" #d "0]", "%[o" #d "1]", "%[o" #d "2]", "%[o" #d "3]", "%[r" #d "]")
+#define DM_NEXT(bytes) "s_add_u32 %[l], %[l], " #bytes "\n\t"
+#define DM_IN3(d) [o##d##0] "v"(o[d][0]), [o##d##1] "v"(o[d][1]), [o##d##2] "v"(o[d][2]), [r##d] "s"(rs[d])
+#define DM_IN4(d) DM_IN3(d), [o##d##3] "v"(o[d][3])
+#define DM_ARGS [xr] "s"(xr), [v0] "v"(xo0), [v1] "v"(xo1)
+template <uint32_t TYPE, int XB, uint32_t SLOTS, uint32_t NL>
+__device__ __forceinline__ void first_loads(floatx4 (&x)[XB][8], v4u xr, uint32_t xo0, uint32_t xo1, uint32_t lds,
+                                            const uint32_t (&o)[SLOTS][NL], const v4u (&rs)[SLOTS]) {
+    if constexpr (TYPE == kQ4_K && XB == 1 && SLOTS == 2) {
+        asm volatile(DM_XQ4 DM_Q4(0) DM_NEXT(2304) DM_Q4(1) "s_waitcnt vmcnt(6)"
+                     : DM_OUT(a, 0), [l] "+&s"(lds)
+                     : DM_ARGS, DM_IN3(0), DM_IN3(1)
+                     : "memory", "scc");
+    } else if constexpr (TYPE == kQ4_K && XB == 1 && SLOTS == 4) {
+        asm volatile(DM_XQ4 DM_Q4(0) DM_NEXT(2304) DM_Q4(1) DM_NEXT(2304) DM_Q4(2) DM_NEXT(2304) DM_Q4(3) "s_waitcnt vmcnt(12)"
+                     : DM_OUT(a, 0), [l] "+&s"(lds)
+                     : DM_ARGS, DM_IN3(0), DM_IN3(1), DM_IN3(2), DM_IN3(3)
+                     : "memory", "scc");
+    } else if constexpr (TYPE == kQ4_K && XB == 2 && SLOTS == 2) {
+        asm volatile(DM_XQ4 DM_XQ4B DM_Q4(0) DM_NEXT(2304) DM_Q4(1) "s_waitcnt vmcnt(6)"
+                     : DM_OUT(a, 0), DM_OUT(b, 1), [l] "+&s"(lds)
+                     : DM_ARGS, DM_IN3(0), DM_IN3(1)
+                     : "memory", "scc");
+    } else if constexpr (TYPE == kQ6_K && XB == 1 && SLOTS == 1) {
+        asm volatile(DM_XQ6 DM_Q6(0) "s_waitcnt vmcnt(4)"
+                     : DM_OUT(a, 0), [l] "+&s"(lds)
+                     : DM_ARGS, DM_IN4(0)
+                     : "memory", "scc");
+    } else if constexpr (TYPE == kQ6_K && XB == 1 && SLOTS == 3) {
+        asm volatile(DM_XQ6 DM_Q6(0) DM_NEXT(3584) DM_Q6(1) DM_NEXT(3584) DM_Q6(2) "s_waitcnt vmcnt(12)"
+                     : DM_OUT(a, 0), [l] "+&s"(lds)
+                     : DM_ARGS, DM_IN4(0), DM_IN4(1), DM_IN4(2)
+                     : "memory", "scc");
+    } else if constexpr (TYPE == kQ6_K && XB == 2 && SLOTS == 1) {
+        asm volatile(DM_XQ6 DM_XQ6B DM_Q6(0) "s_waitcnt vmcnt(4)"
+                     : DM_OUT(a, 0), DM_OUT(b, 1), [l] "+&s"(lds)
+                     : DM_ARGS, DM_IN4(0)
+                     : "memory", "scc");
+    } else {
+        static_assert(TYPE == 0, "no such prologue");
+    }
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
+// Main kernel.  A wave owns a run of up to KB blocks of K: it builds the
+// activation fragments of those columns in registers once, then streams its
+// run of one 16-row tile after another, so the fragments are never read
+// again.  The weights go from memory straight to the wave's LDS ring
+// (buffer loads with the LDS destination), DEPTH - 1 blocks ahead of the one
+// being computed.  The workgroup's wave_k waves cover a K part together
+// (their loads are the whole rows of a tile) and its waves / wave_k wave groups
+// take alternate tiles; every pass_tiles tiles the waves' results meet in
+// LDS and are written.
+// Grid: k_parts x row_groups workgroups, one per CU.  With k_parts > 1 the
+// parts' sums meet pairwise in memory: a workgroup exchanges its pair of
+// sums with the meeting place; the first to come finds it empty and is done,
+// the second adds what it finds and goes on to the next level (a + b is the
+// same in either order, so the result does not depend on who is first).
+// MODE 0: y = W x.  MODE 2: gate/up pair on RMSNorm(x), act = silu(gate) * up
+// (k_parts = 1).
+//
+// What bounds it: bytes in flight.  110 KiB of ring hold two or three tiles'
+// blocks per wave, and each wave asks for the next only when it has finished
+// one, so a tall matrix streams at 4.7 TB/s; the fragments' prologue (x, split,
+// first weights) is about 3 us of every launch.  Measured on MI355X against
+// the form with a launch that prepared the fragments in memory and waves that
+// read them again for every tile: Q4_K 12288 x 4096, 8 tokens 16.8 -> 10.2
+// us, 16 tokens 25.2 -> 15.0; Q6_K 4096 x 12288, 8 tokens 20.6 -> 13.9;
+// 4096 x 4096 Q4_K 10.7 -> 7.0; Q6_K 151936 x 4096 200 -> 112 us.  16 waves
+// of one block beat 8 of two (12.6 us at 12288 x 4096): four waves per SIMD
+// hide each other's LDS and MFMA latency.
+// ---------------------------------------------------------------------------
+template <uint32_t TYPE, int NT, int MODE, int KB, uint32_t W, bool PHASED>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
+qmv_kernel(const QmvArgs p) {
+    constexpr uint32_t BB = StageQ<TYPE>::bytes;
+    constexpr uint32_t RR = MODE == 2 ? 2 : 1;  // matrices streamed
+    constexpr uint32_t DEPTH = ring_depth<TYPE, NT, MODE, W, PHASED>();
+    static_assert(DEPTH >= 2, "a slot in flight while one is read");
+    using ST = StageQ<TYPE>;
+    constexpr uint32_t CH = ST::chunks, NL = ST::loads;
+    constexpr uint32_t SLOT = ST::items;      // chunks of a ring slot
+    constexpr uint32_t PI = pass_tiles<MODE, PHASED>() * RR;  // items of a wave per pass
+    __shared__ v4u red_all[red_floats<NT, MODE, W, PHASED>() / 4];
+    __shared__ v4u split_all[PHASED ? W * 128 : 1];
+    __shared__ uint32_t s_min[W * 64];  // 8 tokens x {hi, lo} x 4 lane groups
+    __shared__ float red_ss[MODE == 2 ? W * 16 : 1];
+    __shared__ float s_up[W * KB * 16];  // 2^e of each wave's blocks and tokens
+    extern __shared__ v4u ring_all[];
+    float *red = (float *)red_all;
+
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t n = lane & 15u, kg = lane >> 4;
-    const uint32_t group = wave / S, kpart = wave % S;
-    const uint32_t first_tile = (blockIdx.x * (WAVES / S) + group) * R;
-    const uint32_t blocks = columns / 256;
-    const uint32_t groups = (blocks + G - 1) / G;
-    const uint32_t g_begin = kpart * groups / S, g_end = (kpart + 1) * groups / S;
-    const uint32_t m2 = 2 * batch;
-    const float *yscale = yscale_global;
+    const uint32_t wk = p.wave_k, wt = (blockDim.x >> 6) / wk, kw = wave % wk, wg = wave / wk;
+    const uint32_t part = blockIdx.x % p.k_parts, rg = blockIdx.x / p.k_parts;
+    const uint32_t blocks = p.columns / 256, tiles = (p.rows + 15) / 16;
+    const uint32_t t_begin = (uint32_t)((uint64_t)rg * tiles / p.row_groups);
+    const uint32_t t_end = (uint32_t)((uint64_t)(rg + 1) * tiles / p.row_groups);
+    const uint32_t phases = PHASED ? p.phases : 1u, units = wk * p.k_parts * phases;
+    v4u *ring = ring_all + wave * DEPTH * SLOT;
+    const uint32_t ring_lds =
+        __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) v4u *)ring);
 
-    // Lanes whose A row carries no token read a zeroed copy of one block's
-    // fragments, so every lane runs the same loads.
-    const half8 *a_lane = nullptr;
-    uint32_t a_block_stride = 0;
-    if constexpr (MB > 0) {
-        // Copy every activation fragment of the row (written by the
-        // preparation kernel) into LDS, followed by one zeroed block.
-        const uint32_t count = blocks * SPB * 4 * MB;
-        const half8 *src = (const half8 *)xp;
-        for (uint32_t i = threadIdx.x; i < count; i += 64 * WAVES) lds_a[i] = src[i];
-        for (uint32_t i = threadIdx.x; i < SPB * 4 * MB; i += 64 * WAVES)
-            lds_a[count + i] = half8{0, 0, 0, 0, 0, 0, 0, 0};
-        if (threadIdx.x < MB / 2) token_scale[threadIdx.x][0] = yscale_global[threadIdx.x];
-        __syncthreads();
-        a_lane = n < (uint32_t)MB ? lds_a + kg * MB + n : lds_a + count + kg * MB;
-        a_block_stride = n < (uint32_t)MB ? SPB * 4 * MB : 0;
-    }
+    // Buffer descriptors over whole dwords: the last dword of the matrix may
+    // extend up to 3 bytes past its end (inside the allocation's
+    // granularity); loads beyond it read 0.
+    const uint32_t records = (p.row_bytes * p.rows + 3u) & ~3u;
+    auto descriptor = [&](const uint8_t *base) {
+        return v4u{(uint32_t)(uintptr_t)base, (uint32_t)((uintptr_t)base >> 32) & 0xffffu, records, 0x00020000u};
+    };
+    const v4u rsrc = descriptor(p.w), rsrc2 = descriptor(MODE == 2 ? p.w2 : p.w);
 
-    // Whole dwords: the last dword of the matrix may extend up to 3 bytes past
-    // its end (inside the allocation's granularity); loads beyond it read 0.
-    const uint32_t records = (total_bytes + 3u) & ~3u;
-    const uint32_t nowhere = records + 256;  // every load from here reads 0
-    const __amdgpu_buffer_rsrc_t rsrc = make_rsrc(w, records);
-    const __amdgpu_buffer_rsrc_t rsrc2 = make_rsrc(MODE == 2 ? w2 : w, records);
+    // Position in the wave's sequence: pass (pass_tiles tiles of each
+    // wave group), phase, item (tile of the pass, matrix).
+    struct Pos {
+        uint32_t tile0, phase, i;  // first tile of the pass
+    };
+    const uint32_t pass_step = pass_tiles<MODE, PHASED>() * wt;
+    auto items = [&](uint32_t tile0) {  // items per wave and phase of the pass at tile0
+        const uint32_t left = t_end - tile0, t = left < pass_step ? left : pass_step;
+        return (t + wt - 1) / wt * RR;
+    };
+    auto advance = [&](Pos &q) {
+        if (++q.i < items(q.tile0)) return;
+        q.i = 0;
+        if (PHASED) {
+            if (++q.phase < phases) return;
+            q.phase = 0;
+        }
+        q.tile0 += pass_step;
+    };
+    auto k_begin = [&](uint32_t phase) { return ((part * phases + phase) * wk + kw) * blocks / units; };
+    auto k_end = [&](uint32_t phase) { return ((part * phases + phase) * wk + kw + 1) * blocks / units; };
 
-    float acc[RR][NT][2];
-#pragma unroll
-    for (int r = 0; r < RR; r++)
-#pragma unroll
-        for (int g = 0; g < NT; g++) acc[r][g][0] = acc[r][g][1] = 0.0f;
-
-    // Row of tile r handled by this lane (may be >= rows: loads return 0).
-    uint32_t row_base[RR];
-#pragma unroll
-    for (int r = 0; r < RR; r++) {
-        const uint32_t tile = first_tile + (MODE == 2 ? r % R : r);
-        const uint32_t row = tile * 16 + n;
-        row_base[r] = row < rows ? row * row_bytes : nowhere;
-    }
-
-    // Staging: the wave's area holds RR tiles of ITEMS chunks; load j of
-    // this lane is chunk src_chunk[j] of row (item / CH) of each tile.
-    using ST = StageQ<TYPE, G>;
-    constexpr uint32_t CH = ST::chunks, NL = ST::loads, ITEMS = ST::items;
-    const size_t a_bytes = MB > 0 ? ((size_t)blocks + 1) * SPB * 4 * MB * 16 : 0;
-    v4u *stage = (v4u *)((uint8_t *)lds_a + a_bytes) + (size_t)wave * RR * ITEMS;
-    uint32_t src_row[RR][NL], src_chunk[NL];
+    // Chunk j * 64 + lane of a block of a tile: offset from the wave's first
+    // block of the tile's first row (16 c is a multiple of the 4 bytes the
+    // sum is aligned to).
+    uint32_t lane_off[NL];
 #pragma unroll
     for (uint32_t j = 0; j < NL; j++) {
-        const uint32_t item = j * 64 + lane, ri = item / CH;
-        src_chunk[j] = 16 * (item - ri * CH);
-#pragma unroll
-        for (int r = 0; r < RR; r++) {
-            const uint32_t row = (first_tile + (MODE == 2 ? r % R : r)) * 16 + ri;
-            src_row[r][j] = (item < ITEMS && row < rows) ? row * row_bytes : nowhere;
-        }
+        const uint32_t item = j * 64 + lane, r = item / CH, c = item % CH;
+        lane_off[j] = r * p.row_bytes + 16 * c;
     }
-    v4u st[RR][NL];
-    auto fetch = [&](uint32_t grp) {
+    // The loads of block b of the wave's run of q's item; a block past the run
+    // or a tile past the end reads past the matrix (zeros), so that the loads
+    // in flight can be counted.
+    auto slot_loads = [&](const Pos &q, uint32_t b, uint32_t (&off)[NL], v4u &rs) {
+        const uint32_t tile = q.tile0 + (q.i / RR) * wt + wg;
+        const uint32_t blk = k_begin(q.phase) + b;
+        const uint32_t base = q.tile0 < t_end && tile < t_end && blk < k_end(q.phase)
+                                  ? tile * 16 * p.row_bytes + blk * BB
+                                  : 0xffffffffu;
 #pragma unroll
-        for (int r = 0; r < RR; r++)
-#pragma unroll
-            for (uint32_t j = 0; j < NL; j++) {
-                const uint32_t off =
-                    src_row[r][j] == nowhere ? nowhere : ((src_row[r][j] + grp * G * BB) & ~3u) + src_chunk[j];
-                st[r][j] = __builtin_bit_cast(v4u, rsrc_load16((MODE == 2 && r >= R) ? rsrc2 : rsrc, off));
-            }
+        for (uint32_t j = 0; j < NL; j++) off[j] = __builtin_elementwise_add_sat(lane_off[j], base) & ~3u;
+        rs = MODE == 2 && (q.i % RR) ? rsrc2 : rsrc;
     };
-    // A wave reads only its own area and its LDS operations run in order; the
-    // wavefront-scope fences keep the compiler from moving another lane's
-    // reads across these writes.
-    auto put = [&]() {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-        for (int r = 0; r < RR; r++)
-#pragma unroll
-            for (uint32_t j = 0; j < NL; j++)
-                if (j + 1 < NL || j * 64 + lane < ITEMS) stage[r * ITEMS + j * 64 + lane] = st[r][j];
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    // nxt, nxt_b: the next block to request.
+    Pos nxt{t_begin, 0, 0};
+    uint32_t nxt_b = 0, issue_slot = 0;
+    auto next_block = [&]() {
+        if (++nxt_b == KB) {
+            nxt_b = 0;
+            advance(nxt);
+        }
     };
-    // Activation fragments of block blk (from LDS, or from the prepared
-    // fragments in global memory one block ahead of their use).
-    auto load_a = [&](uint32_t blk, half8 (&a)[SPB][NT]) {
-#pragma unroll
-        for (int t = 0; t < (int)SPB; t++)
-#pragma unroll
-            for (int g = 0; g < NT; g++) {
-                const uint32_t m = 16 * g + n;
-                if constexpr (MB > 0) {
-                    // one address per block, then immediate offsets per step
-                    a[t][g] = a_lane[blk * a_block_stride + t * 4 * MB];
-                } else if (m < m2) {
-                    const size_t f = ((size_t)blk * SPB + t) * 4 + kg;
-                    a[t][g] = *(const half8 *)(xp + (f * m2 + m) * 8);
-                } else {
-                    a[t][g] = half8{0, 0, 0, 0, 0, 0, 0, 0};
-                }
-            }
+    auto issue_next = [&]() {
+        uint32_t off[NL];
+        v4u rs;
+        slot_loads(nxt, nxt_b, off, rs);
+        // (the slot's last reads have returned)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        load_slot(ring_lds + issue_slot * (SLOT * 16), off, rs);
+        issue_slot = issue_slot + 1 == DEPTH ? 0 : issue_slot + 1;
+        next_block();
     };
 
-    // The loads of group g+1 are in flight while group g is computed, and
-    // the activation fragments of the next block while a block is computed.
-    if (g_begin < g_end) {
-        const uint32_t blk_end = g_end * G < blocks ? g_end * G : blocks;
-        half8 a[SPB][NT];
-        load_a(g_begin * G, a);
-        fetch(g_begin);
-        for (uint32_t grp = g_begin; grp < g_end; grp++) {
-            put();
-            if (grp + 1 < g_end) fetch(grp + 1);
+    half8 a[KB][8][NT];
+    uint32_t amin[KB][NT];  // the min step's fragment (its other columns are zero)
+    float ss[NT * 2];       // MODE 2: the lane's part of its tokens' sums of squares
+    // The fragments of block b, tokens 8 g .. 8 g + 7: the values are scaled
+    // and split as they were loaded (x4[4 u + r], see round_column) and go
+    // through LDS to the lanes that hold the token's A rows, a round (2 KiB)
+    // at a time: the quad (kg, c) of token i is at slot (4 kg + c) ^ i of 16
+    // (so neither side meets bank conflicts), hi pairs then lo pairs.  The
+    // area is the wave's part of red before the first pass, or (PHASED) LDS of
+    // its own; a wave reads only what it wrote.
+    const uint32_t li = lane >> 4, lk = (lane >> 2) & 3u, lc = lane & 3u;
+    uint32_t *sp = (uint32_t *)(PHASED ? split_all : red_all) + wave * (PHASED ? 512 : PI * NT * 128);
+    uint32_t *smn = s_min + wave * 64;
+    auto split = [&](int g, int b, uint32_t phase, const floatx4 (&x4)[8]) {
+        const bool used = k_begin(phase) + b < k_end(phase);
+        float down[2];
 #pragma unroll
-            for (uint32_t b = 0; b < G; b++) {
-                const uint32_t blk = grp * G + b;
-                if (blk >= blk_end) break;
-                half8 a_next[SPB][NT];
-                if (blk + 1 < blk_end) load_a(blk + 1, a_next);
-                Raw<TYPE> raw[RR];
+        for (int u = 0; u < 2; u++) {
+            float mx = 0.0f, q = 0.0f;
 #pragma unroll
-                for (int r = 0; r < RR; r++) {
-                    // the run of row n starts 0 or 2 bytes into its first dword (Q6_K)
-                    const uint32_t s0 = row_base[r] == nowhere ? 0u : ((row_base[r] + grp * G * BB) & 3u);
-                    take_raw(stage + r * ITEMS, CH, n, kg, s0 + b * BB, raw[r]);
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float v = x4[4 * u + r][j];
+                    mx = fmaxf(mx, fabsf(v));
+                    if (MODE == 2) q = __builtin_fmaf(v, v, q);
                 }
+            if (MODE == 2 && used) ss[2 * g + u] += q;
+            const int e = block_exponent(row_max(mx));
+            down[u] = ldexpf(1.0f, -e);
+            // every lane of the row holds the same scale
+            s_up[(wave * KB + b) * 16 + 8 * g + 4 * u + li] = ldexpf(1.0f, e);
+        }
+        uint32_t hi[8][2], lo[8][2];
 #pragma unroll
-                for (int r = 0; r < RR; r++) block_dot<NT>(raw[r], a, kg, acc[r]);
-                if (blk + 1 < blk_end) {
+        for (int u = 0; u < 2; u++) {
+            float sum[2] = {0.0f, 0.0f};
 #pragma unroll
-                    for (int t = 0; t < (int)SPB; t++)
+            for (int r = 0; r < 4; r++) {
+                const floatx4 v = x4[4 * u + r] * down[u];
+                // fragment order of a quad: columns 0, 2, 1, 3 (the byte pairs of a weight dword)
+                split_pair(v[0], v[2], hi[4 * u + r][0], lo[4 * u + r][0]);
+                split_pair(v[1], v[3], hi[4 * u + r][1], lo[4 * u + r][1]);
+                if (TYPE == kQ4_K) sum[r >> 1] += (v[0] + v[1]) + (v[2] + v[3]);
+            }
+            if constexpr (TYPE == kQ4_K) {
+                // sub-blocks 2 kg, 2 kg + 1; 2^-6 keeps |sum| inside fp16
+                uint32_t h, l;
+                split_pair(quad_sum(sum[0]) * 0.015625f, quad_sum(sum[1]) * 0.015625f, h, l);
+                smn[(4 * u + li) * 8 + lk] = h;
+                smn[(4 * u + li) * 8 + 4 + lk] = l;
+            }
+        }
+        const uint32_t token = n >> 1, half = n & 1u;
+        uint32_t f[8][4];
 #pragma unroll
-                        for (int g = 0; g < NT; g++) a[t][g] = a_next[t][g];
+        for (int r = 0; r < 4; r++) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const uint32_t i = 4 * u + li;
+                *(v4u *)&sp[i * 64 + ((4 * lk + lc) ^ i) * 4] =
+                    v4u{hi[4 * u + r][0], hi[4 * u + r][1], lo[4 * u + r][0], lo[4 * u + r][1]};
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (uint32_t c = 0; c < 4; c++) {
+                const u32x2 v = *(const u32x2 *)&sp[token * 64 + ((4 * kg + c) ^ token) * 4 + half * 2];
+                f[quad_step<TYPE>(r, c)][2 * quad_half<TYPE>(r, c)] = v[0];
+                f[quad_step<TYPE>(r, c)][2 * quad_half<TYPE>(r, c) + 1] = v[1];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int t = 0; t < 8; t++) a[b][t][g] = frag(f[t][0], f[t][1], f[t][2], f[t][3]);
+        if constexpr (TYPE == kQ4_K) amin[b][g] = smn[token * 8 + half * 4 + kg];
+    };
+    // Byte of x that load (u, 0) of a block takes (tokens past the batch read
+    // past the end: zeros).
+    auto x_byte = [&](int g, uint32_t blk, int u) {
+        return ((8 * g + 4 * u + li) * p.columns + blk * 256 + round_column<TYPE>(lk) + 4 * lc) * 4;
+    };
+    const v4u xr = v4u{(uint32_t)(uintptr_t)p.x, (uint32_t)((uintptr_t)p.x >> 32) & 0xffffu, p.batch * p.columns * 4,
+                       0x00020000u};
+    const __amdgpu_buffer_rsrc_t xrs = make_rsrc(p.x, p.batch * p.columns * 4);
+    auto load_x = [&](int g, int b, uint32_t phase, floatx4 (&x4)[8]) {
+#pragma unroll
+        for (int i = 0; i < 8; i++)
+            x4[i] = __builtin_bit_cast(
+                floatx4, rsrc_load16(xrs, x_byte(g, k_begin(phase) + b, i / 4) + (i % 4) * round_bytes<TYPE>()));
+    };
+    auto store_ss = [&](uint32_t phase) {
+        if constexpr (MODE == 2) {
+#pragma unroll
+            for (int i = 0; i < NT * 2; i++) {
+                const float v = row_sum(ss[i]);
+                if ((lane & 15u) == 0) {
+                    float &slot = red_ss[wave * 16 + 4 * i + li];
+                    slot = phase == 0 ? v : slot + v;
                 }
             }
         }
-    }
+    };
 
-    // --- split-K reduction through LDS --------------------------------------
-    if constexpr (S > 1) {
 #pragma unroll
-        for (int r = 0; r < RR; r++)
+    for (int i = 0; i < NT * 2; i++) ss[i] = 0.0f;
+    Pos cur{t_begin, 0, 0};
+    {
+        // The first activations are requested before the weights, and waited
+        // for without them: a wave's loads complete in the order they were
+        // issued.
+        constexpr int XB = W == 16 ? KB : 1;  // blocks of x requested here
+        floatx4 x4[XB][8];
+        uint32_t off[DEPTH - 1][NL];
+        v4u rs[DEPTH - 1];
 #pragma unroll
-            for (int g = 0; g < NT; g++)
+        for (uint32_t d = 0; d + 1 < DEPTH; d++) {
+            slot_loads(nxt, nxt_b, off[d], rs[d]);
+            next_block();
+        }
+        issue_slot = DEPTH - 1;
+        first_loads<TYPE, XB>(x4, xr, x_byte(0, k_begin(0), 0), x_byte(0, k_begin(0), 1), ring_lds, off, rs);
 #pragma unroll
-                for (int j = 0; j < 2; j++)
-                    partial[((((wave * RR + r) * NT + g) * 64) + lane) * 2 + j] = acc[r][g][j];
-        __syncthreads();
-        if (kpart != 0) return;
+        for (int b = 0; b < XB; b++) split(0, b, 0, x4[b]);
 #pragma unroll
-        for (int r = 0; r < RR; r++)
+        for (int g = 0; g < NT; g++)
+#pragma unroll
+            for (int b = g == 0 ? XB : 0; b < KB; b++) {
+                load_x(g, b, 0, x4[0]);
+                split(g, b, 0, x4[0]);
+            }
+    }
+    store_ss(0);
+
+    bool first_pass = true;
+    uint32_t slot = 0;
+    while (cur.tile0 < t_end) {
+        const uint32_t tile0 = cur.tile0;
+#pragma clang loop unroll(disable)
+        do {
+            if (PHASED && cur.i == 0 && !(first_pass && cur.phase == 0)) {
+                // the next phase's fragments (K longer than the registers of
+                // the workgroups that split it hold)
+#pragma unroll
+                for (int i = 0; i < NT * 2; i++) ss[i] = 0.0f;
+#pragma unroll
+                for (int g = 0; g < NT; g++)
+#pragma unroll
+                    for (int b = 0; b < KB; b++) {
+                        floatx4 x4[8];
+                        load_x(g, b, cur.phase, x4);
+                        split(g, b, cur.phase, x4);
+                    }
+                if (first_pass) store_ss(cur.phase);
+            }
+            float acc[NT][2];
+#pragma unroll
+            for (int g = 0; g < NT; g++) acc[g][0] = acc[g][1] = 0.0f;
+            const uint32_t k0 = k_begin(cur.phase), nb = k_end(cur.phase) - k0;
+            const uint32_t tile = cur.tile0 + (cur.i / RR) * wt + wg;
+            const uint32_t row_at = (tile * 16 + n) * p.row_bytes + k0 * BB;
+#pragma unroll
+            for (int b = 0; b < KB; b++) {
+                issue_next();
+                // The loads of this slot are the oldest in flight: all but
+                // the DEPTH - 1 blocks requested after them have landed.
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NL * (DEPTH - 1)) : "memory");
+                if ((uint32_t)b < nb) {
+                    // read only by the wave that wrote them
+                    float up[NT][2];
+#pragma unroll
+                    for (int g = 0; g < NT; g++)
+#pragma unroll
+                        for (int j = 0; j < 2; j++) up[g][j] = s_up[(wave * KB + b) * 16 + 8 * g + 2 * kg + j];
+                    Raw<TYPE> raw;
+                    // a Q6_K block starts 0 or 2 bytes into its first dword
+                    take_raw(ring + slot * SLOT, CH, n, kg, (row_at + b * BB) & 3u, raw);
+                    block_dot<NT>(raw, a[b], amin[b], kg, up, acc);
+                }
+                slot = slot + 1 == DEPTH ? 0 : slot + 1;
+            }
+            float *sl = &red[((wave * PI + cur.i) * NT * 2) * 64 + lane];
 #pragma unroll
             for (int g = 0; g < NT; g++)
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
-                    float v = 0.0f;
-                    for (int p = 0; p < S; p++)
-                        v += partial[(((((wave + p) * RR + r) * NT + g) * 64) + lane) * 2 + j];
-                    acc[r][g][j] = v;
+                    float &s = sl[(2 * g + j) * 64];
+                    s = !PHASED || cur.phase == 0 ? acc[g][j] : s + acc[g][j];
                 }
-    }
+            advance(cur);
+        } while (cur.tile0 == tile0);
+        first_pass = false;
 
-    // --- epilogue --------------------------------------------------------------
-    uint64_t best = 0;
-    uint32_t bad = 0;
+        // The cross-wave sums and the output of the pass: thread = row rn of
+        // a tile, tokens tk and tk + 1.
+        lds_barrier();
+        const uint32_t left = t_end - tile0, nt = left < pass_step ? left : pass_step;
+        const uint32_t pairs = (p.batch + 1) / 2;
+        for (uint32_t idx = threadIdx.x; idx < nt * 16 * pairs; idx += blockDim.x) {
+            const uint32_t rn = idx & 15u, pair = (idx >> 4) / nt, tl = (idx >> 4) - pair * nt;
+            // tokens 8 g + 2 kg + {0, 1}: lane rn + 16 kg, elements 2 g + {0, 1}
+            const uint32_t el = 2 * (pair >> 2), ln = rn + 16 * (pair & 3u);
+            const uint32_t group = tl % wt, sl = tl / wt, tk = 2 * pair, row = (tile0 + tl) * 16 + rn;
+            float v[RR][2];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const uint32_t row = (first_tile + r) * 16 + n;
-        if (row >= rows) continue;
-#pragma unroll
-        for (int g = 0; g < NT; g++)
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const uint32_t token = 8 * g + 2 * kg + j;
-                if (token >= batch) continue;
-                const float sc = MB > 0 ? token_scale[token][0] : yscale[token];
-                float v = acc[r][g][j] * sc;
-                if constexpr (MODE == 2) {
-                    const float u = acc[R + r][g][j] * sc;
-                    // silu(gate) * up, stable sigmoid (src/qwen35/cpu.rs:982-993)
-                    float sig;
-                    if (v >= 0.0f) {
-                        sig = 1.0f / (1.0f + expf(-v));
-                    } else {
-                        const float ex = expf(v);
-                        sig = ex / (1.0f + ex);
-                    }
-                    v = v * sig * u;
-                }
-                y[(size_t)token * rows + row] = v;
-                if constexpr (MODE == 1) {
-                    if (!__builtin_isfinite(v)) bad = 1;
-                    const uint64_t key = argmax_key(v, row);
-                    best = key > best ? key : best;
+            for (uint32_t m = 0; m < RR; m++) {
+                v[m][0] = v[m][1] = 0.0f;
+#pragma clang loop unroll_count(4)
+                for (uint32_t k = 0; k < wk; k++) {
+                    const float *r = &red[(((group * wk + k) * PI + sl * RR + m) * NT * 2 + el) * 64 + ln];
+                    v[m][0] += r[0];
+                    v[m][1] += r[64];
                 }
             }
-    }
-    if constexpr (MODE == 1) {
-        // No atomics and no device-wide fence here: each wave writes its own
-        // candidate and a one-workgroup pass reduces them.
-        best = wave_max_u64(best);
-        bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
-        if (lane == 0) {
-            ArgmaxPartial p;
-            p.key = best;
-            p.non_finite = bad;
-            p.pad = 0;
-            partials[blockIdx.x * (WAVES / S) + group] = p;
-        }
-    }
-}
-
-// Reduces the per-wave candidates: the largest key wins (value, then lowest
-// row); any non-finite row marks the result.
-// 1024 threads with eight loads in flight each: a C2-sized candidate list
-// (9496 entries) takes two rounds of memory latency.
-constexpr uint32_t kArgmaxThreads = 1024;
-
-__global__ void __launch_bounds__(kArgmaxThreads) argmax_partials_kernel(
-    const ArgmaxPartial *__restrict__ partials, uint32_t count, ArgmaxState *state, uint32_t *index_out) {
-    constexpr uint32_t U = 8, WAVES = kArgmaxThreads / 64;
-    __shared__ unsigned long long keys[WAVES];
-    __shared__ uint32_t flags[WAVES];
-    uint64_t best = 0;
-    uint32_t bad = 0;
-    for (uint32_t i0 = 0; i0 < count; i0 += kArgmaxThreads * U) {
-        ArgmaxPartial p[U];
+            if constexpr (MODE == 2) {
 #pragma unroll
-        for (uint32_t j = 0; j < U; j++) {
-            const uint32_t i = i0 + kArgmaxThreads * j + threadIdx.x;
-            p[j] = i < count ? partials[i] : ArgmaxPartial{0, 0, 0};
+                for (int j = 0; j < 2; j++) {
+                    // RMSNorm factor inv = (ss/n + eps).sqrt().recip() (src/cpu.rs:98-142)
+                    float q = 0.0f;
+#pragma clang loop unroll_count(4)
+                    for (uint32_t k = 0; k < wk; k++) q += red_ss[k * 16 + tk + j];
+                    const float sc = p.normalize ? 1.0f / __builtin_sqrtf(q / (float)p.columns + p.epsilon) : 1.0f;
+                    const float gate = v[0][j] * sc, u = v[1][j] * sc;
+                    // silu(gate) * up, stable sigmoid (src/qwen35/cpu.rs:982-993)
+                    const float ex = expf(-fabsf(gate));
+                    const float sig = (gate >= 0.0f ? 1.0f : ex) / (1.0f + ex);
+                    v[0][j] = gate * sig * u;
+                }
+            } else {
+                bool mine = true;
+                uint64_t *place = p.meet + ((size_t)(tile0 + tl) * (p.k_parts - 1) * pairs + pair) * 16 + rn;
+                for (uint32_t span = 1, nodes = p.k_parts / 2; span < p.k_parts; span *= 2, nodes /= 2) {
+                    uint64_t *at = place + (size_t)(part / (2 * span)) * pairs * 16;
+                    const uint64_t other = __hip_atomic_exchange(at, pack_pair(v[0][0], v[0][1]), __ATOMIC_RELAXED,
+                                                                 __HIP_MEMORY_SCOPE_AGENT);
+                    if (other == kMeetEmpty) {
+                        mine = false;
+                        break;
+                    }
+                    __hip_atomic_store(at, kMeetEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    v[0][0] += __uint_as_float((uint32_t)other);
+                    v[0][1] += __uint_as_float((uint32_t)(other >> 32));
+                    place += (size_t)nodes * pairs * 16;
+                }
+                if (!mine) continue;
+            }
+            if (row < p.rows) {
+                p.y[(size_t)tk * p.rows + row] = v[0][0];
+                if (tk + 1 < p.batch) p.y[(size_t)(tk + 1) * p.rows + row] = v[0][1];
+            }
         }
-#pragma unroll
-        for (uint32_t j = 0; j < U; j++) {
-            best = p[j].key > best ? p[j].key : best;
-            bad |= p[j].non_finite;
-        }
+        lds_barrier();  // red is written again in the next pass
     }
-    best = wave_max_u64(best);
-    bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
-    if ((threadIdx.x & 63u) == 0) {
-        keys[threadIdx.x >> 6] = best;
-        flags[threadIdx.x >> 6] = bad;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t b = keys[0];
-        uint32_t f = flags[0];
-        for (uint32_t i = 1; i < WAVES; i++) {
-            b = keys[i] > b ? keys[i] : b;
-            f |= flags[i];
-        }
-        state->key = b;
-        state->non_finite = f;
-        state->done = count;
-        *index_out = argmax_key_index(b);
-    }
+    // the ring's last loads have landed before the workgroup's LDS is freed
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 // ---------------------------------------------------------------------------
@@ -753,6 +880,7 @@ bool qmv_supported(uint32_t type, size_t rows, size_t columns, const void *w, si
     const uint64_t row_bytes = (uint64_t)(columns / 256) * (type == kQ4_K ? 144 : 210);
     // Offsets are 32-bit: the matrix plus two rows of slack must fit.
     if (rows == 0 || row_bytes * (rows + 2) + 1024 >= 0xffffffffull) return false;
+    if ((uint64_t)batch * columns * 4 >= 0xffffffffull) return false;
     const uintptr_t a = (uintptr_t)w;
     if (type == kQ4_K ? (a & 15u) : (a & 3u)) return false;
     return true;
@@ -760,242 +888,125 @@ bool qmv_supported(uint32_t type, size_t rows, size_t columns, const void *w, si
 
 namespace {
 
-constexpr size_t kMaxLdsA = 56 * 1024;  // staged activation fragments; + split-K scratch <= 64 KiB
-
 struct Plan {
-    int nt, r, s, mb, g;
+    uint32_t kb, waves, wave_k, k_parts, row_groups, phases;
 };
 
-Plan choose_plan(uint32_t type, uint32_t rows, uint32_t blocks, uint32_t batch, int mode) {
-    Plan p;
-    p.nt = batch > 8 ? 2 : 1;
+// The K split.  A workgroup of 16 waves of up to 128 registers holds the
+// fragments of 8 tokens of up to 32 blocks (2 per wave; a gate/up pair, which
+// needs more registers besides, 16), one of 8 waves of 256 those of 16
+// tokens of 16 blocks, or of 8 tokens of a pair's 24.  Longer rows, and
+// matrices with fewer tiles than CUs, are split over k_parts workgroups;
+// gate/up pairs, whose epilogue needs whole sums, go through longer rows in
+// phases instead.  The split minimises the largest workgroup's share of the
+// weights; within it, the most waves share K.
+Plan choose_plan(uint32_t rows, uint32_t blocks, uint32_t batch, int mode, uint32_t cus) {
     const uint32_t tiles = (rows + 15) / 16;
-    const uint32_t spb = type == kQ4_K ? 9 : 8;
-    const size_t a_lds = ((size_t)blocks + 1) * spb * 4 * 2 * batch * 16;
-    p.mb = (batch <= 2 && a_lds <= kMaxLdsA) ? (int)(2 * batch) : 0;
-    // Two tiles per wave share each activation fragment load (batches above
-    // 2, one matrix, tall matrices); short matrices need the waves more.
-    p.r = (batch > 2 && mode != 2 && tiles >= 2048) ? 2 : 1;
-    const uint32_t rr = mode == 2 ? 2 * p.r : p.r;
-    // Blocks per staged group: 2 (runs of 2 blocks stream faster), or 1 when
-    // the row has a single block or LDS is short.
-    p.g = blocks >= 2 ? 2 : 1;
-    // Split each tile's block groups over S waves of a workgroup until the
-    // launch has about 4096 waves, with at least two groups per wave (S = 8
-    // only for prepared activations of up to 8 tokens, else S <= 4).
-    const uint32_t waves = (tiles + p.r - 1) / p.r;
-    const uint32_t s_max = (p.mb == 0 && p.nt == 1) ? 8 : 4;
-    uint32_t s = 1;
-    while (s < s_max && (size_t)waves * s < 4096 && (blocks + p.g - 1) / p.g >= 4 * s) s *= 2;
-    // Dynamic (activations, staging) plus static (split-K partials) LDS
-    // within the 160 KiB of a workgroup: first one block per group, then a
-    // narrower split.
-    for (;;) {
-        const uint32_t wv = s > 4 ? s : 4;
-        const size_t items = 16 * (type == kQ4_K ? 9 * p.g : (210 * p.g + 2 + 15) / 16);
-        const size_t lds = (p.mb > 0 ? a_lds : 0) + (size_t)wv * rr * items * 16 +
-                           (s > 1 ? (size_t)wv * rr * p.nt * 64 * 2 * 4 : 4) + 256;
-        if (lds <= 160 * 1024 || s == 1) break;
-        if (p.g == 2) {
-            p.g = 1;
+    Plan best{};
+    double best_cost = 0.0;
+    for (uint32_t parts = 1; parts <= 8 && parts <= blocks && parts <= cus; parts *= 2) {
+        if (parts > 1 &&
+            (mode == 2 || (uint64_t)tiles * (parts - 1) * ((batch + 1) / 2) * 16 > kQmvMeetWords))
+            break;
+        Plan p;
+        p.k_parts = parts;
+        const uint32_t part_blocks = (blocks + parts - 1) / parts;
+        p.phases = 1;
+        if (batch <= 8 && part_blocks <= (mode == 2 ? 16u : 32u)) {
+            p.waves = 16;
         } else {
-            s /= 2;
+            p.waves = 8;
+            if (part_blocks > (batch <= 8 ? 24u : 16u)) p.phases = (part_blocks + 15) / 16;
+        }
+        p.row_groups = cus / parts < tiles ? cus / parts : tiles;
+        const uint32_t phase_blocks = (part_blocks + p.phases - 1) / p.phases;
+        p.kb = (phase_blocks + p.waves - 1) / p.waves;
+        p.wave_k = (phase_blocks + p.kb - 1) / p.kb;
+        const uint32_t per = (tiles + p.row_groups - 1) / p.row_groups;
+        // tile blocks the busiest workgroup streams, plus the cost of a
+        // meeting (a round trip of an atomic, as long as about ten tile
+        // blocks) and of rebuilding the fragments of every pass
+        const double cost =
+            (double)per * part_blocks + (parts > 1 ? 10.0 : 0.0) + (p.phases > 1 ? 8.0 * p.phases * per : 0.0);
+        if (best.k_parts == 0 || cost < best_cost) {
+            best = p;
+            best_cost = cost;
         }
     }
-    p.s = (int)s;
-    return p;
+    return best;
 }
 
-struct Args {
-    const void *w, *w2;
-    uint32_t rows, columns, row_bytes, total;
-    const float *x;
-    int normalize;
-    float epsilon;
-    const _Float16 *xp;
-    const float *ysc;
-    uint32_t batch;
-    float *y;
-    ArgmaxPartial *partials;
-};
-
-template <uint32_t TYPE, int NT, int R, int S, int MODE, int MB, uint32_t G>
-hipError_t run(dmhip_ctx *ctx, const Args &a, uint32_t *waves_out) {
-    constexpr uint32_t SPB = Steps<TYPE>::value;
-    constexpr int RR = MODE == 2 ? 2 * R : R;
-    constexpr uint32_t WAVES = S > 4 ? S : 4;
-    const uint32_t tiles = (a.rows + 15) / 16;
-    const uint32_t per_wg = (WAVES / S) * R;
-    const uint32_t grid = (tiles + per_wg - 1) / per_wg;
-    // fragments of every block plus one zeroed block for the idle A rows,
-    // then each wave's weight staging area
-    const size_t lds = (MB > 0 ? ((size_t)(a.columns / 256) + 1) * SPB * 4 * MB * 16 : 0) +
-                       (size_t)WAVES * RR * StageQ<TYPE, G>::items * 16;
-    if (waves_out) *waves_out = grid * (WAVES / S);
-    auto kernel = qmv_kernel<TYPE, NT, R, S, MODE, MB, G>;
-    if (lds > 64 * 1024) {
-        static LdsLimit limit;
-        hipError_t e = limit.ensure((const void *)kernel, lds);
-        if (e != hipSuccess) return e;
-    }
-    return launch_kernel(ctx, kernel, dim3(grid), dim3(64 * WAVES), (uint32_t)lds, (const uint8_t *)a.w,
-                         (const uint8_t *)a.w2, a.rows, a.columns, a.row_bytes, a.total, a.x, a.normalize, a.epsilon,
-                         a.xp, a.ysc, a.batch, a.y, a.partials);
-}
-
-template <uint32_t TYPE, int NT, int R, int MODE, int MB, uint32_t G>
-hipError_t run_sg(dmhip_ctx *ctx, const Plan &p, const Args &a, uint32_t *w) {
-    if (p.s == 1) return run<TYPE, NT, R, 1, MODE, MB, G>(ctx, a, w);
-    if (p.s == 2) return run<TYPE, NT, R, 2, MODE, MB, G>(ctx, a, w);
-    if constexpr (MB == 0 && NT == 1) {
-        // the 8-wave split serves short matrices with prepared activations of
-        // up to 8 tokens (wider splits or two token groups outgrow the
-        // registers of the larger workgroup)
-        if (p.s == 8) return run<TYPE, NT, R, 8, MODE, MB, G>(ctx, a, w);
-    }
-    return run<TYPE, NT, R, 4, MODE, MB, G>(ctx, a, w);
-}
-
-template <uint32_t TYPE, int NT, int R, int MODE, int MB>
-hipError_t run_s(dmhip_ctx *ctx, const Plan &p, const Args &a, uint32_t *w) {
-    if (p.g == 2) return run_sg<TYPE, NT, R, MODE, MB, 2>(ctx, p, a, w);
-    return run_sg<TYPE, NT, R, MODE, MB, 1>(ctx, p, a, w);
+template <uint32_t TYPE, int NT, int MODE, int KB, uint32_t W, bool PHASED = false>
+hipError_t run(dmhip_ctx *ctx, const Plan &p, QmvArgs &a) {
+    // no more wave groups than a workgroup has tiles
+    const uint32_t tiles = (a.rows + 15) / 16, per = (tiles + p.row_groups - 1) / p.row_groups;
+    const uint32_t groups = W / p.wave_k, waves = (groups < per ? groups : per) * p.wave_k;
+    const uint32_t lds = waves * ring_depth<TYPE, NT, MODE, W, PHASED>() * StageQ<TYPE>::items * 16;
+    auto kernel = qmv_kernel<TYPE, NT, MODE, KB, W, PHASED>;
+    static LdsLimit limit;
+    hipError_t e = limit.ensure((const void *)kernel, lds);
+    if (e != hipSuccess) return e;
+    return launch_kernel(ctx, kernel, dim3(p.k_parts * p.row_groups), dim3(64 * waves), lds, a);
 }
 
 template <uint32_t TYPE, int MODE>
-hipError_t dispatch(dmhip_ctx *ctx, const Plan &p, const Args &a, uint32_t *w) {
-    if (p.mb == 2) return run_s<TYPE, 1, 1, MODE, 2>(ctx, p, a, w);
-    if (p.mb == 4) return run_s<TYPE, 1, 1, MODE, 4>(ctx, p, a, w);
-    if constexpr (MODE == 2) {
-        // the gate/up pair already streams two matrices: one tile per wave
-        return p.nt == 1 ? run_s<TYPE, 1, 1, MODE, 0>(ctx, p, a, w) : run_s<TYPE, 2, 1, MODE, 0>(ctx, p, a, w);
-    } else {
-        if (p.nt == 1)
-            return p.r == 1 ? run_s<TYPE, 1, 1, MODE, 0>(ctx, p, a, w) : run_s<TYPE, 1, 2, MODE, 0>(ctx, p, a, w);
-        return p.r == 1 ? run_s<TYPE, 2, 1, MODE, 0>(ctx, p, a, w) : run_s<TYPE, 2, 2, MODE, 0>(ctx, p, a, w);
+hipError_t dispatch(dmhip_ctx *ctx, uint32_t rows, uint32_t columns, const void *w, const void *w2, uint32_t batch,
+                    const float *x, int normalize, float epsilon, float *y) {
+    const uint32_t blocks = columns / 256;
+    const uint32_t cus = ctx->compute_units > 0 ? (uint32_t)ctx->compute_units : 256u;
+    const Plan p = choose_plan(rows, blocks, batch, MODE, cus);
+    QmvArgs a{(const uint8_t *)w, (const uint8_t *)w2, x, y, ctx->qmv_meet, rows, columns,
+              blocks * StageQ<TYPE>::bytes, batch, p.wave_k, p.k_parts, p.row_groups, p.phases, normalize, epsilon};
+    if (p.phases > 1)
+        return batch <= 8 ? run<TYPE, 1, MODE, 2, 8, true>(ctx, p, a) : run<TYPE, 2, MODE, 2, 8, true>(ctx, p, a);
+    if (batch > 8) return p.kb == 1 ? run<TYPE, 2, MODE, 1, 8>(ctx, p, a) : run<TYPE, 2, MODE, 2, 8>(ctx, p, a);
+    if (p.waves == 8) return run<TYPE, 1, MODE, 3, 8>(ctx, p, a);
+    if constexpr (MODE == 0) {
+        if (p.kb == 2) return run<TYPE, 1, MODE, 2, 16>(ctx, p, a);
     }
-}
-
-// Activation fragments for batches above 2 go to the context's aux scratch
-// (or, during an allocation-free call, to the scratch it lent the context):
-// [xp | yscale], written by the preparation kernel.
-hipError_t prepare(dmhip_ctx *ctx, uint32_t type, uint32_t columns, uint32_t batch, const float *x,
-                   int normalize, float eps, _Float16 **xp_out, float **ysc_out) {
-    const uint32_t spb = type == kQ4_K ? 9 : 8;
-    const size_t frags = (size_t)(columns / 256) * spb * 4;
-    const size_t xp_bytes = frags * 2 * batch * 8 * sizeof(_Float16);
-    const size_t need = ((xp_bytes + 255) & ~(size_t)255) + 64 * sizeof(float);
-    void *base;
-    if (ctx->aux_lent) {
-        if (need > ctx->aux_lent_bytes) return hipErrorOutOfMemory;
-        base = ctx->aux_lent;
-    } else {
-        if (ctx->aux.ensure(need) != DMHIP_OK) return hipErrorOutOfMemory;
-        base = ctx->aux.ptr;
-    }
-    _Float16 *xp = (_Float16 *)base;
-    float *ysc = (float *)((char *)base + ((xp_bytes + 255) & ~(size_t)255));
-    uint32_t gx = (uint32_t)((frags + 255) / 256);
-    if (gx > 64) gx = 64;
-    const dim3 grid(gx, batch);
-    if (columns <= kPrepareLdsColumns) {
-        const size_t lds = (size_t)columns * sizeof(float);
-        if (type == kQ4_K)
-            hipLaunchKernelGGL((qmv_prepare_kernel<kQ4_K, true>), grid, dim3(256), lds, ctx->stream, x,
-                               columns, batch, normalize, eps, xp, ysc);
-        else
-            hipLaunchKernelGGL((qmv_prepare_kernel<kQ6_K, true>), grid, dim3(256), lds, ctx->stream, x,
-                               columns, batch, normalize, eps, xp, ysc);
-    } else if (type == kQ4_K) {
-        hipLaunchKernelGGL((qmv_prepare_kernel<kQ4_K, false>), grid, dim3(256), 0, ctx->stream, x,
-                           columns, batch, normalize, eps, xp, ysc);
-    } else {
-        hipLaunchKernelGGL((qmv_prepare_kernel<kQ6_K, false>), grid, dim3(256), 0, ctx->stream, x,
-                           columns, batch, normalize, eps, xp, ysc);
-    }
-    *xp_out = xp;
-    *ysc_out = ysc;
-    return hipGetLastError();
+    return run<TYPE, 1, MODE, 1, 16>(ctx, p, a);
 }
 
 }  // namespace
 
+// What an allocation-free call sets aside for a matrix (the activation
+// fragments of the documented limit; the K-split partials use it).
 size_t qmv_prepare_bytes(uint32_t type, size_t columns, size_t batch) {
     const size_t spb = type == kQ4_K ? 9 : 8;
     const size_t xp_bytes = (columns / 256) * spb * 4 * 2 * batch * 8 * sizeof(_Float16);
     return ((xp_bytes + 255) & ~(size_t)255) + 64 * sizeof(float);
 }
 
-namespace {
-
-Args make_args(uint32_t type, uint32_t rows, uint32_t columns, const void *w, const void *w2,
-               uint32_t batch, const float *x, int normalize, float epsilon, float *y) {
-    Args a;
-    const uint32_t blocks = columns / 256;
-    a.w = w;
-    a.w2 = w2;
-    a.rows = rows;
-    a.columns = columns;
-    a.row_bytes = blocks * (type == kQ4_K ? 144u : 210u);
-    a.total = a.row_bytes * rows;
-    a.x = x;
-    a.normalize = normalize;
-    a.epsilon = epsilon;
-    a.xp = nullptr;
-    a.ysc = nullptr;
-    a.batch = batch;
-    a.y = y;
-    a.partials = nullptr;
-    return a;
-}
-
-}  // namespace
-
 hipError_t launch_qmv(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uint32_t columns, const void *w,
                       uint32_t batch, const float *x, float *y, ArgmaxState *argmax,
                       uint32_t *index_out) {
-    const bool int8_path = qmv8_supported(type, rows, columns, batch);
-    if (!argmax && int8_path) return launch_qmv8(ctx, type, rows, columns, w, batch, x, y, nullptr, nullptr);
-    Args a = make_args(type, rows, columns, w, w, batch, x, 0, 0.0f, y);
-    const Plan p = choose_plan(type, rows, columns / 256, batch, argmax ? 1 : 0);
-    if (!int8_path) {
-        hipError_t pe = prepare(ctx, type, columns, batch, x, 0, 0.0f, (_Float16 **)&a.xp, (float **)&a.ysc);
-        if (pe != hipSuccess) return pe;
-    }
-    if (!argmax)
-        return type == kQ4_K ? dispatch<kQ4_K, 0>(ctx, p, a, nullptr) : dispatch<kQ6_K, 0>(ctx, p, a, nullptr);
-    // One candidate per epilogue wave (at most one per 16-row tile), then a
-    // one-workgroup reduction.
-    const size_t candidates = (size_t)(rows + 15) / 16 + 4;
-    if (ctx->partials.ensure(candidates * sizeof(ArgmaxPartial)) != DMHIP_OK) return hipErrorOutOfMemory;
-    a.partials = (ArgmaxPartial *)ctx->partials.ptr;
-    uint32_t count = 0;
-    hipError_t e;
-    if (int8_path) {
-        // the int8 kernel's last workgroup publishes the argmax itself
-        return launch_qmv8(ctx, type, rows, columns, w, batch, x, y, a.partials, &count,
+    if (qmv8_supported(type, rows, columns, batch)) {
+        if (!argmax) return launch_qmv8(ctx, type, rows, columns, w, batch, x, y, nullptr, nullptr);
+        // the int8 kernel's last workgroup publishes the argmax itself; at
+        // most one candidate per 16-row tile otherwise
+        const size_t candidates = (size_t)(rows + 15) / 16 + 4;
+        if (ctx->partials.ensure(candidates * sizeof(ArgmaxPartial)) != DMHIP_OK) return hipErrorOutOfMemory;
+        uint32_t count = 0;
+        return launch_qmv8(ctx, type, rows, columns, w, batch, x, y, (ArgmaxPartial *)ctx->partials.ptr, &count,
                            ArgmaxFinish{argmax, index_out, ctx->argmax_ticket,
                                         (unsigned long long *)(ctx->argmax_ticket + 2)});
     }
-    e = type == kQ4_K ? dispatch<kQ4_K, 1>(ctx, p, a, &count) : dispatch<kQ6_K, 1>(ctx, p, a, &count);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(argmax_partials_kernel, dim3(1), dim3(kArgmaxThreads), 0, ctx->stream, a.partials, count,
-                       argmax, index_out);
-    return hipGetLastError();
+    const hipError_t e = type == kQ4_K
+                             ? dispatch<kQ4_K, 0>(ctx, rows, columns, w, nullptr, batch, x, 0, 0.0f, y)
+                             : dispatch<kQ6_K, 0>(ctx, rows, columns, w, nullptr, batch, x, 0, 0.0f, y);
+    if (e != hipSuccess || !argmax) return e;
+    return launch_argmax(ctx->stream, y, rows, argmax, index_out);
 }
 
 hipError_t launch_qmv_gate_up(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uint32_t columns,
                               const void *gate, const void *up, uint32_t batch, const float *x,
                               float *act, int normalize, float epsilon) {
-    Args a = make_args(type, rows, columns, gate, up, batch, x, normalize, epsilon, act);
-    const Plan p = choose_plan(type, rows, columns / 256, batch, 2);
-    hipError_t e = prepare(ctx, type, columns, batch, x, normalize, epsilon, (_Float16 **)&a.xp,
-                           (float **)&a.ysc);
-    if (e != hipSuccess) return e;
-    return type == kQ4_K ? dispatch<kQ4_K, 2>(ctx, p, a, nullptr) : dispatch<kQ6_K, 2>(ctx, p, a, nullptr);
+    return type == kQ4_K
+               ? dispatch<kQ4_K, 2>(ctx, rows, columns, gate, up, batch, x, normalize, epsilon, act)
+               : dispatch<kQ6_K, 2>(ctx, rows, columns, gate, up, batch, x, normalize, epsilon, act);
 }
 
 // A kernel of this file: resolving it loads the file's code object.
-const void *module_anchor_qmv() { return (const void *)argmax_partials_kernel; }
+const void *module_anchor_qmv() { return (const void *)qmv_kernel<kQ4_K, 1, 0, 1, 16, false>; }
 
 }  // namespace dm

@@ -1255,8 +1255,8 @@ hipError_t launch8(dmhip_ctx *ctx, uint32_t batch, int mode, const Args8 &a) {
     switch (batch) {
     case 1: return run8_g<TYPE, 0, 1>(ctx, p, a);
     case 2: return run8_g<TYPE, 0, 2>(ctx, p, a);
-    case 3: return run8_g<TYPE, 0, 3>(ctx, p, a);
-    default: return run8_g<TYPE, 0, 4>(ctx, p, a);
+    case 3: return TYPE == kQ6_K ? hipErrorInvalidValue : run8_g<TYPE == kQ6_K ? kQ4_K : TYPE, 0, 3>(ctx, p, a);
+    default: return TYPE != kQ8_0 ? hipErrorInvalidValue : run8_g<kQ8_0, 0, 4>(ctx, p, a);
     }
 }
 
@@ -1265,22 +1265,33 @@ hipError_t launch8(dmhip_ctx *ctx, uint32_t batch, int mode, const Args8 &a) {
 bool qmv8_supported(uint32_t type, size_t rows, size_t columns, size_t batch) {
     if (type != kQ4_K && type != kQ6_K && type != kQ8_0) return false;
     if (batch < 1 || batch > kMaxTokens8 || columns % 256 || columns == 0) return false;
-    // 3-4 tokens of Q4_K / Q6_K: the int8 kernel against the fp16 one and its
-    // preparation launch, measured per launch on MI355X: 4096 x 4096 Q4_K
-    // 7.4 / 8.5 us against 11.0 us, Q6_K 9.4 / 10.8 against 12.3 us, but
-    // 12288 x 4096 Q4_K 17.4 / 21.1 against 17.7 / 17.8 us (the records of
-    // every token make each block's work longer than its bytes take to
-    // arrive).  Q8_0 has only this kernel.
-    if (batch > 2 && type != kQ8_0 && (uint64_t)rows * columns > (20ull << 20)) return false;
+    // Q4_K / Q6_K of several tokens: the int8 kernel against the fp16 one,
+    // measured per launch on MI355X.  The int8 kernel takes each token's
+    // records through the matrix cores apart, so its work per block grows with
+    // the tokens; the fp16 one costs as much for 1 token as for 8, and its
+    // prologue about 2 us more.
+    //  2 tokens: Q4_K 4096 x 5120 6.5 against 9.1 us, 6144 x 4096 9.6 against
+    //    8.5, 20000 x 4096 15.3 against 12.7, 32768 x 4096 16.0 against 16.7;
+    //    Q6_K 4096 x 5120 8.5 against 9.5, 8192 x 4096 11.8 against 9.7,
+    //    32768 x 4096 29.8 against 25.9, 151936 x 4096 103 against 112.
+    //  3 tokens: Q4_K 4096 x 4096 6.8 against 7.1, 1024 x 4096 6.6 against
+    //    5.2; Q6_K 4096 x 4096 8.7 against 7.5.
+    // From 4 tokens on the fp16 kernel is faster throughout.
+    if (type != kQ8_0) {
+        const uint64_t weights = (uint64_t)rows * columns, m = 1u << 20;
+        if (batch > 3) return false;
+        if (batch == 3 && (type == kQ6_K || rows < 2048 || weights > 20 * m)) return false;
+        if (batch == 2 && weights > 22 * m && weights <= (type == kQ4_K ? 100 * m : 300 * m)) return false;
+    }
     return plan8(type, (uint32_t)rows, (uint32_t)columns, (uint32_t)batch, 1).s != 0;
 }
 
 bool qmv8_gate_up_supported(uint32_t type, size_t rows, size_t columns, size_t batch) {
     if (type != kQ4_K && type != kQ6_K) return false;
     // Gate/up pairs of 3-4 tokens measured slower here than on the fp16
-    // kernels with their preparation launch (C3, Q4_K 12288 x 4096, 4
-    // tokens: 37.5 us against 19.4 + 4.6 us): the records of both matrices'
-    // token blocks leave one 8-wave workgroup per CU.
+    // kernel (C3, Q4_K 12288 x 4096, 4 tokens: 37.5 us against 19 us): the
+    // records of both matrices' token blocks leave one 8-wave workgroup per
+    // CU.  Pairs of 2 tokens take 16.4 us here against 17.7 us.
     if (batch < 1 || batch > 2 || columns % 256 || columns == 0) return false;
     return plan8(type, (uint32_t)rows, (uint32_t)columns, (uint32_t)batch, 2).s != 0;
 }

@@ -104,8 +104,8 @@ struct dmhip_ctx {
     dm::Scratch attn;                        // attention chunk partials
     dm::Scratch attn_tickets;                // attention combine counters, zero between calls
     size_t attn_ticket_count = 0;            // counters in attn_tickets already zeroed
-    // Device memory an allocation-free call lends the fp16 path in place of
-    // `aux` for its duration (null otherwise).
+    // Device memory an allocation-free call lends the fp16 matvec (K-split
+    // partial sums) in place of `aux` for its duration (null otherwise).
     void *aux_lent = nullptr;
     size_t aux_lent_bytes = 0;
     dm::ArgmaxState *argmax_state = nullptr;  // device
@@ -114,6 +114,7 @@ struct dmhip_ctx {
     uint32_t attn_mark = 0;                   // mark of the last attention call (flags[kAttnFlagWord])
     uint32_t *argmax_ticket = nullptr;        // device, zero between launches: ticket, then (at +8) the best key
     uint32_t *argmax_index = nullptr;         // device
+    uint64_t *qmv_meet = nullptr;             // device, kQmvMeetWords words, all ones between launches
     uint32_t *flags = nullptr;                // device: [0] router, [1] read probe, [2] top-k, [3] MoE router, [4] attention
     bool argmax_pending = false;
     bool router_pending = false;  // a dmhip_router_top_k_device awaits dmhip_router_result

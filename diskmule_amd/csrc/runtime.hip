@@ -469,12 +469,14 @@ int dmhip_context_new(int device, dmhip_ctx **out) {
         hipMalloc((void **)&ctx->flags, 64) != hipSuccess ||
         hipMalloc((void **)&ctx->argmax_ticket, 64) != hipSuccess ||
         hipMalloc((void **)&ctx->router_tickets, kRouterTickets * 4) != hipSuccess ||
+        hipMalloc((void **)&ctx->qmv_meet, kQmvMeetWords * 8) != hipSuccess ||
         // Counters start at zero.  Cleared by the library's own fill kernel:
         // the first launch from the library's code object materialises its
         // data (the allocation-free entry point's scratch array) on this
         // device here, at set-up, rather than inside a later call.
         launch_fill_u32(ctx->stream, ctx->argmax_ticket, 16, 0) != hipSuccess ||
         launch_fill_u32(ctx->stream, ctx->router_tickets, kRouterTickets, 0) != hipSuccess ||
+        launch_fill_u32(ctx->stream, (uint32_t *)ctx->qmv_meet, kQmvMeetWords * 2, ~0u) != hipSuccess ||
         launch_fill_u32(ctx->stream, ctx->flags, 16, 0) != hipSuccess ||
         hipHostMalloc((void **)&ctx->done_word, 64, hipHostMallocDefault) != hipSuccess ||
         hipHostGetDevicePointer(&ctx->done_word_dev, (void *)ctx->done_word, 0) != hipSuccess ||
@@ -511,6 +513,7 @@ void dmhip_context_free(dmhip_ctx *ctx) {
     if (ctx->argmax_state) (void)hipFree(ctx->argmax_state);
     if (ctx->argmax_ticket) (void)hipFree(ctx->argmax_ticket);
     if (ctx->router_tickets) (void)hipFree(ctx->router_tickets);
+    if (ctx->qmv_meet) (void)hipFree(ctx->qmv_meet);
     if (ctx->argmax_index) (void)hipFree(ctx->argmax_index);
     if (ctx->flags) (void)hipFree(ctx->flags);
     if (ctx->done_word) (void)hipHostFree((void *)ctx->done_word);

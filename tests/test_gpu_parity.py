@@ -233,6 +233,57 @@ def test_batched_gemv_short_and_misaligned_shapes(ctx, kind, rows, cols, batch):
         assert_channel_close(got[b], exact[b], scale[b], CHANNEL_TOL_GEMV, f"token {b}")
 
 
+@pytest.mark.parametrize("kind,rows,cols,batch", [
+    (Q4_K, 40, 256, 4), (Q6_K, 777, 768, 13),       # one block, one wave; three waves sharing K
+    (Q4_K, 4100, 4096, 8), (Q6_K, 2048, 8192, 5),   # 16 waves of one and of two blocks
+    (Q4_K, 65, 2304, 16), (Q6_K, 300, 4096, 9),     # 16 tokens: 8 waves of two blocks, of one
+    (Q6_K, 1000, 12288, 8), (Q4_K, 130, 4608, 7),   # K split over 2 to 8 workgroups
+    (Q4_K, 5000, 13824, 6), (Q6_K, 70, 13824, 16),
+    (Q4_K, 20, 69632, 6), (Q6_K, 200, 34816, 12),     # K beyond every split: in phases
+])
+def test_batched_gemv_plans(ctx, kind, rows, cols, batch):
+    """Every plan of the fp16 matvec at its edges, x at a 4-byte boundary: each
+    channel within the GEMV bar of the exact product (22-bit activations and
+    fp32 sums, as derived in tolerance.py), and repeated calls bit-identical
+    whichever workgroup of a K split comes first."""
+    w = synth.quantized_matrix(kind, rows, cols, synth.weight_seed(160, rows))
+    if kind == Q6_K:  # scales over their whole int8 range, as quantizers leave them
+        w.reshape(-1, 210)[:, 192:208] = np.random.default_rng(rows).integers(0, 256, (w.size // 210, 16))
+    x = synth.normal(synth.activation_seed(160, cols), batch * cols).reshape(batch, cols)
+    wb, yb = dev(ctx, w), dev_out(ctx, batch * rows * 4)
+    xb = dev(ctx, np.concatenate([np.zeros(1, np.float32), x.ravel()]))
+    runs = []
+    for _ in range(3):
+        ctx.matvec_device(kind, rows, cols, wb.device_ptr, batch, xb.device_ptr + 4, yb.device_ptr)
+        runs.append(yb.read(0, batch * rows * 4, np.float32).copy())
+    assert all(np.array_equal(bits(r), bits(runs[0])) for r in runs[1:])
+    got = runs[0].reshape(batch, rows)
+    pick = np.unique(np.linspace(0, rows - 1, min(rows, 512)).astype(int))  # 512 rows of a tall matrix
+    part = np.ascontiguousarray(w.reshape(rows, -1)[pick]).ravel()
+    exact, scale = exact_products(kind, pick.size, cols, part, x)
+    assert_channel_close(got[:, pick], exact, scale, CHANNEL_TOL_GEMV, f"type {kind} {rows}x{cols} batch {batch}")
+
+
+@pytest.mark.parametrize("hidden,ffn,batch", [(2048, 530, 3), (5120, 300, 8), (7168, 200, 4), (4096, 2100, 16),
+                                              (5120, 700, 12)])
+def test_batched_ffn_plans(ctx, hidden, ffn, batch):
+    """The gate/up pairs' plans (16 and 8 waves, phases) with the RMSNorm and
+    the SiLU folded in, against the oracle."""
+    ffn = -(-ffn // 256) * 256
+    mats = [synth.quantized_matrix(k, r, c, synth.weight_seed(161, i))
+            for i, (k, r, c) in enumerate(((Q4_K, ffn, hidden), (Q4_K, ffn, hidden), (Q6_K, hidden, ffn)))]
+    h = synth.normal(synth.activation_seed(161, batch), batch * hidden).reshape(batch, hidden)
+    g, u, d = (dev(ctx, m) for m in mats)
+    hb, yb = dev(ctx, h), dev_out(ctx, batch * hidden * 4)
+    ws = dev_out(ctx, ctx.ffn_workspace_bytes(batch, hidden, ffn))
+    ctx.ffn_device(batch, hidden, ffn, Q4_K, g.device_ptr, Q4_K, u.device_ptr, Q6_K, d.device_ptr, 1e-6,
+                   hb.device_ptr, yb.device_ptr, ws.device_ptr, len(ws))
+    got = yb.read(0, batch * hidden * 4, np.float32).reshape(batch, hidden)
+    want = capi.dense_ffn(batch, hidden, ffn, Q4_K, mats[0], Q4_K, mats[1], Q6_K, mats[2], h)
+    for b in range(batch):
+        assert_close(got[b], want.reshape(batch, hidden)[b], f"ffn {hidden}/{ffn} batch {batch} token {b}")
+
+
 @pytest.mark.parametrize("kind,rows,cols,x_stride", [(Q4_K, 1000, 2048, 0), (Q6_K, 1000, 2048, 2048),
                                                      (Q4_K, 4096, 4096, 0), (Q8_0, 300, 512, 512)])
 def test_matvec_batch_matches_one_matvec_per_matrix(ctx, kind, rows, cols, x_stride):
