@@ -94,7 +94,7 @@ hipError_t launch_top_k(hipStream_t s, const float *logits, uint32_t rows, uint3
 // token t, the addresses at [t * k + s], and per token a go word (device and
 // pinned host copies): 1 when every selected expert of the token is resident
 // and its logits are finite, else 0.
-constexpr uint32_t kMaxLookupTokens = 8;
+constexpr uint32_t kMaxLookupTokens = 16;
 struct ExpertLookup {
     const uint64_t *gate_up_of, *down_of;
     uint64_t *gate_up_w, *down_w;

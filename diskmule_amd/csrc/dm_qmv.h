@@ -95,6 +95,17 @@ hipError_t launch_qmv8_grouped(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uin
 // whole 256-value super-blocks at a 16-byte aligned base, batch 1-2.
 bool qmv_supported(uint32_t type, size_t rows, size_t columns, const void *w, size_t batch);
 
+// The routed experts of a layer call on the fp16 kernel, their tokens grouped
+// on the device: pair i (selection i % k of token i / k) goes to expert ids[i],
+// whose rows are at w_of[expert] (16-byte aligned); nothing is done unless
+// go[0 .. tokens) are all 1 (ids, go: written by a kernel earlier on the
+// stream).  gate_up: y[i] = (g / (1 + exp(-g))) * u for token i / k's row of x
+// (the up rows up_offset bytes from the gate rows); otherwise y[i] = W x[i].
+bool qmv_experts_supported(uint32_t type, size_t rows, size_t columns, size_t experts, size_t pairs, size_t x_rows);
+hipError_t launch_qmv_experts(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uint32_t columns, bool gate_up,
+                              uint64_t up_offset, const uint64_t *w_of, const uint32_t *ids, const uint32_t *go,
+                              uint32_t tokens, uint32_t k, const float *x, float *y);
+
 // Bytes of the activation fragments the fp16 kernel prepares for `batch`
 // tokens (batches above 2) of rows of `columns` values.
 size_t qmv_prepare_bytes(uint32_t type, size_t columns, size_t batch);

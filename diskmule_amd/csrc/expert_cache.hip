@@ -76,9 +76,11 @@ __global__ void moe_combine_pos_kernel(const float *__restrict__ expert_out,
                                        uint32_t batch, uint32_t k, uint32_t hidden,
                                        float *__restrict__ y, const uint32_t *__restrict__ go) {
     // the device-side lookup found a slot missing (go: one word per token)
-    if (go)
-        for (uint32_t t = 0; t < batch; t++)
-            if (go[t] == 0) return;
+    // (every word read at once: up to 16 tokens)
+    if (go) {
+        const uint32_t t = threadIdx.x & 63u;
+        if (__builtin_amdgcn_ballot_w64(t < batch && go[t] == 0)) return;
+    }
     for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < (size_t)batch * hidden;
          e += (size_t)gridDim.x * blockDim.x) {
         uint32_t t = (uint32_t)(e / hidden), i = (uint32_t)(e - (size_t)t * hidden);
@@ -194,6 +196,14 @@ namespace {
 constexpr size_t kSelectionPairs = 16 * dm::kMaxTopK;  // batch <= 16
 constexpr size_t kSelectionBytes = kSelectionPairs * 8 + 16 * 4 + 16 * 4;  // ids, probabilities, per-token flags, go
 constexpr size_t kReleaseEvents = 64;
+// Layer calls whose selected experts' bytes, counted per pair, reach this
+// group the tokens by expert on the device (launch_qmv_experts).  Measured on
+// MI355X, one job per pair against grouped: 2048 x 768, 128 experts top 8
+// (24.5 MB a token) 2 / 4 / 6 / 8 tokens 46 / 62 / 77 / 87 against
+// 52 / 63 / 75 / 83 us; 4096 x 1536, 32 experts top 4 (49 MB a token) 2 / 4 / 8
+// tokens 52 / 77 / 109 against 61 / 77 / 98 us; 1024 x 512, 60 experts top 2 8
+// tokens (12 MB in all) 37 against 46 us.
+constexpr size_t kExpertGroupBytes = 140u << 20;
 constexpr size_t kCombineTickets = 4096;  // row-tile workgroups of a fused down + combine launch
 constexpr size_t kStagingEntries = 4;  // file source: experts in flight from storage
 // Memory source: uploads whose timing is kept until it is read.  The ring is
@@ -761,7 +771,14 @@ int dmhip_moe_layer(dmhip_ctx *ctx, dmhip_expert_cache *c, size_t layer, size_t 
     // path below with the selection in hand.  Every earlier upload is
     // already waited for on the compute stream, before the table copy and
     // the router.
-    const bool lookup = Lay.try_lookup && grouped && pairs <= kMaxGroupedJobs &&
+    // Grouping streams each expert once for all its tokens; its launches cost
+    // about 8 us more than those of one job per pair, whose bytes grow with
+    // the pairs.
+    const bool by_expert = (batch > 8 || pairs > kMaxGroupedJobs ||
+                            pairs * (L.gate_up_bytes + L.down_bytes) >= kExpertGroupBytes) &&
+                           qmv_experts_supported(gate_up_type, width, hidden, experts, pairs, batch) &&
+                           qmv_experts_supported(down_type, hidden, width, experts, pairs, pairs);
+    const bool lookup = Lay.try_lookup && grouped && (by_expert || (batch <= 8 && pairs <= kMaxGroupedJobs)) &&
                         router_takes_lookup((uint32_t)hidden, (uint32_t)experts, (uint32_t)batch, router_bf16, x);
     if (lookup) {
         for (size_t t = 0; t < batch; t++) sel_go[t] = 0;
@@ -776,13 +793,24 @@ int dmhip_moe_layer(dmhip_ctx *ctx, dmhip_expert_cache *c, size_t layer, size_t 
         DM_HIP(launch_router_top_k(ctx->stream, router_bf16, (uint32_t)hidden, (uint32_t)experts, (uint32_t)k,
                                    (uint32_t)batch, x, d_logits, d_ids, d_probs, BadFlag{ctx->flags + kMoeFlagWord, 1},
                                    sel_ids, sel_probs, ctx->router_tickets, sel_bad, &el, true));
+        const uint32_t tokens = (uint32_t)batch;
+        if (by_expert) {
+            DM_HIP(launch_qmv_experts(ctx, gate_up_type, (uint32_t)width, (uint32_t)hidden, true, up_offset, Lay.table,
+                                      d_ids, c->lookup_go, tokens, (uint32_t)k, x, d_act));
+            DM_HIP(launch_qmv_experts(ctx, down_type, (uint32_t)hidden, (uint32_t)width, false, 0,
+                                      Lay.table + L.expert_count, d_ids, c->lookup_go, tokens, (uint32_t)k, d_act,
+                                      d_eo));
+            hipLaunchKernelGGL(moe_combine_pos_kernel, dim3((uint32_t)((batch * hidden + 255) / 256)), dim3(256), 0,
+                               ctx->stream, d_eo, nullptr, d_probs, tokens, (uint32_t)k, (uint32_t)hidden, y,
+                               c->lookup_go);
+            DM_HIP(hipGetLastError());
+        } else {
         // job p: selection p % k of token p / k
         std::vector<QmvJob> gu_jobs(pairs), dn_jobs(pairs);
         for (size_t p = 0; p < pairs; p++) {
             gu_jobs[p] = QmvJob{nullptr, 1u, (uint32_t)(p / k * hidden), (uint32_t)(p * width), 0, 0};
             dn_jobs[p] = QmvJob{nullptr, 1u, (uint32_t)(p * width), (uint32_t)(p * hidden), 0, 0};
         }
-        const uint32_t tokens = (uint32_t)batch;
         DM_HIP(launch_qmv8_grouped(ctx, gate_up_type, (uint32_t)width, (uint32_t)hidden, 1, up_offset,
                                    gu_jobs.data(), pairs, x, d_act, c->lookup_gate_up, c->lookup_go, nullptr, tokens));
         // the down launch also makes the ordered combine when its split
@@ -797,6 +825,7 @@ int dmhip_moe_layer(dmhip_ctx *ctx, dmhip_expert_cache *c, size_t layer, size_t 
                                ctx->stream, d_eo, nullptr, d_probs, tokens, (uint32_t)k, (uint32_t)hidden, y,
                                c->lookup_go);
             DM_HIP(hipGetLastError());
+        }
         }
     } else {
         DM_HIP(launch_router_top_k(ctx->stream, router_bf16, (uint32_t)hidden, (uint32_t)experts,

@@ -382,6 +382,19 @@ struct QmvArgs {
     float epsilon;
 };
 
+// The routed experts of a MoE layer call (GROUPED): pair i of `pairs` is
+// selection i % k of token i / k, expert ids[i]; expert e's matrix is at
+// w_of[e] (the up rows at w2_offset bytes from it).  Nothing is done unless
+// go[0 .. go_count) are all 1.  Input row of a pair: its token's (k = 0: its
+// own); output row: the pair's.
+struct QmvExperts {
+    const uint64_t *w_of;
+    uint64_t w2_offset;
+    const uint32_t *ids, *go;
+    uint32_t go_count, pairs, k, x_rows;
+};
+constexpr uint32_t kGroupExperts = 256, kGroupPairs = 128;
+
 // Two tokens' sums of one row as one word; a NaN becomes the canonical one,
 // so no published pair equals kMeetEmpty.
 __device__ __forceinline__ uint64_t pack_pair(float a, float b) {
@@ -389,16 +402,18 @@ __device__ __forceinline__ uint64_t pack_pair(float a, float b) {
     return (uint64_t)ub << 32 | ua;
 }
 
-// Tiles of a wave group between two cross-wave sums, whose LDS (red) leaves
-// room for the ring.
+// Tiles of a wave group between two cross-wave sums of all 8 NT tokens, whose
+// LDS (red) leaves room for the ring; fewer tokens take less, and then more
+// tiles share a sum.
 template <int MODE, bool PHASED> constexpr uint32_t pass_tiles() { return (MODE == 2 ? 2 : 4) / (PHASED ? 2 : 1); }
 template <int NT, int MODE, uint32_t W, bool PHASED> constexpr uint32_t red_floats() {
     return W * pass_tiles<MODE, PHASED>() * (MODE == 2 ? 2 : 1) * NT * 2 * 64;
 }
 // Slots of a wave's ring (one being read, the others in flight): what the
-// 160 KiB of LDS hold, at most 5 or 4 (first_loads).
-template <uint32_t TYPE, int NT, int MODE, uint32_t W, bool PHASED> constexpr uint32_t ring_depth() {
-    constexpr uint32_t fit = (156 * 1024 - red_floats<NT, MODE, W, PHASED>() * 4 - (PHASED ? W * 2048 : 0)) /
+// 160 KiB of LDS (GROUPED: of two workgroups) hold, at most 5 or 4 (first_loads).
+template <uint32_t TYPE, int NT, int MODE, uint32_t W, bool PHASED, bool GROUPED = false>
+constexpr uint32_t ring_depth() {
+    constexpr uint32_t fit = ((GROUPED ? 155 * 512 : 156 * 1024) - red_floats<NT, MODE, W, PHASED>() * 4 - (PHASED ? W * 2048 : 0)) /
                              (W * StageQ<TYPE>::items * 16);
     constexpr uint32_t most = TYPE == kQ4_K ? 5 : 4;
     return fit < most ? fit : most;
@@ -443,6 +458,11 @@ __device__ __forceinline__ void first_loads(floatx4 (&x)[XB][8], v4u xr, uint32_
                      : DM_OUT(a, 0), [l] "+&s"(lds)
                      : DM_ARGS, DM_IN3(0), DM_IN3(1), DM_IN3(2), DM_IN3(3)
                      : "memory", "scc");
+    } else if constexpr (TYPE == kQ4_K && XB == 1 && SLOTS == 3) {
+        asm volatile(DM_XQ4 DM_Q4(0) DM_NEXT(2304) DM_Q4(1) DM_NEXT(2304) DM_Q4(2) "s_waitcnt vmcnt(9)"
+                     : DM_OUT(a, 0), [l] "+&s"(lds)
+                     : DM_ARGS, DM_IN3(0), DM_IN3(1), DM_IN3(2)
+                     : "memory", "scc");
     } else if constexpr (TYPE == kQ4_K && XB == 2 && SLOTS == 2) {
         asm volatile(DM_XQ4 DM_XQ4B DM_Q4(0) DM_NEXT(2304) DM_Q4(1) "s_waitcnt vmcnt(6)"
                      : DM_OUT(a, 0), DM_OUT(b, 1), [l] "+&s"(lds)
@@ -452,6 +472,11 @@ __device__ __forceinline__ void first_loads(floatx4 (&x)[XB][8], v4u xr, uint32_
         asm volatile(DM_XQ6 DM_Q6(0) "s_waitcnt vmcnt(4)"
                      : DM_OUT(a, 0), [l] "+&s"(lds)
                      : DM_ARGS, DM_IN4(0)
+                     : "memory", "scc");
+    } else if constexpr (TYPE == kQ6_K && XB == 1 && SLOTS == 2) {
+        asm volatile(DM_XQ6 DM_Q6(0) DM_NEXT(3584) DM_Q6(1) "s_waitcnt vmcnt(8)"
+                     : DM_OUT(a, 0), [l] "+&s"(lds)
+                     : DM_ARGS, DM_IN4(0), DM_IN4(1)
                      : "memory", "scc");
     } else if constexpr (TYPE == kQ6_K && XB == 1 && SLOTS == 3) {
         asm volatile(DM_XQ6 DM_Q6(0) DM_NEXT(3584) DM_Q6(1) DM_NEXT(3584) DM_Q6(2) "s_waitcnt vmcnt(12)"
@@ -499,17 +524,17 @@ __device__ __forceinline__ void first_loads(floatx4 (&x)[XB][8], v4u xr, uint32_
 // of one block beat 8 of two (12.6 us at 12288 x 4096): four waves per SIMD
 // hide each other's LDS and MFMA latency.
 // ---------------------------------------------------------------------------
-template <uint32_t TYPE, int NT, int MODE, int KB, uint32_t W, bool PHASED>
-__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
-qmv_kernel(const QmvArgs p) {
+template <uint32_t TYPE, int NT, int MODE, int KB, uint32_t W, bool PHASED, bool GROUPED>
+__device__ __forceinline__ void qmv_body(const QmvArgs &p, uint32_t part, uint32_t rg, uint32_t x_rows,
+                                         const uint32_t *x_row, const uint32_t *y_row) {
     constexpr uint32_t BB = StageQ<TYPE>::bytes;
     constexpr uint32_t RR = MODE == 2 ? 2 : 1;  // matrices streamed
-    constexpr uint32_t DEPTH = ring_depth<TYPE, NT, MODE, W, PHASED>();
+    constexpr uint32_t DEPTH = ring_depth<TYPE, NT, MODE, W, PHASED, GROUPED>();
     static_assert(DEPTH >= 2, "a slot in flight while one is read");
     using ST = StageQ<TYPE>;
     constexpr uint32_t CH = ST::chunks, NL = ST::loads;
     constexpr uint32_t SLOT = ST::items;      // chunks of a ring slot
-    constexpr uint32_t PI = pass_tiles<MODE, PHASED>() * RR;  // items of a wave per pass
+    constexpr uint32_t PI = pass_tiles<MODE, PHASED>() * RR;  // items of a wave per pass (of 8 NT tokens)
     __shared__ v4u red_all[red_floats<NT, MODE, W, PHASED>() / 4];
     __shared__ v4u split_all[PHASED ? W * 128 : 1];
     __shared__ uint32_t s_min[W * 64];  // 8 tokens x {hi, lo} x 4 lane groups
@@ -522,7 +547,6 @@ qmv_kernel(const QmvArgs p) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t n = lane & 15u, kg = lane >> 4;
     const uint32_t wk = p.wave_k, wt = (blockDim.x >> 6) / wk, kw = wave % wk, wg = wave / wk;
-    const uint32_t part = blockIdx.x % p.k_parts, rg = blockIdx.x / p.k_parts;
     const uint32_t blocks = p.columns / 256, tiles = (p.rows + 15) / 16;
     const uint32_t t_begin = (uint32_t)((uint64_t)rg * tiles / p.row_groups);
     const uint32_t t_end = (uint32_t)((uint64_t)(rg + 1) * tiles / p.row_groups);
@@ -545,7 +569,11 @@ qmv_kernel(const QmvArgs p) {
     struct Pos {
         uint32_t tile0, phase, i;  // first tile of the pass
     };
-    const uint32_t pass_step = pass_tiles<MODE, PHASED>() * wt;
+    // Token pairs kept per item of red (a power of two), and how many more
+    // items a pass has for it.
+    const uint32_t pairs = (p.batch + 1) / 2, pp = pairs <= 1 ? 1u : pairs <= 2 ? 2u : pairs <= 4 ? 4u : 8u;
+    const uint32_t more = NT * 4 / pp, pass_items = PI * more;
+    const uint32_t pass_step = pass_tiles<MODE, PHASED>() * more * wt;
     auto items = [&](uint32_t tile0) {  // items per wave and phase of the pass at tile0
         const uint32_t left = t_end - tile0, t = left < pass_step ? left : pass_step;
         return (t + wt - 1) / wt * RR;
@@ -612,10 +640,10 @@ qmv_kernel(const QmvArgs p) {
     // through LDS to the lanes that hold the token's A rows, a round (2 KiB)
     // at a time: the quad (kg, c) of token i is at slot (4 kg + c) ^ i of 16
     // (so neither side meets bank conflicts), hi pairs then lo pairs.  The
-    // area is the wave's part of red before the first pass, or (PHASED) LDS of
-    // its own; a wave reads only what it wrote.
+    // area is the ring slot the prologue leaves free, or (PHASED) LDS of its
+    // own; a wave reads only what it wrote.
     const uint32_t li = lane >> 4, lk = (lane >> 2) & 3u, lc = lane & 3u;
-    uint32_t *sp = (uint32_t *)(PHASED ? split_all : red_all) + wave * (PHASED ? 512 : PI * NT * 128);
+    uint32_t *sp = PHASED ? (uint32_t *)split_all + wave * 512 : (uint32_t *)(ring + (DEPTH - 1) * SLOT);
     uint32_t *smn = s_min + wave * 64;
     auto split = [&](int g, int b, uint32_t phase, const floatx4 (&x4)[8]) {
         const bool used = k_begin(phase) + b < k_end(phase);
@@ -684,11 +712,13 @@ qmv_kernel(const QmvArgs p) {
     // Byte of x that load (u, 0) of a block takes (tokens past the batch read
     // past the end: zeros).
     auto x_byte = [&](int g, uint32_t blk, int u) {
-        return ((8 * g + 4 * u + li) * p.columns + blk * 256 + round_column<TYPE>(lk) + 4 * lc) * 4;
+        const uint32_t i = 8 * g + 4 * u + li;
+        const uint32_t at = ((GROUPED ? x_row[i] : i) * p.columns + blk * 256 + round_column<TYPE>(lk) + 4 * lc) * 4;
+        return GROUPED && i >= p.batch ? 0xfffff000u : at;
     };
-    const v4u xr = v4u{(uint32_t)(uintptr_t)p.x, (uint32_t)((uintptr_t)p.x >> 32) & 0xffffu, p.batch * p.columns * 4,
-                       0x00020000u};
-    const __amdgpu_buffer_rsrc_t xrs = make_rsrc(p.x, p.batch * p.columns * 4);
+    const uint32_t x_bytes = x_rows * p.columns * 4;
+    const v4u xr = v4u{(uint32_t)(uintptr_t)p.x, (uint32_t)((uintptr_t)p.x >> 32) & 0xffffu, x_bytes, 0x00020000u};
+    const __amdgpu_buffer_rsrc_t xrs = make_rsrc(p.x, x_bytes);
     auto load_x = [&](int g, int b, uint32_t phase, floatx4 (&x4)[8]) {
 #pragma unroll
         for (int i = 0; i < 8; i++)
@@ -785,14 +815,17 @@ qmv_kernel(const QmvArgs p) {
                 }
                 slot = slot + 1 == DEPTH ? 0 : slot + 1;
             }
-            float *sl = &red[((wave * PI + cur.i) * NT * 2) * 64 + lane];
+            // row n, token pair 4 g + kg: two runs of 16 rows
+            float *sl = &red[(wave * pass_items + cur.i) * pp * 32 + n];
 #pragma unroll
-            for (int g = 0; g < NT; g++)
+            for (int g = 0; g < NT; g++) {
+                if (4 * g + kg >= pp) continue;
 #pragma unroll
                 for (int j = 0; j < 2; j++) {
-                    float &s = sl[(2 * g + j) * 64];
+                    float &s = sl[(4 * g + kg) * 32 + j * 16];
                     s = !PHASED || cur.phase == 0 ? acc[g][j] : s + acc[g][j];
                 }
+            }
             advance(cur);
         } while (cur.tile0 == tile0);
         first_pass = false;
@@ -801,11 +834,8 @@ qmv_kernel(const QmvArgs p) {
         // a tile, tokens tk and tk + 1.
         lds_barrier();
         const uint32_t left = t_end - tile0, nt = left < pass_step ? left : pass_step;
-        const uint32_t pairs = (p.batch + 1) / 2;
         for (uint32_t idx = threadIdx.x; idx < nt * 16 * pairs; idx += blockDim.x) {
             const uint32_t rn = idx & 15u, pair = (idx >> 4) / nt, tl = (idx >> 4) - pair * nt;
-            // tokens 8 g + 2 kg + {0, 1}: lane rn + 16 kg, elements 2 g + {0, 1}
-            const uint32_t el = 2 * (pair >> 2), ln = rn + 16 * (pair & 3u);
             const uint32_t group = tl % wt, sl = tl / wt, tk = 2 * pair, row = (tile0 + tl) * 16 + rn;
             float v[RR][2];
 #pragma unroll
@@ -813,9 +843,9 @@ qmv_kernel(const QmvArgs p) {
                 v[m][0] = v[m][1] = 0.0f;
 #pragma clang loop unroll_count(4)
                 for (uint32_t k = 0; k < wk; k++) {
-                    const float *r = &red[(((group * wk + k) * PI + sl * RR + m) * NT * 2 + el) * 64 + ln];
+                    const float *r = &red[(((group * wk + k) * pass_items + sl * RR + m) * pp + pair) * 32 + rn];
                     v[m][0] += r[0];
-                    v[m][1] += r[64];
+                    v[m][1] += r[16];
                 }
             }
             if constexpr (MODE == 2) {
@@ -827,10 +857,15 @@ qmv_kernel(const QmvArgs p) {
                     for (uint32_t k = 0; k < wk; k++) q += red_ss[k * 16 + tk + j];
                     const float sc = p.normalize ? 1.0f / __builtin_sqrtf(q / (float)p.columns + p.epsilon) : 1.0f;
                     const float gate = v[0][j] * sc, u = v[1][j] * sc;
-                    // silu(gate) * up, stable sigmoid (src/qwen35/cpu.rs:982-993)
-                    const float ex = expf(-fabsf(gate));
-                    const float sig = (gate >= 0.0f ? 1.0f : ex) / (1.0f + ex);
-                    v[0][j] = gate * sig * u;
+                    if constexpr (GROUPED) {
+                        // routed-expert activation (src/glm52/expert.rs:260-267)
+                        v[0][j] = (gate / (1.0f + expf(-gate))) * u;
+                    } else {
+                        // silu(gate) * up, stable sigmoid (src/qwen35/cpu.rs:982-993)
+                        const float ex = expf(-fabsf(gate));
+                        const float sig = (gate >= 0.0f ? 1.0f : ex) / (1.0f + ex);
+                        v[0][j] = gate * sig * u;
+                    }
                 }
             } else {
                 bool mine = true;
@@ -851,14 +886,114 @@ qmv_kernel(const QmvArgs p) {
                 if (!mine) continue;
             }
             if (row < p.rows) {
-                p.y[(size_t)tk * p.rows + row] = v[0][0];
-                if (tk + 1 < p.batch) p.y[(size_t)(tk + 1) * p.rows + row] = v[0][1];
+                p.y[(size_t)(GROUPED ? y_row[tk] : tk) * p.rows + row] = v[0][0];
+                if (tk + 1 < p.batch) p.y[(size_t)(GROUPED ? y_row[tk + 1] : tk + 1) * p.rows + row] = v[0][1];
             }
         }
         lds_barrier();  // red is written again in the next pass
     }
     // the ring's last loads have landed before the workgroup's LDS is freed
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <uint32_t TYPE, int NT, int MODE, int KB, uint32_t W, bool PHASED>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W / 4, W / 4)))
+qmv_kernel(const QmvArgs p) {
+    qmv_body<TYPE, NT, MODE, KB, W, PHASED, false>(p, blockIdx.x % p.k_parts, blockIdx.x / p.k_parts, p.batch, nullptr,
+                                                   nullptr);
+}
+
+// The routed experts of up to kGroupPairs pairs in one launch (MODE 2 with
+// the GLM activation, then MODE 0): each expert's matrix is streamed once
+// for all its tokens, up to 8 at a time.  Every workgroup finds from the ids
+// which experts are selected and takes its share of one of them: with n
+// (expert, 8 tokens) entries, gridDim.x / n workgroups each.  The grid is two
+// 8-wave workgroups per CU, so one's prologue runs beside the other's
+// stream.
+template <uint32_t TYPE, int MODE, int KB, uint32_t W>
+__global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(KB > 2 ? 2 : 4, KB > 2 ? 2 : 4)))
+qmv_experts_kernel(const QmvArgs args, const QmvExperts ex) {
+    __shared__ uint32_t s_count[kGroupExperts], s_pair[8], s_x[8], s_entry[4];
+    const uint32_t tid = threadIdx.x;
+    // The first wave reads every word it needs at once.
+    uint32_t id0 = 0, id1 = 0, go = 1;
+    if (tid < 64) {
+        if (tid < ex.pairs) id0 = ex.ids[tid];
+        if (tid + 64 < ex.pairs) id1 = ex.ids[tid + 64];
+        if (tid < ex.go_count) go = ex.go[tid];
+    }
+    for (uint32_t e = tid; e < kGroupExperts; e += blockDim.x) s_count[e] = 0;
+    if (tid < 8) s_pair[tid] = s_x[tid] = 0;
+    if (tid == 0) s_entry[0] = 0;
+    lds_barrier();
+    if (tid < 64 && __builtin_amdgcn_ballot_w64(go == 0) == 0) {
+        if (tid < ex.pairs) atomicAdd(&s_count[id0], 1u);
+        if (tid + 64 < ex.pairs) atomicAdd(&s_count[id1], 1u);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // entries of experts 4 tid .. + 3, their running sum over the lanes
+        uint32_t n[4], sum = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            n[j] = (s_count[4 * tid + j] + 7) / 8;
+            sum += n[j];
+        }
+        uint32_t upto = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const uint32_t v = __shfl_up(upto, d, 64);
+            if ((int)tid >= d) upto += v;
+        }
+        const uint32_t total = __shfl(upto, 63, 64);
+        const uint32_t share = gridDim.x / total ? gridDim.x / total : 1u;
+        const uint32_t entry = blockIdx.x / share;
+        if (entry < total) {
+            uint32_t base = upto - sum, mine = ~0u, from = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (entry >= base && entry < base + n[j]) {
+                    mine = 4 * tid + j;
+                    from = 8 * (entry - base);
+                }
+                base += n[j];
+            }
+            const int owner = __builtin_ctzll(__builtin_amdgcn_ballot_w64(mine != ~0u));
+            const uint32_t expert = __shfl(mine, owner, 64), first = __shfl(from, owner, 64);
+            // the entry's pairs, in order
+            const bool h0 = tid < ex.pairs && id0 == expert, h1 = tid + 64 < ex.pairs && id1 == expert;
+            const uint64_t b0 = __builtin_amdgcn_ballot_w64(h0), b1 = __builtin_amdgcn_ballot_w64(h1);
+            const uint64_t below = (1ull << tid) - 1;
+            const uint32_t r0 = __builtin_popcountll(b0 & below);
+            const uint32_t r1 = __builtin_popcountll(b0) + __builtin_popcountll(b1 & below);
+            if (h0 && r0 >= first && r0 < first + 8) {
+                s_pair[r0 - first] = tid;
+                s_x[r0 - first] = ex.k ? tid / ex.k : tid;
+            }
+            if (h1 && r1 >= first && r1 < first + 8) {
+                s_pair[r1 - first] = tid + 64;
+                s_x[r1 - first] = ex.k ? (tid + 64) / ex.k : tid + 64;
+            }
+            if (tid == 0) {
+                const uint32_t left = __builtin_popcountll(b0) + __builtin_popcountll(b1) - first;
+                s_entry[0] = left < 8 ? left : 8;
+                s_entry[1] = expert;
+                s_entry[2] = share;
+            }
+        }
+    }
+    lds_barrier();
+    const uint32_t count = __builtin_amdgcn_readfirstlane(s_entry[0]);
+    if (count == 0) return;
+    const uint32_t expert = __builtin_amdgcn_readfirstlane(s_entry[1]);
+    const uint32_t share = __builtin_amdgcn_readfirstlane(s_entry[2]);
+    QmvArgs p = args;
+    const uint64_t at = ex.w_of[expert];  // the same for every lane: kept in scalar registers
+    const uint32_t at_lo = __builtin_amdgcn_readfirstlane((uint32_t)at);
+    const uint32_t at_hi = __builtin_amdgcn_readfirstlane((uint32_t)(at >> 32));
+    p.w = (const uint8_t *)((uint64_t)at_hi << 32 | at_lo);
+    p.w2 = p.w + ex.w2_offset;
+    p.batch = count;
+    p.row_groups = share;
+    qmv_body<TYPE, 1, MODE, KB, W, false, true>(p, 0, blockIdx.x % share, ex.x_rows, s_x, s_pair);
 }
 
 // ---------------------------------------------------------------------------
@@ -968,6 +1103,57 @@ hipError_t dispatch(dmhip_ctx *ctx, uint32_t rows, uint32_t columns, const void 
 }
 
 }  // namespace
+
+// Experts' rows: fragments of up to 3 blocks per wave, 8 waves.
+constexpr uint32_t kGroupBlocks = 24;
+
+bool qmv_experts_supported(uint32_t type, size_t rows, size_t columns, size_t experts, size_t pairs, size_t x_rows) {
+    if ((type != kQ4_K && type != kQ6_K) || columns % 256 || columns == 0 || rows == 0) return false;
+    if (columns / 256 > kGroupBlocks || experts > kGroupExperts || pairs > kGroupPairs) return false;
+    const uint64_t row_bytes = (uint64_t)(columns / 256) * (type == kQ4_K ? 144 : 210);
+    return row_bytes * (rows + 2) + 1024 < 0xffffffffull && (uint64_t)x_rows * columns * 4 < 0xffff0000ull;
+}
+
+namespace {
+
+template <uint32_t TYPE, int MODE, int KB, uint32_t W>
+hipError_t run_experts(dmhip_ctx *ctx, const QmvArgs &a, const QmvExperts &ex, uint32_t waves, uint32_t grid) {
+    const uint32_t lds = waves * ring_depth<TYPE, 1, MODE, W, false, true>() * StageQ<TYPE>::items * 16;
+    auto kernel = qmv_experts_kernel<TYPE, MODE, KB, W>;
+    static LdsLimit limit;
+    hipError_t e = limit.ensure((const void *)kernel, lds);
+    if (e != hipSuccess) return e;
+    return launch_kernel(ctx, kernel, dim3(grid), dim3(64 * waves), lds, a, ex);
+}
+
+template <uint32_t TYPE, int MODE>
+hipError_t dispatch_experts(dmhip_ctx *ctx, uint32_t rows, uint32_t columns, const float *x, float *y,
+                            const QmvExperts &ex) {
+    const uint32_t blocks = columns / 256, kb = (blocks + 7) / 8, wave_k = (blocks + kb - 1) / kb;
+    const uint32_t waves = 8 / wave_k * wave_k;
+    const uint32_t cus = ctx->compute_units > 0 ? (uint32_t)ctx->compute_units : 256u;
+    const QmvArgs a{nullptr, nullptr, x, y, nullptr, rows, columns, blocks * StageQ<TYPE>::bytes, 0, wave_k, 1, 1, 1, 0, 0.0f};
+    // (rows of 3 or 6 blocks keep 6 waves busy, whose ring has room for
+    // another slot each)
+    if (waves == 6 && kb == 1) return run_experts<TYPE, MODE, 1, 6>(ctx, a, ex, waves, 2 * cus);
+    if (kb == 1) return run_experts<TYPE, MODE, 1, 8>(ctx, a, ex, waves, 2 * cus);
+    if (kb == 2) return run_experts<TYPE, MODE, 2, 8>(ctx, a, ex, waves, 2 * cus);
+    return run_experts<TYPE, MODE, 3, 8>(ctx, a, ex, waves, 2 * cus);
+}
+
+}  // namespace
+
+hipError_t launch_qmv_experts(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uint32_t columns, bool gate_up,
+                              uint64_t up_offset, const uint64_t *w_of, const uint32_t *ids, const uint32_t *go,
+                              uint32_t tokens, uint32_t k, const float *x, float *y) {
+    const uint32_t pairs = tokens * k;
+    const QmvExperts ex{w_of, up_offset, ids, go, tokens, pairs, gate_up ? k : 0, gate_up ? tokens : pairs};
+    if (gate_up)
+        return type == kQ4_K ? dispatch_experts<kQ4_K, 2>(ctx, rows, columns, x, y, ex)
+                             : dispatch_experts<kQ6_K, 2>(ctx, rows, columns, x, y, ex);
+    return type == kQ4_K ? dispatch_experts<kQ4_K, 0>(ctx, rows, columns, x, y, ex)
+                         : dispatch_experts<kQ6_K, 0>(ctx, rows, columns, x, y, ex);
+}
 
 // What an allocation-free call sets aside for a matrix (the activation
 // fragments of the documented limit; the K-split partials use it).

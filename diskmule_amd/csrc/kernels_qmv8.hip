@@ -953,9 +953,12 @@ __global__ void __launch_bounds__(64 * (S > 8 ? S : 8))
     // Jobs whose matrices a kernel earlier on the stream looked up: their
     // addresses come from dev_w, and the launch does nothing unless each of
     // the go_count tokens' go words is 1.
-    if (go)
-        for (uint32_t t = 0; t < go_count; t++)
-            if (go[t] == 0) return;
+    // (One load for all words: tested one after another they cost a memory
+    // round trip each.)
+    if (go) {
+        const uint32_t t = threadIdx.x & 63u;
+        if (__builtin_amdgcn_ballot_w64(t < go_count && go[t] == 0)) return;
+    }
     const Job8 j = jobs.job[blockIdx.y];
     const uint8_t *w = (const uint8_t *)(dev_w ? dev_w[blockIdx.y] : j.w);
     constexpr uint32_t WAVES = S > 8 ? S : 8;

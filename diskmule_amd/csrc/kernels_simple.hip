@@ -1342,7 +1342,7 @@ hipError_t launch_router_top_k(hipStream_t s, const uint16_t *router, uint32_t h
             return hipGetLastError();
         };
         static LdsLimit limit4, limit8;
-        return batch <= kMaxLookupTokens ? launch(router_cert_kernel<4>, 4, limit4)
+        return batch <= 8 ? launch(router_cert_kernel<4>, 4, limit4)
                                          : launch(router_cert_kernel<8>, 8, limit8);
     }
     if (staged && experts >= 2 * RF_EXPERTS) {

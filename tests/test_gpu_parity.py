@@ -1293,6 +1293,46 @@ def test_moe_layer_resident_lookup_batches(ctx, batch, slots):
     src.free()
 
 
+@pytest.mark.parametrize("hidden,width,experts,k,batch,equal", [
+    (2048, 768, 64, 8, 16, False),  # every pair count, experts of 1 to 16 tokens
+    (2304, 256, 32, 4, 16, True),   # every token on the same experts: two entries of 8 tokens each
+    (5120, 1536, 16, 2, 9, False),  # three blocks per wave, six waves
+    (1024, 1280, 40, 3, 11, False), (4096, 512, 16, 8, 8, True),
+])
+def test_moe_layer_groups_tokens_by_expert(ctx, hidden, width, experts, k, batch, equal):
+    """Calls whose tokens are grouped by expert on the device (all experts
+    resident): output within the GEMV tolerance of the oracle, ids exact, and
+    repeated calls bit-identical."""
+    router = synth.to_bf16_bits(synth.normal(synth.weight_seed(52, 0), experts * hidden) * np.float32(0.02))
+    if equal:
+        router = np.tile(router[:hidden], experts)  # ties: the lowest k experts for every token
+    gu_bytes, dn_bytes = 2 * width * synth.row_bytes(Q4_K, hidden), hidden * synth.row_bytes(Q6_K, width)
+    gu = synth.quantized_matrix(Q4_K, experts * 2 * width, hidden, synth.weight_seed(52, 1))
+    dn = synth.quantized_matrix(Q6_K, experts * hidden, width, synth.weight_seed(52, 2))
+    src = PinnedHostBuffer(gu.size + dn.size)
+    src.array[:gu.size] = gu
+    src.array[gu.size:] = dn
+    cache = ExpertCache(ctx, src, [ExpertLayerLayout(experts, 0, gu_bytes, gu.size, dn_bytes)], experts)
+    for e in range(experts):
+        cache.release(0, cache.acquire(0, e)[0])
+    x = synth.normal(synth.activation_seed(52, batch), batch * hidden).reshape(batch, hidden)
+    sel, wts, out = capi.moe_layer(batch, hidden, width, experts, k, router, Q4_K, gu, Q6_K, dn, x)
+    rb, yb, xb = dev(ctx, router), dev_out(ctx, batch * hidden * 4), dev(ctx, x)
+    runs = []
+    for _ in range(4):
+        ids, probs = ctx.moe_layer(cache, 0, batch, hidden, width, experts, k, rb.device_ptr, Q4_K, Q6_K,
+                                   xb.device_ptr, yb.device_ptr)
+        assert np.array_equal(ids, sel)
+        assert np.allclose(probs, wts, rtol=1e-5, atol=1e-7)
+        runs.append(yb.read(0, batch * hidden * 4, np.float32).reshape(batch, hidden).copy())
+    for t in range(batch):
+        for r in runs:
+            assert_close(r[t], out[t], f"token {t}")
+    assert all(np.array_equal(bits(r), bits(runs[1])) for r in runs[2:])
+    cache.free()
+    src.free()
+
+
 def test_moe_layer_lookup_wide_router(ctx):
     """Two tokens over a router wider than 8192 columns (the exact fold's
     expert-parallel kernel, which writes the device-side lookup itself):
