@@ -7,14 +7,17 @@
 // reference's buffers).  Position p lives in slot p % capacity.
 //
 // Two kernels per call:
-//  * attn_chunk_kernel: workgroup (chunk, kv head, head group) scores the
-//    chunk's positions for the query heads that share the KV head, takes the
-//    chunk's softmax statistics and its unnormalised weighted value sum;
+//  * attn_stream_kernel (head dimensions 128, 256 and 512, up to 8 query heads
+//    per KV head) or attn_chunk_kernel (every other shape): workgroup (chunk,
+//    kv head, head group) scores the chunk's positions for the query heads
+//    that share the KV head, takes the chunk's softmax statistics and its
+//    unnormalised weighted value sum;
 //  * attn_combine_kernel: workgroup (query head, 64 dims) merges the chunks.
-// Each score is the reference's sequential fma over the head dimension
-// (d ascending, one lane per position), so scores are bit-identical to the
-// CPU fold; the keys reach the lanes through LDS so that every HBM read is a
-// coalesced row segment.
+// Scores are fp32 fma sums over the head dimension.  attn_chunk_kernel takes
+// them in the reference's order (d ascending, one lane per position; the keys
+// reach the lanes through LDS so that every HBM read is a coalesced row
+// segment), attn_stream_kernel as 8-term chains added in a tree, whose error
+// is smaller.
 #include "dm_device.h"
 #include "runtime.h"
 
@@ -325,6 +328,317 @@ attn_chunk_kernel(const float *__restrict__ query, const float *__restrict__ key
     if (t < gz) part_ml[prow + t] = make_float2(s_m[t], s_l[t]);
 }
 
+// ---------------------------------------------------------------------------
+// Streaming form for head dimensions of 128, 256 and 512 and groups of up to 8
+// query heads.  A row is held by HD / 8 lanes, 8 dims each (two 16-byte loads
+// of contiguous lanes), so a wave takes R rows of each of its 512 / HD lane
+// groups at a time straight into registers (R = 8 up to 2 heads; 4 above,
+// where 8 rows and the heads' sums do not fit 256 registers): no staging and
+// no barrier until the end, 16 or 32 KiB of keys and values in flight per
+// wave.  Scores are 8-term fma chains per lane added in a fixed tree over the
+// lanes; the sums of R rows and of the heads are reduced together (each
+// exchange halves the values a lane keeps), which leaves one row and head with
+// each lane, so the softmax costs two exponentials per block of rows, not two
+// per head.  It is the online one (earlier sums rescaled when a larger maximum
+// arrives); the waves meet in LDS at the chunk's end.
+//
+// Large windows are bound by the reads of the keys and values: 16 query on 2
+// KV heads of 512 dims at 32768 positions, 52.8 us for 268 MB (5.1 TB/s); the
+// chunk kernel took 61.6.  Small ones by their chain of latencies.  Whole
+// calls, chunk kernel against this one, in us at 64 / 1024 / 4096 / 32768
+// positions: 16 on 2 x 512: 24.4 / 25.4 / 29.5 / 68.5 against 12.2 / 15.8 /
+// 19.7 / 58.3; 16 on 8 x 256: 13.9 / 15.2 / 22.2 / 105.9 against 9.4 / 11.1 /
+// 18.7 / 92.6; 32 on 8 x 128: 14.7 / 15.5 / 22.4 / 85.3 against 9.8 / 11.1 /
+// 16.7 / 56.9; 8 on 8 x 128: 13.5 / 14.5 / 20.1 / 76.5 against 9.3 / 10.1 /
+// 14.2 / 55.0.  With the scores reduced over the lanes head by head and an
+// exponential per head in every lane: 60.3 and 54.5 in the kernel at 2 x 512.
+// ---------------------------------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ float attn_dpp(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+// DPP controls: lane ^ 1, ^ 2, ^ 3 (quads), ^ 7 (half rows), ^ 8 (rotation by 8 of 16).
+constexpr int kAXor1 = 0xb1, kAXor2 = 0x4e, kAXor3 = 0x1b, kAXor7 = 0x141, kAXor8 = 0x128;
+
+// (a, b) -> per lane the sum over the lanes differing in lane bit BIT of a
+// (bit clear) or of b (bit set).  For bit 2 the partner is lane ^ 7: the
+// reductions over bits 1 and 0 that follow make that the same sum.
+template <int BIT>
+__device__ __forceinline__ float attn_fold(float a, float b, uint32_t lane) {
+    const uint32_t ua = __float_as_uint(a), ub = __float_as_uint(b);
+    if constexpr (BIT == 5) {
+        const auto r = __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else if constexpr (BIT == 4) {
+        const auto r = __builtin_amdgcn_permlane16_swap(ua, ub, false, false);
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    } else {
+        const bool set = (lane >> BIT) & 1u;
+        const float keep = set ? b : a, give = set ? a : b;
+        return keep + attn_dpp<BIT == 3 ? kAXor8 : BIT == 2 ? kAXor7 : BIT == 1 ? kAXor2 : kAXor1>(give);
+    }
+}
+
+// v combined with the partner's across lane bit BIT, in every lane.
+template <int BIT, class F>
+__device__ __forceinline__ float attn_across(float v, F f) {
+    const uint32_t u = __float_as_uint(v);
+    if constexpr (BIT == 5) {
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else if constexpr (BIT == 4) {
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    } else {
+        const float w = BIT == 2 ? attn_dpp<kAXor3>(v) : v;  // ^ 7 after ^ 3 is ^ 4
+        return f(v, attn_dpp<BIT == 3 ? kAXor8 : BIT == 2 ? kAXor7 : BIT == 1 ? kAXor2 : kAXor1>(w));
+    }
+}
+
+constexpr uint32_t kStreamWaves = 8;
+constexpr uint32_t stream_r(uint32_t gt) { return gt <= 2 ? 8 : 4; }  // rows of a lane group at a time
+// LDS of a workgroup: the query rows, each lane group's weights and rescaling
+// factors, the merge's maxima and sums, and (in the place of the first two)
+// the lane groups' sums.
+template <int HD, int GT>
+constexpr uint32_t stream_lds(uint32_t waves) {
+    const uint32_t lanes_groups = waves * 512 / HD;
+    const uint32_t run = GT * HD + lanes_groups * GT * (stream_r(GT) + 1), merge = lanes_groups * GT * HD;
+    return 4 * ((run > merge ? run : merge) + 2 * lanes_groups * GT);
+}
+
+template <int HD, int GT>
+__global__ void __launch_bounds__(64 * kStreamWaves)
+attn_stream_kernel(const float *__restrict__ query, const float *__restrict__ keys,
+                   const float *__restrict__ values, uint64_t capacity, uint64_t width, uint32_t group,
+                   uint64_t start, uint32_t visible, uint32_t chunk, uint32_t chunks, float *__restrict__ part_o,
+                   float2 *__restrict__ part_ml, BadFlag bad) {
+    constexpr uint32_t LPR = HD / 8, G = 64 / LPR, RPI = stream_r(GT) * G;
+    constexpr int R = (int)stream_r(GT);
+    constexpr int TOP = LPR == 64 ? 5 : LPR == 32 ? 4 : 3;  // highest lane bit inside a group
+    // Lane bits of a group from the top: the row whose scores the lane ends
+    // with, the head, and bits over which lanes hold the same; NV heads a lane.
+    constexpr int RB = R == 8 ? 3 : 2, HB0 = GT == 8 ? 3 : GT == 4 ? 2 : GT == 2 ? 1 : 0;
+    constexpr int HB = HB0 < TOP + 1 - RB ? HB0 : TOP + 1 - RB, NV = GT >> HB, LOW = TOP + 1 - RB - HB;
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const uint32_t t = threadIdx.x, lane = t & 63u, waves = blockDim.x >> 6;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t l = lane % LPR, lg = lane / LPR;              // lane in its group, group
+    const uint32_t my_row = (l >> (TOP + 1 - RB)) & (R - 1u), my_head = NV * ((l >> LOW) & ((1u << HB) - 1u));
+    const uint32_t sets = waves * G, set = wave * G + lg;        // lane groups of the workgroup
+    float *qs = lds, *ps = lds + GT * HD + set * GT * R, *sc = lds + GT * HD + sets * GT * R + set * GT;
+    const uint32_t run = GT * HD + sets * GT * (R + 1), merge = sets * GT * HD;
+    float *s_m = lds + (run > merge ? run : merge), *s_l = s_m + sets * GT;
+
+    const uint32_t c = blockIdx.x, kh = blockIdx.y, g_base = blockIdx.z * GT;
+    const uint32_t gz = min((uint32_t)GT, group - g_base);  // heads of this workgroup
+    const uint32_t p0 = c * chunk, n = min(chunk, visible - p0);
+    const uint64_t slot0 = (start + p0) % capacity;
+    const uint64_t qbase = (uint64_t)kh * group + g_base;
+    const float *kb = keys + (uint64_t)kh * HD + 4 * l, *vb = values + (uint64_t)kh * HD + 4 * l;
+
+    // Row i of the wave's block at position j0 (clamped into the chunk: the
+    // loads stay unconditional; what a row past the end gives is dropped).
+    floatx4 kr[R][2], vr[R][2];
+    auto load = [&](const float *base, floatx4 (&r)[R][2], uint32_t j0) {
+#pragma unroll
+        for (uint32_t i = 0; i < R; i++) {
+            uint64_t slot = slot0 + min(j0 + R * lg + i, n - 1);
+            if (slot >= capacity) slot -= capacity;
+            const float *src = base + slot * width;
+            r[i][0] = *(const floatx4 *)src;
+            r[i][1] = *(const floatx4 *)(src + HD / 2);
+        }
+    };
+    // Wave w takes the blocks w, w + waves, ... of the chunk.
+    const uint32_t step = waves * RPI;
+    uint32_t j0 = wave * RPI;
+    // The query rows go to LDS 16 bytes a lane, four loads at a time; the first
+    // four are asked for before the keys and values, so that the wait for them
+    // leaves those in flight.
+    const uint32_t units = gz * (HD / 4);
+    const floatx4 *q4 = (const floatx4 *)(query + qbase * HD);
+    floatx4 qv[4];
+    auto ask = [&](uint32_t i0) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) qv[k] = q4[min(i0 + k * blockDim.x, units - 1)];
+    };
+    auto put = [&](uint32_t i0) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            const uint32_t i = i0 + k * blockDim.x;
+            if (i < GT * HD / 4) ((floatx4 *)qs)[i] = qv[k];  // (heads past the last: scored, then dropped)
+        }
+    };
+    ask(t);
+    __builtin_amdgcn_sched_barrier(0);
+    load(kb, kr, j0);
+    load(vb, vr, j0);
+    __builtin_amdgcn_sched_barrier(0);
+    put(t);
+    for (uint32_t i = t + 4 * blockDim.x; i < GT * HD / 4; i += 4 * blockDim.x) {
+        ask(i);
+        put(i);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+
+    float o[GT][8], m[NV], ls[NV];
+#pragma unroll
+    for (int h = 0; h < GT; h++)
+#pragma unroll
+        for (int d = 0; d < 8; d++) o[h][d] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) m[i] = -INFINITY, ls[i] = 0.0f;
+    bool flag = false;
+    const auto add = [](float a, float b) { return a + b; };
+    const auto big = [](float a, float b) { return fmaxf(a, b); };
+    for (; j0 < n; j0 += step) {
+        const bool mine = j0 + R * lg + my_row < n;
+        float s[GT];
+#pragma unroll
+        for (int h = 0; h < GT; h++) {
+            const floatx4 q0 = *(const floatx4 *)&qs[h * HD + 4 * l], q1 = *(const floatx4 *)&qs[h * HD + HD / 2 + 4 * l];
+            float d[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                float v = q0[0] * kr[r][0][0];
+#pragma unroll
+                for (int e = 1; e < 4; e++) v = __builtin_fmaf(q0[e], kr[r][0][e], v);
+#pragma unroll
+                for (int e = 0; e < 4; e++) v = __builtin_fmaf(q1[e], kr[r][1][e], v);
+                d[r] = v;
+            }
+            float v;
+            if constexpr (R == 8) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) d[r] = attn_fold<TOP>(d[r], d[r + 4], lane);
+#pragma unroll
+                for (int r = 0; r < 2; r++) d[r] = attn_fold<TOP - 1>(d[r], d[r + 2], lane);
+                v = attn_fold<TOP - 2>(d[0], d[1], lane);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 2; r++) d[r] = attn_fold<TOP>(d[r], d[r + 2], lane);
+                v = attn_fold<TOP - 1>(d[0], d[1], lane);
+            }
+            s[h] = v;
+        }
+        // ... then the heads' sums together, over the next bits
+        constexpr int B = TOP - RB;  // the highest of them
+        if constexpr (HB >= 1) {
+#pragma unroll
+            for (int i = 0; i < GT / 2; i++) s[i] = attn_fold<(HB >= 1 ? B : 0)>(s[i], s[i + GT / 2], lane);
+        }
+        if constexpr (HB >= 2) {
+#pragma unroll
+            for (int i = 0; i < GT / 4; i++) s[i] = attn_fold<(HB >= 2 ? B - 1 : 0)>(s[i], s[i + GT / 4], lane);
+        }
+        if constexpr (HB >= 3) s[0] = attn_fold<(HB >= 3 ? B - 2 : 0)>(s[0], s[1], lane);
+        static_assert(LOW <= 3, "bits left over");
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            float v = s[i];
+            if constexpr (LOW >= 3) v = attn_across<2>(v, add);
+            if constexpr (LOW >= 2) v = attn_across<1>(v, add);
+            if constexpr (LOW >= 1) v = attn_across<0>(v, add);
+            if (mine && my_head + i < gz) flag |= __builtin_isnan(v) || v == INFINITY;
+            s[i] = mine ? v : -INFINITY;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (j0 + step < n) load(kb, kr, j0 + step);
+        __builtin_amdgcn_sched_barrier(0);
+        bool moved = false;
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            float mx = attn_across<TOP>(s[i], big);
+            mx = attn_across<TOP - 1>(mx, big);
+            if constexpr (R == 8) mx = attn_across<TOP - 2>(mx, big);
+            mx = fmaxf(mx, m[i]);
+            // nothing finite yet: every weight is 0
+            const float e = mx == -INFINITY ? 0.0f : expf(s[i] - mx);
+            const float scale = mx == -INFINITY ? 1.0f : expf(m[i] - mx);
+            moved |= mx != m[i];
+            m[i] = mx;
+            ls[i] = __builtin_fmaf(ls[i], scale, e);
+            // (lanes of one row and head hold the same)
+            ps[(my_head + i) * R + my_row] = e;
+            sc[my_head + i] = scale;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (__builtin_amdgcn_ballot_w64(moved)) {
+#pragma unroll
+            for (int h = 0; h < GT; h++) {
+                const float scale = sc[h];
+#pragma unroll
+                for (int d = 0; d < 8; d++) o[h][d] *= scale;
+            }
+        }
+        if (j0 + RPI > n) {
+            // rows past the end: their weight is 0, their values must not count
+#pragma unroll
+            for (uint32_t r = 0; r < R; r++)
+                if (j0 + R * lg + r >= n) vr[r][0] = vr[r][1] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int h = 0; h < GT; h++) {
+            floatx4 pw[R / 4];
+#pragma unroll
+            for (int r = 0; r < R / 4; r++) pw[r] = *(const floatx4 *)&ps[h * R + 4 * r];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float w = pw[r / 4][r % 4];
+#pragma unroll
+                for (int d = 0; d < 8; d++) o[h][d] = __builtin_fmaf(w, vr[r][d / 4][d % 4], o[h][d]);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_sched_barrier(0);
+        if (j0 + step < n) load(vb, vr, j0 + step);
+    }
+    if (flag) *bad.word = bad.mark;
+
+    // ---- the lane groups' sums meet in LDS ----
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        float v = attn_across<TOP>(ls[i], add);
+        v = attn_across<TOP - 1>(v, add);
+        if constexpr (R == 8) v = attn_across<TOP - 2>(v, add);
+        if (my_row == 0) {
+            s_m[set * GT + my_head + i] = m[i];
+            s_l[set * GT + my_head + i] = v;
+        }
+    }
+    __syncthreads();  // and every wave is done with qs and ps
+#pragma unroll
+    for (int h = 0; h < GT; h++) {
+        float mx = -INFINITY;
+        for (uint32_t k = 0; k < sets; k++) mx = fmaxf(mx, s_m[k * GT + h]);
+        const float mine = s_m[set * GT + h], w = mine == -INFINITY ? 0.0f : expf(mine - mx);
+        float *dst = &lds[(set * GT + h) * HD + 4 * l];
+        *(floatx4 *)dst = floatx4{o[h][0] * w, o[h][1] * w, o[h][2] * w, o[h][3] * w};
+        *(floatx4 *)(dst + HD / 2) = floatx4{o[h][4] * w, o[h][5] * w, o[h][6] * w, o[h][7] * w};
+    }
+    __syncthreads();
+    const uint64_t prow = ((uint64_t)kh * chunks + c) * group + g_base;
+    for (uint32_t i = t; i < units; i += blockDim.x) {
+        floatx4 v = *(const floatx4 *)&lds[4 * i];
+        for (uint32_t k = 1; k < sets; k++) {
+            const floatx4 u = *(const floatx4 *)&lds[k * GT * HD + 4 * i];
+#pragma unroll
+            for (int d = 0; d < 4; d++) v[d] += u[d];
+        }
+        *(floatx4 *)(part_o + prow * HD + 4 * i) = v;
+    }
+    if (t < gz) {
+        float mx = -INFINITY, sum = 0.0f;
+        for (uint32_t k = 0; k < sets; k++) mx = fmaxf(mx, s_m[k * GT + t]);
+        for (uint32_t k = 0; k < sets; k++)
+            if (s_m[k * GT + t] != -INFINITY) sum = __builtin_fmaf(s_l[k * GT + t], expf(s_m[k * GT + t] - mx), sum);
+        part_ml[prow + t] = make_float2(mx, sum);
+    }
+}
+
 // out[h][d] = sum_c w_c o_c[d] / sum_c w_c l_c, w_c = exp(m_c - max_c m_c).
 // Workgroup (query head, 64 dims, split s) sums the chunks of split s, in
 // chunk order per wave and a fixed tree across the four waves.  With more
@@ -470,8 +784,33 @@ static hipError_t launch_chunk_gt(dmhip_ctx *ctx, bool kv4, int vv, dim3 grid, c
     return launch_chunk<GT, true, 1>(ctx, grid, q, k, v, capacity, width, group, hd, start, visible, chunk, chunks, po, pml, bad);
 }
 
+template <int HD, int GT>
+static hipError_t launch_stream(dmhip_ctx *ctx, dim3 grid, uint32_t waves, const float *q, const float *k,
+                                const float *v, uint64_t capacity, uint64_t width, uint32_t group, uint64_t start,
+                                uint32_t visible, uint32_t chunk, uint32_t chunks, float *po, float2 *pml,
+                                BadFlag bad) {
+    const uint32_t bytes = stream_lds<HD, GT>(waves);
+    static LdsLimit limit;
+    const hipError_t e = limit.ensure((const void *)attn_stream_kernel<HD, GT>, bytes);
+    if (e != hipSuccess) return e;
+    return launch_kernel(ctx, attn_stream_kernel<HD, GT>, grid, dim3(64 * waves), bytes, q, k, v, capacity, width, group,
+                         start, visible, chunk, chunks, po, pml, bad);
+}
+
+template <int HD>
+static hipError_t launch_stream_gt(dmhip_ctx *ctx, uint32_t gt, dim3 grid, uint32_t waves, const float *q,
+                                   const float *k, const float *v, uint64_t capacity, uint64_t width, uint32_t group,
+                                   uint64_t start, uint32_t visible, uint32_t chunk, uint32_t chunks, float *po,
+                                   float2 *pml, BadFlag bad) {
+    if (gt == 1) return launch_stream<HD, 1>(ctx, grid, waves, q, k, v, capacity, width, group, start, visible, chunk, chunks, po, pml, bad);
+    if (gt == 2) return launch_stream<HD, 2>(ctx, grid, waves, q, k, v, capacity, width, group, start, visible, chunk, chunks, po, pml, bad);
+    if (gt == 4) return launch_stream<HD, 4>(ctx, grid, waves, q, k, v, capacity, width, group, start, visible, chunk, chunks, po, pml, bad);
+    return launch_stream<HD, 8>(ctx, grid, waves, q, k, v, capacity, width, group, start, visible, chunk, chunks, po, pml, bad);
+}
+
 // The launch plan of one attention call.
 struct AttnPlan {
+    uint32_t stream_waves;  // waves of the streaming form's workgroups, 0: the chunk kernel
     uint32_t gt, chunk, chunks, zgroups;
     bool kv4;
     int vv;
@@ -479,7 +818,7 @@ struct AttnPlan {
     size_t part_o_floats, part_ml_pairs;
 };
 
-static AttnPlan attn_plan(size_t kv_heads, size_t group, size_t hd, size_t visible, bool aligned16) {
+static AttnPlan attn_plan(size_t kv_heads, size_t group, size_t hd, size_t visible, bool aligned16, uint32_t cus) {
     AttnPlan p{};
     p.gt = group > 8 ? 16 : group > 4 ? 8 : group > 2 ? 4 : (uint32_t)group;
     p.zgroups = (uint32_t)((group + p.gt - 1) / p.gt);
@@ -490,6 +829,19 @@ static AttnPlan attn_plan(size_t kv_heads, size_t group, size_t hd, size_t visib
     p.chunk = (uint32_t)(k * kAttnRows);
     p.chunks = (uint32_t)((visible + p.chunk - 1) / p.chunk);
     p.kv4 = hd % 4 == 0 && aligned16;
+    if (p.kv4 && (hd == 128 || hd == 256 || hd == 512) && group <= 8) {
+        // One workgroup per CU: as many waves as give each a block of rows,
+        // then as many blocks as make one round of workgroups.  Never one wave
+        // alone: at 300 positions of 16 on 2 x 512 one wave took 17.4 us, two
+        // 15.6 and four 14.4 (fewer chunks to combine), but four cost 1 us at
+        // the other shapes (32 on 8 x 128, 300 positions: 11.2 / 10.5 / 11.5).
+        const size_t rows = stream_r(p.gt) * 512 / hd, blocks = (visible + rows - 1) / rows;
+        const size_t per_cu = (blocks * kv_heads + cus - 1) / cus;
+        p.stream_waves = per_cu >= 8 ? 8 : per_cu >= 4 ? 4 : 2;
+        const size_t per = per_cu > 8 ? (per_cu + 7) / 8 : 1;
+        p.chunk = (uint32_t)(p.stream_waves * per * rows);
+        p.chunks = (uint32_t)((visible + p.chunk - 1) / p.chunk);
+    }
     // four value dims per thread only up to 8 heads (16 x 4 accumulators spill)
     p.vv = p.kv4 && hd >= 1024 && p.gt <= 8 ? 4 : (p.kv4 && hd >= 512 ? 2 : 1);
     // about 32 chunks per combine workgroup, at most kCombineBlock
@@ -509,7 +861,8 @@ static int enqueue_attention(dmhip_ctx *ctx, const float *query, const float *ke
                              size_t start, size_t visible, float *output, BadFlag bad) {
     const size_t group = query_heads / kv_heads;
     const bool aligned16 = (((uintptr_t)query | (uintptr_t)keys | (uintptr_t)values) & 15u) == 0;
-    const AttnPlan p = attn_plan(kv_heads, group, hd, visible, aligned16);
+    const AttnPlan p = attn_plan(kv_heads, group, hd, visible, aligned16,
+                                 ctx->compute_units > 0 ? (uint32_t)ctx->compute_units : 256u);
     const size_t blocks = (hd + 63) / 64;
     const size_t stage_o_floats = p.splits > 1 ? query_heads * blocks * p.splits * 64 : 0;
     const size_t stage_l_floats = p.splits > 1 ? query_heads * blocks * p.splits : 0;
@@ -535,12 +888,18 @@ static int enqueue_attention(dmhip_ctx *ctx, const float *query, const float *ke
     }
     const dim3 grid(p.chunks, (uint32_t)kv_heads, p.zgroups);
     hipError_t e;
-    switch (p.gt) {
-    case 1: e = launch_chunk_gt<1>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
-    case 2: e = launch_chunk_gt<2>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
-    case 4: e = launch_chunk_gt<4>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
-    case 8: e = launch_chunk_gt<8>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
-    default: e = launch_chunk_gt<16>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
+    if (p.stream_waves) {
+        auto launch = hd == 128 ? launch_stream_gt<128> : hd == 256 ? launch_stream_gt<256> : launch_stream_gt<512>;
+        e = launch(ctx, p.gt, grid, p.stream_waves, query, keys, values, capacity, width, (uint32_t)group, start,
+                   (uint32_t)visible, p.chunk, p.chunks, po, pml, bad);
+    } else {
+        switch (p.gt) {
+        case 1: e = launch_chunk_gt<1>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
+        case 2: e = launch_chunk_gt<2>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
+        case 4: e = launch_chunk_gt<4>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
+        case 8: e = launch_chunk_gt<8>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
+        default: e = launch_chunk_gt<16>(ctx, p.kv4, p.vv, grid, query, keys, values, capacity, width, (uint32_t)group, (uint32_t)hd, start, (uint32_t)visible, p.chunk, p.chunks, po, pml, bad); break;
+        }
     }
     if (e != hipSuccess) return hip_fail(e, "attention chunk kernel");
     e = launch_kernel(ctx, attn_combine_kernel, dim3((uint32_t)query_heads, (uint32_t)blocks, p.splits), dim3(256),

@@ -215,6 +215,63 @@ def test_many_chunks_combined_in_splits(ctx):
     assert np.array_equal(again.view(np.uint32), out.view(np.uint32))
 
 
+@pytest.mark.parametrize("hd", [128, 256, 512])
+@pytest.mark.parametrize("group", [1, 2, 3, 4, 7, 8])
+def test_streaming_form_edges(ctx, hd, group):
+    """Head dimensions 128, 256 and 512 with up to 8 heads per KV head: windows
+    of one row, one row on either side of a wave's block (512 / hd lane groups
+    of 8 or 4 rows), of two blocks and of several waves and chunks, ring
+    wrapped inside a block; then a row of -inf scores, whose weight is 0.
+    Scores are 8-term chains and at most 6 levels of sums, one exact fold in
+    float64 away by at most 14 u sum |q k| each: with the fold's own hd u, the
+    weights of the budget's exact result move by twice that."""
+    kvh = 3
+    width, qh = kvh * hd, 3 * group
+    block = (8 if group <= 2 else 4) * 512 // hd
+    rng = np.random.default_rng(hd * 10 + group)
+    for visible in (1, block - 1, block, block + 1, 2 * block + 3, 7 * block + 5, 400):
+        print(f"stream hd={hd} group={group} visible={visible}", flush=True)
+        positions = visible + 5
+        keys = rng.standard_normal((positions, width)).astype(np.float32)
+        values = rng.standard_normal((positions, width)).astype(np.float32)
+        q = (rng.standard_normal(qh * hd) / np.sqrt(hd)).astype(np.float32)
+        minus_inf = visible > 1
+        if minus_inf:  # the row in the middle: -inf for every head
+            q[::hd] = np.abs(q[::hd]) + np.float32(0.1)
+            keys[5 + visible // 2, ::hd] = -np.inf
+        layer = ctx.new_kv_layer(width, 4096, visible)
+        fill_layer(ctx, layer, keys, values)
+        out = np.zeros(qh * hd, dtype=np.float32)
+        ctx.attention_cached(q, layer, qh, kvh, hd, out)
+        again = np.zeros_like(out)
+        ctx.attention_cached(q, layer, qh, kvh, hd, again)
+        assert np.array_equal(again.view(np.uint32), out.view(np.uint32))
+        k, v = keys[5:], values[5:]
+        if minus_inf:
+            keep = np.arange(visible) != visible // 2
+            k, v = k[keep], v[keep]
+        n = k.shape[0]
+        exact, w, w2, _ = attention_exact(q, k, v, n, width, qh, kvh, hd, 0, n)
+        heads = np.repeat(np.arange(kvh), group)
+        qk = np.einsum("hd,nhd->hn", np.abs(q.reshape(qh, hd)).astype(np.float64),
+                       np.abs(k.reshape(n, kvh, hd)[:, heads]).astype(np.float64)).max(axis=1)
+        budget = attention_budget(w, w2, n) + 4.0 * (14 + hd) * 2.0 ** -24 * qk[:, None] * w
+        assert np.all(np.abs(out.reshape(qh, hd) - exact) <= budget)
+        layer.free()
+    # every score -inf, and one NaN, are refused as by the other form
+    layer = ctx.new_kv_layer(width, 16, None)
+    ctx.append_kv(layer, 0, np.full(width, -np.inf, np.float32), np.ones(width, np.float32))
+    expect_error("NonFinite", ctx.attention_cached, np.ones(qh * hd, np.float32), layer, qh, kvh, hd, out)
+    ctx.append_kv(layer, 1, np.ones(width, np.float32), np.ones(width, np.float32))
+    ctx.attention_cached(np.ones(qh * hd, np.float32), layer, qh, kvh, hd, out)
+    assert np.all(out == 1.0)
+    bad = np.ones(width, np.float32)
+    bad[-1] = np.nan
+    ctx.append_kv(layer, 2, bad, np.ones(width, np.float32))
+    expect_error("NonFinite", ctx.attention_cached, np.ones(qh * hd, np.float32), layer, qh, kvh, hd, out)
+    layer.free()
+
+
 # ---- non-finite scores ---------------------------------------------------------------
 
 def test_non_finite_scores_are_rejected(ctx):
