@@ -30,23 +30,34 @@
 // (per format below), chosen so that a lane's 8 weights come from one or two
 // aligned dwords of the block.  The A preparation stores A in that order.
 //
-// Tiling: a workgroup of 4 waves (one per SIMD) owns a 128 x 64 tile of C;
-// wave w sums over the w-th quarter of the K blocks (no operand is shared
-// between waves), with 4 x 2 MFMA tiles of 32 x 32 in AGPRs, so every
-// dequantized weight feeds four MFMAs.  A arrives from global memory already
-// in fragment order (one 1 KiB load per 32 rows and step, kADist steps ahead
-// of its use); W for the wave's 64 rows is staged one block at a time in the
-// wave's own LDS area, fetched into registers one block ahead and written to
-// LDS two thirds through the current block, so the next block's scales are
-// decoded while the current block's MFMAs run.  Workgroups are persistent
-// (one per CU): a wave walks its tiles' blocks as one sequence, so the next
-// tile's first loads are in flight during a tile's final sum.  The quarters'
-// partial tiles are added through LDS (two regions, column-major, 16-byte
-// accesses).  Tiles are ordered so that each XCD keeps half of A in its L2.
+// Tiling: a workgroup of 4 waves owns a 128 x 64 tile of C, and two workgroups
+// run on a CU, so that a SIMD has a second wave to issue from while the first
+// waits for its operands or its matrix instructions.  Wave w sums over the
+// w-th quarter of the K blocks (no operand is shared between waves), with
+// 4 x 2 MFMA tiles of 32 x 32, so every dequantized weight feeds four MFMAs.
+// A arrives from global memory already in fragment order (the four row tiles
+// of a step are 4 KiB in a row, one 1 KiB load each, kADist steps ahead of
+// their use); W for the wave's 64 rows goes one block at a time from global
+// memory straight to the wave's own LDS area, asked for when the block before
+// it has been read.  The quarters' partial tiles are added through LDS, in the
+// place of W (column-major, 16-byte accesses).  Tiles are ordered so that each
+// XCD keeps half of A in its L2.
+//
+// Against one persistent workgroup per CU with W a block ahead in registers
+// and A 4 steps ahead (one wave per SIMD, 512 registers), whole calls in us,
+// Q4_K / Q6_K / Q8_0: 2048 x 12288 x 4096 238.7 / 287.8 / 267.4 -> 222.3 /
+// 253.8 / 246.6; 512 x 12288 x 4096 62.3 / 74.0 / 70.0 -> 59.0 / 68.9 / 65.2;
+// 333 x 4096 x 12288 52.7 / 64.0 / 62.5 -> 52.6 / 61.1 / 60.6; 100 x 4096 x
+// 4096 20.7 / 25.1 / 23.4 -> 20.5 / 24.0 / 22.6.  What bounds it: at 2048
+// rows, with the A loads left out 177 us of 224, with the MFMAs left out 170,
+// with neither A loads nor dequantization 160: the matrix cores and the A
+// fragments through the vector memory path, which no wave shares.  Not the
+// latency of either operand: a ring of 4 A steps, W double-buffered in LDS, and
+// both, measured within 2% of this form; 8 waves with an eighth of K each,
+// 10-20% slower (a longer final sum with nothing beside it).
 #include "dm_device.h"
 #include "dm_qmv.h"
 #include "runtime.h"
-
 
 namespace dm {
 
@@ -54,35 +65,23 @@ namespace {
 
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));  // 16-byte aligned
 
-constexpr uint32_t kBN = 64, kWaves = 4;
-constexpr uint32_t kPadRows = 128;  // workspace rows are padded to every tile height
-// MFMA steps between the load of an A fragment and its use.  Loads complete
-// in order, so this is also the time every W load has to arrive.
-constexpr uint32_t kADist = 4;
+constexpr uint32_t kBM = 128, kBN = 64, kWaves = 4;
+constexpr uint32_t kPadRows = 128;  // workspace rows are padded to the tile height
+// MFMA steps between the load of an A fragment and its use.
+constexpr uint32_t kADist = 2;
 static_assert(16 % kADist == 0, "the A ring repeats every block");
 
-// Tile shape: RM = 4 MFMA row tiles per wave, a 128 x 64 tile per workgroup,
-// one persistent workgroup per CU (one wave per SIMD).  (64 x 64 tiles with
-// two workgroups per CU measured no faster: the loop's MFMA share is the
-// same, and each weight then feeds two MFMAs instead of four.)  W of a
-// tile's next block is staged during the current tile's last block, so the
-// partial tiles have LDS of their own: [W staging][2 partial tiles][row
-// scales].
-template <uint32_t RM>
-struct Tile {
-    static constexpr uint32_t kRM = RM, kBM = 32 * RM;
-    static constexpr uint32_t kRedLd = kBM / 2 + 4;  // floats per column of an exchange region (64 rows)
-    static constexpr uint32_t kRedBytes = kWaves * kBN * kRedLd * 4;
-    template <class F>
-    static constexpr uint32_t stage_bytes() { return kWaves * 64 * F::kChunks * 16; }
-    template <class F>
-    static constexpr uint32_t red_offset() { return stage_bytes<F>(); }
-    template <class F>
-    static constexpr uint32_t rsl_offset() { return stage_bytes<F>() + kRedBytes; }
-    template <class F>
-    static constexpr uint32_t lds_bytes() { return rsl_offset<F>() + kWaves * kBM * 4; }
-};
-constexpr uint32_t kRowTiles = 4;
+// LDS of a workgroup: the waves' W staging, and in its place after the K loop
+// the partial tiles that the waves exchange (64 rows a wave); then the waves'
+// row scales.
+constexpr uint32_t kRedLd = kBM / 2 + 4;  // floats per column of an exchange region
+template <class F>
+constexpr uint32_t gemm_stage() {
+    const uint32_t stage = kWaves * 64 * F::kChunks * 16, red = kWaves * kBN * kRedLd * 4;
+    return stage > red ? stage : red;
+}
+template <class F>
+constexpr uint32_t gemm_lds() { return gemm_stage<F>() + kWaves * kBM * 4; }
 
 __device__ __forceinline__ floatx16 mfma32(half8 a, half8 b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
@@ -108,6 +107,11 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// 16 bytes of every lane's offset straight to LDS, lane l's to dst + 16 l.
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t rs, uint32_t *dst, uint32_t off, uint32_t soff) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)dst, 16, off, soff, 0, 0);
 }
 
 // Dword x of a span that starts o bytes (0..3) into the aligned dwords d.
@@ -273,16 +277,17 @@ struct FormatQ80 {
     }
 };
 
-// The K blocks [begin, end) wave (or quarter) w of 4 sums over.
-__host__ __device__ inline uint32_t quarter_begin(uint32_t blocks, uint32_t w) { return blocks * w / kWaves; }
+// The K blocks [begin, end) of quarter q.
+__host__ __device__ inline uint32_t quarter_begin(uint32_t blocks, uint32_t q) { return blocks * q / kWaves; }
 
 }  // namespace
 
 // ---------------------------------------------------------------------------
 // A preparation over the padded workspace (rows beyond M are zero).  For the
 // 32-row tile T = m / 32 and lane l = m % 32 + 32 h:
-//   a16[((T * blocks + b) * 16 + s) * 64 + l]  half8: A[m][k] * 2^-e at the
-//       8 columns of step s, half h of block b (F::base, F::kRun)
+//   a16[(((T / 4 * blocks + b) * 16 + s) * 4 + T % 4) * 64 + l]  half8:
+//       A[m][k] * 2^-e at the 8 columns of step s, half h of block b (F::base,
+//       F::kRun)
 //   rowscale[q * mp + m]                       2^e of quarter q of row m
 // Workgroup (g, q) takes rows 8 g .. 8 g + 7 and the K blocks of quarter q:
 // 32 threads per row load the quarter's columns into LDS and find their max,
@@ -364,323 +369,225 @@ __global__ void __launch_bounds__(256) gemm_prep_kernel(const uint16_t *__restri
             v[2 * x] = (_Float16)(__uint_as_float(u[x] << 16) * down);
             v[2 * x + 1] = (_Float16)(__uint_as_float(u[x] & 0xffff0000u) * down);
         }
-        a16[((size_t)(tl * blocks + b0 + bq) * 16 + st) * 64 + l0 + i + 32 * h] = v;
+        a16[(((size_t)(tl / 4 * blocks + b0 + bq) * 16 + st) * 4 + tl % 4) * 64 + l0 + i + 32 * h] = v;
     }
 }
 
 // ---------------------------------------------------------------------------
-// GEMM main kernel.  Grid: one persistent workgroup per CU (at most one per
-// tile); workgroup g takes tiles g, g + grid, ...  Wave w sums over the K
-// blocks of quarter w of each tile; its (tile, block) pairs form one sequence
-// whose loads run ahead across tile boundaries.  Per block: 16 MFMA steps of
-// 4 x 2 MFMAs; step s issues the A loads of step s + kADist, the LDS reads of
-// step s + 2 and the dequantization of step s + 1.  At step 14 (after the
-// last read of the block, made at step 13) the next block's W, fetched into
-// registers a block earlier, is written to the wave's LDS area and the W of
-// the block after it is fetched; the next block's header and first steps
-// are read at steps 14 and 15.
+// GEMM main kernel.  Grid: one workgroup per tile.  Wave w sums over the K
+// blocks of quarter w.  Per block: 16 MFMA steps of 4 x 2 MFMAs; step s issues
+// the A loads of step s + kADist, the LDS reads of step s + 2 and the
+// dequantization of step s + 1.  At step 14 (after the last read of the block,
+// made at step 13) the next block's W is asked for, into the same LDS.
 // ---------------------------------------------------------------------------
-template <class F, uint32_t RM>
-__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(1, 1)))
+template <class F>
+__global__ void __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_kernel(const half8 *__restrict__ a16, uint32_t a_bytes, const float *__restrict__ rowscale, uint32_t mp,
             const uint8_t *__restrict__ w, uint32_t w_bytes, uint32_t m_rows, uint32_t n_rows, uint32_t k,
             uint32_t m_tiles, uint32_t n_tiles, float *__restrict__ c) {
-    using T = Tile<RM>;
-    constexpr uint32_t kChunks = F::kChunks, kStageDwords = 64 * kChunks * 4, kRM = RM, kBM = T::kBM;
-    constexpr uint32_t kRedLd = T::kRedLd;
+    constexpr uint32_t kChunks = F::kChunks, kStageDwords = 64 * kChunks * 4, kRM = kBM / 32;
     extern __shared__ v4u gsm[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: scalar offsets
     const uint32_t ln = lane & 31u, h = lane >> 5;
-    const uint32_t blocks = k / 256, row_bytes = blocks * F::kSpan, tiles = m_tiles * n_tiles;
+    const uint32_t blocks = k / 256, row_bytes = blocks * F::kSpan;
     const uint32_t kb0 = quarter_begin(blocks, wave), kb1 = quarter_begin(blocks, wave + 1);
     uint32_t *stage = (uint32_t *)gsm + wave * kStageDwords;
-    float *red = (float *)((char *)gsm + T::template red_offset<F>());
-    float *rsl = (float *)((char *)gsm + T::template rsl_offset<F>()) + wave * kBM;  // the wave's row scales of the tile
+    float *red = (float *)gsm;
+    float *rsl = (float *)((char *)gsm + gemm_stage<F>()) + wave * kBM;  // the wave's row scales
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(w, w_bytes), ars = make_rsrc(a16, a_bytes);
     const __amdgpu_buffer_rsrc_t crs = make_rsrc(c, m_rows * n_rows * 4);
 
-    // Position in the wave's (tile, block) sequence; t >= tiles past the end.
-    // The 8 XCDs take workgroups round-robin (XCD = id % 8, and the grid is a
-    // multiple of 8 or the tile count), each with its own L2: when the tiles
-    // split evenly, XCD x works on M half x % 2 and N quarter x / 2, so its
-    // half of A stays in its L2 and the tiles sharing a W tile run there.
-    struct Pos {
-        uint32_t t, b, mt, nt;
-    };
-    auto at = [&](uint32_t t, uint32_t b) {
-        Pos p{t, b, 0, 0};
+    // The 8 XCDs take workgroups round-robin (XCD = id % 8), each with its own
+    // L2: when the tiles split evenly, XCD x works on M half x % 2 and N
+    // quarter x / 2, so its half of A stays in its L2 and the tiles sharing a
+    // W tile run there.
+    uint32_t mt, nt;
+    {
+        const uint32_t t = blockIdx.x;
         if (m_tiles % 2 == 0 && n_tiles % 4 == 0) {
             const uint32_t xcd = t % 8, j = t / 8, mh = m_tiles / 2;
-            p.mt = (xcd & 1u) * mh + j % mh;
-            p.nt = (xcd >> 1) * (n_tiles / 4) + j / mh;
+            mt = (xcd & 1u) * mh + j % mh;
+            nt = (xcd >> 1) * (n_tiles / 4) + j / mh;
         } else {
-            p.mt = t % m_tiles;
-            p.nt = t / m_tiles;
+            mt = t % m_tiles;
+            nt = t / m_tiles;
         }
-        return p;
-    };
-    auto next = [&](const Pos &p) { return p.b + 1 < kb1 ? Pos{p.t, p.b + 1, p.mt, p.nt} : at(p.t + gridDim.x, kb0); };
+    }
+    const uint32_t m0 = mt * kBM, n0 = nt * kBN;
+    // this quarter's row scales for the final sum
+    *(float2 *)&rsl[2 * lane] = *(const float2 *)&rowscale[(size_t)wave * mp + m0 + 2 * lane];
 
-    // W staging: chunk j * 64 + lane of the block's 64 rows x kChunks pieces,
-    // which is also its 16-byte slot in the wave's LDS area.  wlane[j] is the
-    // chunk's offset from the first row's span; rows past n start at or past
-    // w_bytes, where buffer loads read zeros (the range check covers the
-    // lane offset, so every row-dependent term goes there).
+    // W staging, straight to LDS: chunk j * 64 + lane of the block's 64 rows x
+    // kChunks pieces goes to its 16-byte slot of the wave's area.  Rows past n
+    // start at or past w_bytes, where buffer loads read zeros (the range check
+    // covers the lane offset, so every row-dependent term goes there).
     uint32_t wlane[kChunks];
 #pragma unroll
     for (uint32_t j = 0; j < kChunks; j++) {
         const uint32_t chunk = j * 64 + lane;
-        wlane[j] = chunk / kChunks * row_bytes + chunk % kChunks * 16;
+        wlane[j] = n0 * row_bytes + chunk / kChunks * row_bytes + chunk % kChunks * 16;
     }
-    v4u wreg[kChunks];
-    auto fetch_w = [&](const Pos &p) {
-        const uint32_t u = p.nt * kBN * row_bytes;
+    auto fetch_w = [&](uint32_t b) {
 #pragma unroll
         for (uint32_t j = 0; j < kChunks; j++) {
-            uint32_t off, soff;
-            if constexpr (F::kAligned) {
-                off = wlane[j] + u;
-                soff = F::kSpan * p.b;
-            } else {
-                off = (wlane[j] + u + F::kSpan * p.b) & ~3u;  // the span's aligned-down start
-                soff = 0;
-            }
-            wreg[j] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(wrs, off, soff, 0));
+            // spans that start between dwords: from their aligned-down start
+            const uint32_t off = F::kAligned ? wlane[j] : (wlane[j] + F::kSpan * b) & ~3u;
+            load_to_lds(wrs, stage + j * 256, off, F::kAligned ? F::kSpan * b : 0);
         }
     };
-    auto put_w = [&]() {
-#pragma unroll
-        for (uint32_t j = 0; j < kChunks; j++) ((v4u *)stage)[j * 64 + lane] = wreg[j];
-    };
-    // A fragment of row tile r (32 rows), step s of p's block.
-    // (The step within its group of 4 goes to the instruction's offset field.)
-    auto a_frag = [&](const Pos &p, uint32_t r, uint32_t s) {
-        const uint32_t off = (((kRM * p.mt + r) * blocks + p.b) * 16 + (s & ~3u)) * 1024;
-        return __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(ars, 16 * lane + 1024 * (s % 4), off, 0));
+    // A fragment of row tile r (32 rows), step s of block b.
+    // (The row tile goes to the instruction's offset field.)
+    auto a_frag = [&](uint32_t b, uint32_t r, uint32_t s) {
+        const uint32_t off = ((mt * blocks + b) * 16 + s) * (kRM * 1024);
+        return __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(ars, 16 * lane + 1024 * r, off, 0));
     };
     // The lane's staged rows (column tile t: row 32 t + ln of the block) and
-    // the span offsets of p's block in them.
+    // the span offsets of block b in them.
     const uint32_t *rows[2] = {stage + ln * kChunks * 4, stage + (32 + ln) * kChunks * 4};
-    auto shift = [&](const Pos &p, int t) { return F::span_shift((p.nt * kBN + 32 * t + ln) * row_bytes, p.b); };
+    auto shift = [&](uint32_t b, int t) { return F::span_shift((n0 + 32 * t + ln) * row_bytes, b); };
 
-    if (blockIdx.x >= tiles) return;
     floatx16 acc[kRM][2];
-    Pos cur = at(blockIdx.x, kb0);
-    const bool any = kb0 < kb1;  // waves of a K shorter than 4 blocks may have none
-    typename F::Scales sc[2];
-    typename F::Step sa[2];  // the LDS data of the step after the current one
-    half8 afr[kRM][kADist], bv[2];
-    uint32_t sh[2] = {0, 0};
-    if (any) {
-        fetch_w(cur);
-        put_w();
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        const Pos n1 = next(cur);
-        if (n1.t < tiles) fetch_w(n1);
+#pragma unroll
+    for (uint32_t r = 0; r < kRM; r++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int j = 0; j < 16; j++) acc[r][t][j] = 0.0f;
+    half8 afr[kRM][kADist];
+    if (kb0 < kb1) {
+        fetch_w(kb0);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (uint32_t s = 0; s < kADist; s++)
 #pragma unroll
-            for (uint32_t r = 0; r < kRM; r++) afr[r][s] = a_frag(cur, r, s);
+            for (uint32_t r = 0; r < kRM; r++) afr[r][s] = a_frag(kb0, r, s);
+    }
+    for (uint32_t b = kb0; b < kb1; b++) {
+        // The block's W is in LDS when the wave's own loads have arrived.
+        uint32_t sh[2];
+        typename F::Scales sc[2];
+        typename F::Step sa[2];  // the LDS data of the step after the current one
+        half8 bv[2];
+        // (the 8 A loads of steps 14 and 15, or of the first two, came after them)
+        __builtin_amdgcn_s_waitcnt(0x0f78);  // vmcnt(8)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
         for (int t = 0; t < 2; t++) {
-            sh[t] = shift(cur, t);
+            sh[t] = shift(b, t);
             sc[t] = F::scales(F::head(rows[t], h, sh[t]), h);
             bv[t] = F::weights(sc[t], F::step(rows[t], h, 0, sh[t]), 0);
             sa[t] = F::step(rows[t], h, 1, sh[t]);
         }
-    }
-    float2 rsv = {0.0f, 0.0f};
-    for (;;) {
-        const uint32_t m0 = cur.mt * kBM, n0 = cur.nt * kBN, tile = cur.t;
+        const uint32_t bn1 = b + 1 < kb1 ? b + 1 : b;  // the A ring's next block (clamped at the end)
 #pragma unroll
-        for (uint32_t r = 0; r < kRM; r++)
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int j = 0; j < 16; j++) acc[r][t][j] = 0.0f;
-        for (uint32_t b = kb0; b < kb1; b++) {
-            const Pos n1 = next(cur);
-            const bool have1 = n1.t < tiles;
-            const Pos &pa = have1 ? n1 : cur;  // the A ring's next block (clamped at the end)
-            if (b + 1 == kb1) {
-                // this quarter's row scales for the final sum, kBM / 64 per lane
-                if constexpr (kBM == 128) {
-                    rsv = *(const float2 *)&rowscale[(size_t)wave * mp + m0 + 2 * lane];
-                } else {
-                    rsv.x = rowscale[(size_t)wave * mp + m0 + lane];
-                }
-            }
-            typename F::Head hn[2];
-            uint32_t shn[2] = {0, 0};
-#pragma unroll
-            for (uint32_t s = 0; s < 16; s++) {
-                __builtin_amdgcn_sched_barrier(0);
-                if (s == 14 && have1) {
-                    // Every LDS read of this block is done (the last, of step
-                    // 15, at step 13); other lanes read what a lane stores, and
-                    // the wave's LDS operations run in order.
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    put_w();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                    const Pos n2 = next(n1);
-                    if (n2.t < tiles) fetch_w(n2);
-#pragma unroll
-                    for (int t = 0; t < 2; t++) {
-                        shn[t] = shift(n1, t);
-                        hn[t] = F::head(rows[t], h, shn[t]);
-                    }
-                }
-                // LDS data of step s + 2 (the next block's first steps at the end)
-                typename F::Step sb[2];
-                if (s + 2 < 16) {
-#pragma unroll
-                    for (int t = 0; t < 2; t++) sb[t] = F::step(rows[t], h, s + 2, sh[t]);
-                } else if (have1) {
-#pragma unroll
-                    for (int t = 0; t < 2; t++) sb[t] = F::step(rows[t], h, s + 2 - 16, shn[t]);
-                }
-                // The A fragments of step s + kADist and the weights of step
-                // s + 1 are produced before this step's MFMAs consume the
-                // current ones, so they live in other registers.
-                half8 an[kRM];
-#pragma unroll
-                for (uint32_t r = 0; r < kRM; r++)
-                    an[r] = s + kADist < 16 ? a_frag(cur, r, s + kADist) : a_frag(pa, r, s + kADist - 16);
-                half8 bn[2];
-                if (s + 1 < 16) {
-#pragma unroll
-                    for (int t = 0; t < 2; t++) bn[t] = F::weights(sc[t], sa[t], s + 1);
-                } else if (have1) {
-#pragma unroll
-                    for (int t = 0; t < 2; t++) {
-                        sc[t] = F::scales(hn[t], h);
-                        bn[t] = F::weights(sc[t], sa[t], 0);
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < 2; t++)
-#pragma unroll
-                    for (uint32_t r = 0; r < kRM; r++) acc[r][t] = mfma32(afr[r][s % kADist], bv[t], acc[r][t]);
-#pragma unroll
-                for (uint32_t r = 0; r < kRM; r++) afr[r][s % kADist] = an[r];
-                if (s + 1 < 16 || have1) {
-#pragma unroll
-                    for (int t = 0; t < 2; t++) {
-                        bv[t] = bn[t];
-                        sa[t] = sb[t];
-                    }
-                }
-            }
+        for (uint32_t s = 0; s < 16; s++) {
             __builtin_amdgcn_sched_barrier(0);
-            sh[0] = shn[0];
-            sh[1] = shn[1];
-            cur = n1;
-        }
-        if (!any) cur = at(tile + gridDim.x, kb0);
-
-        // Final sum of the tile.  Each wave multiplies its quarter's partial
-        // tile by the quarter's row scales, then partners exchange halves
-        // through LDS in two rounds (every wave busy in both): with waves
-        // 0/2 and 1/3 as partners, wave w keeps rows 64 (w / 2) .. + 63 and
-        // hands the other 64 rows to its partner; then with waves 0/1 and 2/3
-        // as partners it keeps rows 32 w .. 32 w + 31 and hands over the
-        // other 32.  Wave w then holds the sum of all four quarters for rows
-        // 32 w .. + 31 and stores them.  Regions are laid out [column][row]
-        // (a lane's 4 consecutive rows of one column are one 16-byte
-        // access); the second round writes into the region the wave itself
-        // read in the first, which no other wave reads.
-        if constexpr (kBM == 128) {
-            *(float2 *)&rsl[2 * lane] = rsv;
-        } else {
-            rsl[lane] = rsv.x;
-        }
-        lds_barrier();  // every wave is done with its K blocks and with the previous tile's final sum
-        constexpr uint32_t kRegion = kBN * kRedLd;  // floats of one exchange region
-        auto slot = [&](uint32_t region, uint32_t row, int t) {
-            return (floatx4 *)&red[region * kRegion + (32 * t + ln) * kRedLd + row];
-        };
-        const uint32_t keep_half = wave >> 1, keep_quarter = wave & 1u;
+            if (s == 14 && b + 1 < kb1) {
+                // Every LDS read of this block is done (the last, of step 15,
+                // at step 13): the next block's W may take its place.
+                __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                fetch_w(b + 1);
+                __builtin_amdgcn_sched_barrier(0);  // the A loads counted on below stay behind it
+            }
+            // LDS data of step s + 2
+            typename F::Step sb[2];
+            if (s + 2 < 16) {
 #pragma unroll
-        for (uint32_t r = 0; r < kRM; r++) {
-            floatx4 rs[4];
+                for (int t = 0; t < 2; t++) sb[t] = F::step(rows[t], h, s + 2, sh[t]);
+            }
+            // The A fragments of step s + kADist and the weights of step
+            // s + 1 are produced before this step's MFMAs consume the
+            // current ones, so they live in other registers.
+            half8 an[kRM];
 #pragma unroll
-            for (int g = 0; g < 4; g++) rs[g] = *(const floatx4 *)&rsl[32 * r + 8 * g + 4 * h];
+            for (uint32_t r = 0; r < kRM; r++)
+                an[r] = s + kADist < 16 ? a_frag(b, r, s + kADist) : a_frag(bn1, r, s + kADist - 16);
+            half8 bn[2];
+            if (s + 1 < 16) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) bn[t] = F::weights(sc[t], sa[t], s + 1);
+            }
 #pragma unroll
             for (int t = 0; t < 2; t++)
 #pragma unroll
-                for (int g = 0; g < 4; g++)
+                for (uint32_t r = 0; r < kRM; r++) acc[r][t] = mfma32(afr[r][s % kADist], bv[t], acc[r][t]);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc[r][t][4 * g + e] *= rs[g][e];
+            for (uint32_t r = 0; r < kRM; r++) afr[r][s % kADist] = an[r];
+            if (s + 1 < 16) {
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    bv[t] = bn[t];
+                    sa[t] = sb[t];
+                }
+            }
         }
-        // first exchange: rows of the other half to region `wave`
-#pragma unroll
-        for (uint32_t r = 0; r < kRM; r++) {
-            if (r / 2 == keep_half) continue;
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-                    *slot(wave, 32 * (r % 2) + 8 * g + 4 * h, t) =
-                        floatx4{acc[r][t][4 * g], acc[r][t][4 * g + 1], acc[r][t][4 * g + 2], acc[r][t][4 * g + 3]};
-        }
-        lds_barrier();
-#pragma unroll
-        for (uint32_t r = 0; r < kRM; r++) {
-            if (r / 2 != keep_half) continue;
-            floatx4 o[2][4];
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int g = 0; g < 4; g++) o[t][g] = *slot(wave ^ 2u, 32 * (r % 2) + 8 * g + 4 * h, t);
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) acc[r][t][4 * g + e] += o[t][g][e];
-        }
-        // second exchange: the other 32 rows of the kept half to region wave ^ 2
-#pragma unroll
-        for (uint32_t r = 0; r < kRM; r++) {
-            if (r / 2 != keep_half || r % 2 == keep_quarter) continue;
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-                    *slot(wave ^ 2u, 8 * g + 4 * h, t) =
-                        floatx4{acc[r][t][4 * g], acc[r][t][4 * g + 1], acc[r][t][4 * g + 2], acc[r][t][4 * g + 3]};
-        }
-        lds_barrier();
-        // rows 32 wave + 8 g + 4 h + e, column n0 + 32 t + ln; rows past m
-        // lie past the end of C, where buffer stores are dropped (the range
-        // check covers the lane offset, which holds the row).  The stores are
-        // non-temporal: C is not read again here, and keeping it out of the
-        // L2 left the N = 4096 kernels 0.5-0.6 us faster (all three types).
-        const bool whole_n = n0 + kBN <= n_rows;
-#pragma unroll
-        for (uint32_t r = 0; r < kRM; r++) {
-            if (r != wave) continue;
-            floatx4 o[2][4];
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int g = 0; g < 4; g++) o[t][g] = *slot(wave ^ 3u, 8 * g + 4 * h, t);
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float v = acc[r][t][4 * g + e] + o[t][g][e];
-                        const uint32_t m = m0 + 32 * r + 8 * g + 4 * h + e, n = n0 + 32 * t + ln;
-                        if (whole_n || n < n_rows)
-                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), crs,
-                                                                  (m * n_rows + n) * 4, 0, 2);
-                    }
-        }
-        if (cur.t >= tiles) break;
+        __builtin_amdgcn_sched_barrier(0);
     }
+
+    // Final sum of the tile.  Each wave multiplies its partial tile by its
+    // quarter's row scales; then partners exchange halves of the rows that both
+    // hold through LDS, in two rounds (every wave busy in both): partners
+    // differ in one bit of the wave, the highest first, and a wave keeps the
+    // upper half of the rows when its bit is set.  Wave w then holds the sum of
+    // all of K for the rows 32 w .. 32 w + 31 and stores them.  Regions are laid
+    // out [column][row] (a lane's 4 consecutive rows of one column are one
+    // 16-byte access); from the second round on a wave writes into the region
+    // it read in the round before, which no other wave reads.
+    // (The lane is taken anew: its pieces need not live through the loop.)
+    const uint32_t lane2 = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    const uint32_t ln2 = lane2 & 31u, h2 = lane2 >> 5;
+    // sum[u][t]: the lane's rows 8 u + 4 h .. + 3 of the rows that the wave holds
+    floatx4 sum[kBM / 8][2];
+#pragma unroll
+    for (uint32_t u = 0; u < kBM / 8; u++) {
+        const floatx4 rs = *(const floatx4 *)&rsl[8 * u + 4 * h2];
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) sum[u][t][e] = acc[u / 4][t][4 * (u % 4) + e] * rs[e];
+    }
+    lds_barrier();  // every wave is done with its W
+    constexpr uint32_t kRegion = kBN * kRedLd;  // floats of one exchange region
+    auto slot = [&](uint32_t region, uint32_t u, int t) {
+        return (floatx4 *)&red[region * kRegion + (32 * t + ln2) * kRedLd + 8 * u + 4 * h2];
+    };
+    uint32_t mine = wave;  // the region it writes
+#pragma unroll
+    for (uint32_t bit = kWaves / 2, units = kBM / 16; bit >= 1; bit >>= 1, units >>= 1) {
+        const bool up = (wave & bit) != 0;
+#pragma unroll
+        for (uint32_t u = 0; u < units; u++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) *slot(mine, u, t) = up ? sum[u][t] : sum[units + u][t];
+        lds_barrier();
+        mine ^= bit;
+#pragma unroll
+        for (uint32_t u = 0; u < units; u++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const floatx4 o = *slot(mine, u, t);
+#pragma unroll
+                for (int e = 0; e < 4; e++) sum[u][t][e] = (up ? sum[units + u][t][e] : sum[u][t][e]) + o[e];
+            }
+    }
+    // rows 8 u + 4 h + e, column n0 + 32 t + ln; rows past m lie past the end
+    // of C, where buffer stores are dropped (the range check covers the lane
+    // offset, which holds the row).  The stores are non-temporal: C is not
+    // read again here, and keeping it out of the L2 left the N = 4096 kernels
+    // 0.5-0.6 us faster (all three types).
+    const bool whole_n = n0 + kBN <= n_rows;
+#pragma unroll
+    for (uint32_t u = 0; u < kBM / 8 / kWaves; u++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const uint32_t m = m0 + kBM / kWaves * wave + 8 * u + 4 * h2 + e, n = n0 + 32 * t + ln2;
+                if (whole_n || n < n_rows)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(sum[u][t][e]), crs, (m * n_rows + n) * 4, 0, 2);
+            }
 }
 
 __global__ void bf16_to_f32_kernel(const uint16_t *__restrict__ a, size_t count, float *__restrict__ out) {
@@ -699,24 +606,18 @@ size_t mfma_workspace(size_t m, size_t k) {
     return mp * k * 2 + 4 * mp * 4 + 2 * 256;
 }
 
-static_assert(Tile<kRowTiles>::lds_bytes<FormatQ80>() <= 160 * 1024, "one workgroup's LDS");
+static_assert(gemm_lds<FormatQ80>() <= 80 * 1024, "two workgroups a CU");
 
-template <class F, uint32_t RM>
+template <class F>
 int launch_gemm(dmhip_ctx *ctx, size_t mp, size_t m, size_t n, size_t k, const half8 *a16, const float *rowscale,
                 const void *weights, uint64_t w_bytes, float *c) {
-    using T = Tile<RM>;
-    const uint32_t m_tiles = (uint32_t)(mp / T::kBM), n_tiles = (uint32_t)((n + kBN - 1) / kBN);
-    const uint32_t tiles = m_tiles * n_tiles;
-    // one workgroup per CU, a multiple of the 8 XCDs
-    uint32_t grid = ctx->compute_units > 0 ? (uint32_t)ctx->compute_units / 8 * 8 : 256u;
-    if (grid == 0) grid = 8;
-    if (tiles < grid) grid = tiles;
-    constexpr uint32_t lds = T::template lds_bytes<F>();
+    const uint32_t m_tiles = (uint32_t)(mp / kBM), n_tiles = (uint32_t)((n + kBN - 1) / kBN);
+    constexpr uint32_t lds = gemm_lds<F>();
     static LdsLimit limit;
-    DM_HIP(limit.ensure((const void *)gemm_kernel<F, RM>, lds));
-    DM_HIP(launch_kernel(ctx, gemm_kernel<F, RM>, dim3(grid), dim3(64 * kWaves), lds, a16, (uint32_t)(mp * k * 2),
-                         rowscale, (uint32_t)mp, (const uint8_t *)weights, (uint32_t)w_bytes, (uint32_t)m, (uint32_t)n,
-                         (uint32_t)k, m_tiles, n_tiles, c));
+    DM_HIP(limit.ensure((const void *)gemm_kernel<F>, lds));
+    DM_HIP(launch_kernel(ctx, gemm_kernel<F>, dim3(m_tiles * n_tiles), dim3(64 * kWaves), lds, a16,
+                         (uint32_t)(mp * k * 2), rowscale, (uint32_t)mp, (const uint8_t *)weights, (uint32_t)w_bytes,
+                         (uint32_t)m, (uint32_t)n, (uint32_t)k, m_tiles, n_tiles, c));
     return DMHIP_OK;
 }
 
@@ -736,7 +637,7 @@ int run_gemm(dmhip_ctx *ctx, size_t m, size_t n, size_t k, const uint16_t *a_bf1
     hipLaunchKernelGGL(gemm_prep_kernel<F>, dim3((uint32_t)(mp / 8), kWaves), dim3(256), prep_lds, ctx->stream,
                        a_bf16, (uint32_t)m, (uint32_t)k, (uint32_t)mp, a16, rowscale);
     DM_HIP(hipGetLastError());
-    return launch_gemm<F, kRowTiles>(ctx, mp, m, n, k, a16, rowscale, weights, w_bytes, c);
+    return launch_gemm<F>(ctx, mp, m, n, k, a16, rowscale, weights, w_bytes, c);
 }
 
 }  // namespace

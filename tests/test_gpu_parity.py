@@ -1573,6 +1573,24 @@ def test_prefill_gemm_ragged_shapes(ctx, kind, m, n, k):
     _gemm_check(ctx, kind, m, n, k, 7, "ragged")
 
 
+@pytest.mark.parametrize("kind", [Q4_K, Q6_K, Q8_0])
+@pytest.mark.parametrize("m,n,k", [(128, 65, 512), (129, 128, 768), (257, 1028, 1280)])
+def test_prefill_gemm_tile_edges(ctx, kind, m, n, k):
+    """One row or column past a tile, quarters of 0, 1 and 2 or of unequal
+    blocks.  Held to the per-channel bound alone: it is derived per element, while the
+    per-token metric divides by the largest of a token's n outputs, which at
+    65 columns is no bound on the rest."""
+    print(f"tile edges: type {kind} m={m} n={n} k={k}", flush=True)
+    a = synth.to_bf16_bits(synth.normal(synth.activation_seed(8, kind), m * k))
+    w = synth.quantized_matrix(kind, n, k, synth.weight_seed(8, n * 31 + kind))
+    ab, wb, cb = dev(ctx, a), dev(ctx, w), dev_out(ctx, m * n * 4)
+    ws = dev_out(ctx, ctx.gemm_workspace_bytes(m, k))
+    ctx.gemm_device(kind, m, n, k, ab.device_ptr, wb.device_ptr, cb.device_ptr, ws.device_ptr, len(ws))
+    got = cb.read(0, m * n * 4, np.float32).reshape(m, n)
+    exact, scale = exact_products(kind, n, k, w, synth.bf16_bits_to_f32(a).reshape(m, k))
+    assert_channel_close(got, exact, scale, CHANNEL_TOL_GEMM, f"type {kind}")
+
+
 def test_objects_outliving_their_context_exit_cleanly():
     """Regression: device buffers and caches freed after their context was
     closed (the order Python's collector may pick at exit)."""
