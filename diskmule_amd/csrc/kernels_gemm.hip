@@ -395,7 +395,9 @@ gemm_kernel(const half8 *__restrict__ a16, uint32_t a_bytes, const float *__rest
     uint32_t *stage = (uint32_t *)gsm + wave * kStageDwords;
     float *red = (float *)gsm;
     float *rsl = (float *)((char *)gsm + gemm_stage<F>()) + wave * kBM;  // the wave's row scales
-    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(w, w_bytes), ars = make_rsrc(a16, a_bytes);
+    // (the range ends with a whole dword: the last one of a length that is not a
+    // multiple of 4 would read as 0)
+    const __amdgpu_buffer_rsrc_t wrs = make_rsrc(w, (w_bytes + 3) & ~3u), ars = make_rsrc(a16, a_bytes);
     const __amdgpu_buffer_rsrc_t crs = make_rsrc(c, m_rows * n_rows * 4);
 
     // The 8 XCDs take workgroups round-robin (XCD = id % 8), each with its own

@@ -1574,10 +1574,12 @@ def test_prefill_gemm_ragged_shapes(ctx, kind, m, n, k):
 
 
 @pytest.mark.parametrize("kind", [Q4_K, Q6_K, Q8_0])
-@pytest.mark.parametrize("m,n,k", [(128, 65, 512), (129, 128, 768), (257, 1028, 1280)])
+@pytest.mark.parametrize("m,n,k", [(128, 65, 512), (129, 127, 768), (257, 1027, 1280), (200, 61, 2304)])
 def test_prefill_gemm_tile_edges(ctx, kind, m, n, k):
     """One row or column past a tile, quarters of 0, 1 and 2 or of unequal
-    blocks.  Held to the per-channel bound alone: it is derived per element, while the
+    blocks, and odd row counts of odd block counts, whose Q6_K bytes end
+    between dwords (the last block's d lies in the last, partial one).  Held
+    to the per-channel bound alone: it is derived per element, while the
     per-token metric divides by the largest of a token's n outputs, which at
     65 columns is no bound on the rest."""
     print(f"tile edges: type {kind} m={m} n={n} k={k}", flush=True)
