@@ -117,9 +117,9 @@ int dmhip_ffn_device_noalloc(dmhip_ctx *ctx, size_t batch, size_t hidden, size_t
     if (batch < 1 || batch > 16)
         return fail(DMHIP_ERR_INVALID_ARGUMENT, "batch %zu is outside 1..=16", batch);
     const size_t ws = dmhip_ffn_workspace_bytes(batch, hidden, ffn);
-    // batches above 2 prepare activation fragments of h (gate and up, whose
-    // types may differ and need different fragment sets) and of the
-    // activation rows (down); the largest of the three regions is lent
+    // batches above 2 are accepted up to the scratch that their activations as
+    // fp16 pairs take: h (gate and up, whose types may differ) or the
+    // activation rows (down), the largest of the three
     size_t lend = 0;
     if (batch > 2) {
         const uint32_t types[3] = {gate_type, up_type, down_type};
@@ -137,16 +137,6 @@ int dmhip_ffn_device_noalloc(dmhip_ctx *ctx, size_t batch, size_t hidden, size_t
     const int device = ctx->device;
     void *base = (device >= 0 && device < 64) ? g_scratch_address[device].load(std::memory_order_acquire) : nullptr;
     if (!base) return fail(DMHIP_ERR_COMMAND, "the allocation-free scratch of device %d is not resolved", device);
-    // the fp16 path's fragments go to the lent region for this call only
-    struct Lend {
-        dmhip_ctx *c;
-        ~Lend() {
-            c->aux_lent = nullptr;
-            c->aux_lent_bytes = 0;
-        }
-    } guard{ctx};
-    ctx->aux_lent = batch > 2 ? (char *)base + ws : nullptr;
-    ctx->aux_lent_bytes = batch > 2 ? lend : 0;
     return dmhip_ffn_device(ctx, batch, hidden, ffn, gate_type, gate, up_type, up, down_type, down, epsilon, h, y,
                            base, ws);
 }

@@ -106,8 +106,8 @@ hipError_t launch_qmv_experts(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uint
                               uint64_t up_offset, const uint64_t *w_of, const uint32_t *ids, const uint32_t *go,
                               uint32_t tokens, uint32_t k, const float *x, float *y);
 
-// Bytes of the activation fragments the fp16 kernel prepares for `batch`
-// tokens (batches above 2) of rows of `columns` values.
+// The scratch that the allocation-free entry point reckons per batch above 2 of
+// rows of `columns` values when it accepts or rejects a shape.
 size_t qmv_prepare_bytes(uint32_t type, size_t columns, size_t batch);
 
 // y[b][r] = W[r] . x[b]; when `argmax` is non-null (batch 1) the kernels

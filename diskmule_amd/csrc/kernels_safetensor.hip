@@ -14,7 +14,7 @@
 // st_gemv_kernel is the wide-load form (rows of whole 16-byte chunks, the
 // activation in LDS): a workgroup of 4 waves stages x once and walks row
 // pairs persistently; lane l reads chunks l, l + 64, ... of each row, eight
-// per row in flight.  The block or group scale multiplies a chunk's partial
+// per row in flight (rows of at most four: the next step's too).  The block or group scale multiplies a chunk's partial
 // sum (one rounding order; the sum runs in a different order than the
 // reference's sequential fold, within the dot-product tolerance).  INT4
 // chunks sum n * x with one v_cvt_f32_ubyte per code and subtract 8 times
@@ -61,10 +61,17 @@ __device__ __forceinline__ float fp8_formula(uint32_t b) {
 
 }  // namespace
 
+// Workgroup barrier ordering LDS only: weights in flight are not waited for.
+__device__ __forceinline__ void st_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // y[r] = sum_c W[r][c] x[c], one token.  scales: F8 [ceil(rows/128)][sc],
 // INT8 [rows], INT4 [rows][sc] with `group` columns per scale.
 // R rows per wave step, C chunks of each row in flight per lane.
-template <uint32_t FMT, uint32_t kStRows, uint32_t kStChunks>
+template <uint32_t FMT, uint32_t kStRows, uint32_t kStChunks, bool PIPE>
 __global__ void __launch_bounds__(64 * kStWaves)
 st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, size_t row_bytes,
                const float *__restrict__ scales, uint32_t scale_columns, uint32_t group, const float *__restrict__ x,
@@ -76,17 +83,55 @@ st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, s
     extern __shared__ __attribute__((aligned(16))) float xs[];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t chunks = columns / E;
+    // One step: kStChunks chunks of a lane in each of kStRows rows.  The
+    // chunks' weights and their block / group scales are all in flight before
+    // the first is used.
+    constexpr int NS = FMT == kStF8 || FMT == kStI4 ? (FMT == kStI4 ? 2 : 1) : 0;
+    struct Step {
+        u32x4 v[kStRows][kStChunks];
+        float sv[kStRows][kStChunks][NS > 0 ? NS : 1];
+    };
+    auto load = [&](Step &st, uint32_t r0, uint32_t c0) {
+#pragma unroll
+        for (uint32_t r = 0; r < kStRows; r++)
+#pragma unroll
+            for (uint32_t j = 0; j < kStChunks; j++) {
+                const uint32_t c = c0 + 64 * j + lane;
+                const bool ok = r0 + r < rows && c < chunks;
+                st.v[r][j] = ok ? *(const u32x4 *)(w + (size_t)(r0 + r) * row_bytes + (size_t)c * 16)
+                                : u32x4{0, 0, 0, 0};
+                if constexpr (FMT == kStF8) {
+                    // the chunk's 16 columns lie in one 128-column block
+                    st.sv[r][j][0] = ok ? scales[((r0 + r) / 128) * scale_columns + c / 8] : 0.0f;
+                } else if constexpr (FMT == kStI4) {
+                    const float *srow = scales + (size_t)(r0 + r) * scale_columns;
+                    // group 16: a scale per half chunk; else one per chunk
+                    st.sv[r][j][0] = ok ? srow[group == 16 ? 2 * c : (32 * c) / group] : 0.0f;
+                    st.sv[r][j][1] = ok && group == 16 ? srow[2 * c + 1] : 0.0f;
+                }
+            }
+    };
+    const uint32_t step = gridDim.x * kStWaves * kStRows;
+    uint32_t r0 = (blockIdx.x * kStWaves + wave) * kStRows;
+    // PIPE (rows of one step): a step's weights are asked for before the step
+    // before it is summed, the first before x is staged.
+    Step cur;
     {
         // every load of a thread in flight before the first store (columns <= 16384;
         // measured at 12288 x 6144: F8 16.6 -> 15.9 us, INT8 16.3 -> 15.5 us, BF16
         // 26.2 -> 25.6 us per launch against one load in flight at a time)
-        constexpr uint32_t kXU = 16;
+        constexpr uint32_t kXU = PIPE ? E * kStChunks / 16 : 16;
         const uint32_t n4 = columns / 4;
         floatx4 t[kXU];
 #pragma unroll
         for (uint32_t j = 0; j < kXU; j++) {
             const uint32_t i = j * 64 * kStWaves + threadIdx.x;
             t[j] = i < n4 ? ((const floatx4 *)x)[i] : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        if constexpr (PIPE) {
+            __builtin_amdgcn_sched_barrier(0);
+            load(cur, r0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (uint32_t j = 0; j < kXU; j++) {
@@ -96,7 +141,7 @@ st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, s
     }
     float *xsum = xs + chunks * XP;
     if constexpr (FMT == kStI4) {
-        __syncthreads();
+        st_barrier();
         for (uint32_t i = threadIdx.x; i < columns / 16; i += 64 * kStWaves) {
             const float *src = xs + (i / 2) * XP + 16 * (i % 2);
             floatx4 q[4];
@@ -108,103 +153,101 @@ st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, s
             xsum[i] = s;
         }
     }
-    __syncthreads();
-    const uint32_t step = gridDim.x * kStWaves * kStRows;
-    for (uint32_t r0 = (blockIdx.x * kStWaves + wave) * kStRows; r0 < rows; r0 += step) {
-        float acc[kStRows] = {};
-        for (uint32_t c0 = 0; c0 < chunks; c0 += 64 * kStChunks) {
-            // the chunks' weights and their block / group scales, all in flight
-            // before the first is used
-            constexpr int NS = FMT == kStF8 || FMT == kStI4 ? (FMT == kStI4 ? 2 : 1) : 0;
-            u32x4 v[kStRows][kStChunks];
-            float sv[kStRows][kStChunks][NS > 0 ? NS : 1];
+    st_barrier();
+    auto add = [&](const Step &st, uint32_t c0, float (&acc)[kStRows]) {
 #pragma unroll
-            for (uint32_t r = 0; r < kStRows; r++)
+        for (uint32_t j = 0; j < kStChunks; j++) {
+            const uint32_t c = c0 + 64 * j + lane;
+            if (c >= chunks) break;
+            float xv[E];
 #pragma unroll
-                for (uint32_t j = 0; j < kStChunks; j++) {
-                    const uint32_t c = c0 + 64 * j + lane;
-                    const bool ok = r0 + r < rows && c < chunks;
-                    v[r][j] = ok ? *(const u32x4 *)(w + (size_t)(r0 + r) * row_bytes + (size_t)c * 16)
-                                 : u32x4{0, 0, 0, 0};
-                    if constexpr (FMT == kStF8) {
-                        // the chunk's 16 columns lie in one 128-column block
-                        sv[r][j][0] = ok ? scales[((r0 + r) / 128) * scale_columns + c / 8] : 0.0f;
-                    } else if constexpr (FMT == kStI4) {
-                        const float *srow = scales + (size_t)(r0 + r) * scale_columns;
-                        // group 16: a scale per half chunk; else one per chunk
-                        sv[r][j][0] = ok ? srow[group == 16 ? 2 * c : (32 * c) / group] : 0.0f;
-                        sv[r][j][1] = ok && group == 16 ? srow[2 * c + 1] : 0.0f;
+            for (uint32_t q = 0; q < E / 4; q++) {
+                const floatx4 f = *(const floatx4 *)&xs[c * XP + 4 * q];
+#pragma unroll
+                for (int e = 0; e < 4; e++) xv[4 * q + e] = f[e];
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < kStRows; r++) {
+                if constexpr (FMT == kStBf16) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        acc[r] = __builtin_fmaf(bf16_bits(st.v[r][j][i] & 0xffffu), xv[2 * i], acc[r]);
+                        acc[r] = __builtin_fmaf(bf16_bits(st.v[r][j][i] >> 16), xv[2 * i + 1], acc[r]);
                     }
-                }
+                } else if constexpr (FMT == kStI8) {
 #pragma unroll
-            for (uint32_t j = 0; j < kStChunks; j++) {
-                const uint32_t c = c0 + 64 * j + lane;
-                if (c >= chunks) break;
-                float xv[E];
+                    for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (uint32_t q = 0; q < E / 4; q++) {
-                    const floatx4 f = *(const floatx4 *)&xs[c * XP + 4 * q];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) xv[4 * q + e] = f[e];
-                }
-#pragma unroll
-                for (uint32_t r = 0; r < kStRows; r++) {
-                    if constexpr (FMT == kStBf16) {
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            acc[r] = __builtin_fmaf(bf16_bits(v[r][j][i] & 0xffffu), xv[2 * i], acc[r]);
-                            acc[r] = __builtin_fmaf(bf16_bits(v[r][j][i] >> 16), xv[2 * i + 1], acc[r]);
+                        for (int b = 0; b < 4; b++) {
+                            const float q = (float)(int32_t)((int32_t)(st.v[r][j][i] << (24 - 8 * b)) >> 24);
+                            acc[r] = __builtin_fmaf(q, xv[4 * i + b], acc[r]);
                         }
-                    } else if constexpr (FMT == kStI8) {
+                } else if constexpr (FMT == kStF8) {
+                    float s = 0.0f;
 #pragma unroll
-                        for (int i = 0; i < 4; i++)
+                    for (int i = 0; i < 4; i++) {
+                        float d[4];
+                        fp8x4(st.v[r][j][i], d);
 #pragma unroll
-                            for (int b = 0; b < 4; b++) {
-                                const float q = (float)(int32_t)((int32_t)(v[r][j][i] << (24 - 8 * b)) >> 24);
-                                acc[r] = __builtin_fmaf(q, xv[4 * i + b], acc[r]);
-                            }
-                    } else if constexpr (FMT == kStF8) {
-                        float s = 0.0f;
+                        for (int b = 0; b < 4; b++) s = __builtin_fmaf(d[b], xv[4 * i + b], s);
+                    }
+                    acc[r] = __builtin_fmaf(st.sv[r][j][0], s, acc[r]);
+                } else {
+                    // 32 codes: dword i holds columns 8i .. 8i + 7, low nibble first
+                    float s[2] = {0.0f, 0.0f};
 #pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            float d[4];
-                            fp8x4(v[r][j][i], d);
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t even = st.v[r][j][i] & 0x0f0f0f0fu, odd = (st.v[r][j][i] >> 4) & 0x0f0f0f0fu;
 #pragma unroll
-                            for (int b = 0; b < 4; b++) s = __builtin_fmaf(d[b], xv[4 * i + b], s);
+                        for (int b = 0; b < 4; b++) {
+                            s[i >> 1] = __builtin_fmaf((float)((even >> (8 * b)) & 0xffu), xv[8 * i + 2 * b], s[i >> 1]);
+                            s[i >> 1] = __builtin_fmaf((float)((odd >> (8 * b)) & 0xffu), xv[8 * i + 2 * b + 1], s[i >> 1]);
                         }
-                        acc[r] = __builtin_fmaf(sv[r][j][0], s, acc[r]);
+                    }
+                    const float h0 = __builtin_fmaf(-8.0f, xsum[2 * c], s[0]);
+                    const float h1 = __builtin_fmaf(-8.0f, xsum[2 * c + 1], s[1]);
+                    if (group == 16) {
+                        acc[r] = __builtin_fmaf(st.sv[r][j][0], h0, acc[r]);
+                        acc[r] = __builtin_fmaf(st.sv[r][j][1], h1, acc[r]);
                     } else {
-                        // 32 codes: dword i holds columns 8i .. 8i + 7, low nibble first
-                        float s[2] = {0.0f, 0.0f};
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const uint32_t even = v[r][j][i] & 0x0f0f0f0fu, odd = (v[r][j][i] >> 4) & 0x0f0f0f0fu;
-#pragma unroll
-                            for (int b = 0; b < 4; b++) {
-                                s[i >> 1] = __builtin_fmaf((float)((even >> (8 * b)) & 0xffu), xv[8 * i + 2 * b], s[i >> 1]);
-                                s[i >> 1] = __builtin_fmaf((float)((odd >> (8 * b)) & 0xffu), xv[8 * i + 2 * b + 1], s[i >> 1]);
-                            }
-                        }
-                        const float h0 = __builtin_fmaf(-8.0f, xsum[2 * c], s[0]);
-                        const float h1 = __builtin_fmaf(-8.0f, xsum[2 * c + 1], s[1]);
-                        if (group == 16) {
-                            acc[r] = __builtin_fmaf(sv[r][j][0], h0, acc[r]);
-                            acc[r] = __builtin_fmaf(sv[r][j][1], h1, acc[r]);
-                        } else {
-                            // group a multiple of 32: one scale for the chunk
-                            acc[r] = __builtin_fmaf(sv[r][j][0], h0 + h1, acc[r]);
-                        }
+                        // group a multiple of 32: one scale for the chunk
+                        acc[r] = __builtin_fmaf(st.sv[r][j][0], h0 + h1, acc[r]);
                     }
                 }
             }
         }
+    };
+    auto finish = [&](uint32_t row, const float (&acc)[kStRows]) {
 #pragma unroll
         for (uint32_t r = 0; r < kStRows; r++) {
             float s = wave_sum(acc[r]);
-            if (lane == 0 && r0 + r < rows) {
-                if constexpr (FMT == kStI8) s *= scales[r0 + r];
-                y[r0 + r] = s;
+            if (lane == 0 && row + r < rows) {
+                if constexpr (FMT == kStI8) s *= scales[row + r];
+                y[row + r] = s;
             }
+        }
+    };
+    if constexpr (PIPE) {
+        Step next;
+        for (; r0 < rows; r0 += 2 * step) {
+            float acc[kStRows] = {};
+            load(next, r0 + step, 0);
+            add(cur, 0, acc);
+            finish(r0, acc);
+            if (r0 + step >= rows) break;
+            float acc2[kStRows] = {};
+            load(cur, r0 + 2 * step, 0);
+            add(next, 0, acc2);
+            finish(r0 + step, acc2);
+        }
+    } else {
+        for (; r0 < rows; r0 += step) {
+            float acc[kStRows] = {};
+            for (uint32_t c0 = 0; c0 < chunks; c0 += 64 * kStChunks) {
+                load(cur, r0, c0);
+                add(cur, c0, acc);
+            }
+            finish(r0, acc);
         }
     }
 }
@@ -239,17 +282,22 @@ st_gemv_generic_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t co
 
 namespace {
 
-template <uint32_t FMT, uint32_t R, uint32_t C>
+template <uint32_t FMT, uint32_t R, uint32_t C, bool PIPE>
 hipError_t launch_st_rc(hipStream_t s, int cus, const uint8_t *w, uint32_t rows, uint32_t columns, size_t row_bytes,
                         const float *scales, uint32_t scale_columns, uint32_t group, const float *x, float *y) {
     const uint32_t lds = (columns / kStPerChunk<FMT>) * (kStPerChunk<FMT> + 4) * 4 + (FMT == kStI4 ? (columns / 16) * 4 : 0);
     static LdsLimit limit;
-    hipError_t e = limit.ensure((const void *)st_gemv_kernel<FMT, R, C>, lds);
+    hipError_t e = limit.ensure((const void *)st_gemv_kernel<FMT, R, C, PIPE>, lds);
     if (e != hipSuccess) return e;
     const uint32_t groups = (rows + kStWaves * R - 1) / (kStWaves * R);
     const uint32_t cap = (uint32_t)(cus > 0 ? cus : 256) * 4;
-    const uint32_t grid = groups < cap ? groups : cap;
-    hipLaunchKernelGGL((st_gemv_kernel<FMT, R, C>), dim3(grid), dim3(64 * kStWaves), lds, s, w, rows, columns,
+    uint32_t grid = groups < cap ? groups : cap;
+    if (PIPE) {
+        // the same number of steps for every workgroup
+        const uint32_t steps = (groups + grid - 1) / grid;
+        grid = (groups + steps - 1) / steps;
+    }
+    hipLaunchKernelGGL((st_gemv_kernel<FMT, R, C, PIPE>), dim3(grid), dim3(64 * kStWaves), lds, s, w, rows, columns,
                        row_bytes, scales, scale_columns, group, x, y);
     return hipGetLastError();
 }
@@ -261,7 +309,16 @@ hipError_t launch_st_t(hipStream_t s, int cus, const uint8_t *w, uint32_t rows, 
     // INT4 12288 x 6144 in 19.3 against 16.5 us, fewer workgroups; so did
     // 3 rows x 8 chunks for every format, e.g. INT4 18.0 against 16.3 us and
     // F8 18.7 against 17.0 us)
-    return launch_st_rc<FMT, 2, 8>(s, cus, w, rows, columns, row_bytes, scales, scale_columns, group, x, y);
+    // Rows of at most 4 chunks a lane run pipelined (a step's weights asked for
+    // before the step before it is summed, the first before x is staged, every
+    // workgroup the same number of steps).  In us, without / with: 16384 x 1024
+    // F8 8.5 / 5.3, INT8 6.7 / 5.9, BF16 7.6 / 7.1; 6144 x 4096 equal (F8 7.2 /
+    // 7.3, INT8 7.4 / 7.2).  INT4 up to one chunk a lane only: 16384 x 1024
+    // 10.8 / 9.5, but 6144 x 4096 7.0 / 9.7 and 12288 x 6144 14.3 / 17.3 (174
+    // registers leave two workgroups on a CU).
+    if (columns / kStPerChunk<FMT> <= (FMT == kStI4 ? 64 : 64 * 4))
+        return launch_st_rc<FMT, 2, 4, true>(s, cus, w, rows, columns, row_bytes, scales, scale_columns, group, x, y);
+    return launch_st_rc<FMT, 2, 8, false>(s, cus, w, rows, columns, row_bytes, scales, scale_columns, group, x, y);
 }
 
 template <uint32_t FMT>
@@ -307,7 +364,7 @@ hipError_t launch_st_gemv(hipStream_t s, int cus, uint32_t fmt, const void *w, u
 }
 
 // A kernel of this file: resolving it loads the file's code object.
-const void *module_anchor_safetensor() { return (const void *)st_gemv_kernel<kStBf16, 2, 8>; }
+const void *module_anchor_safetensor() { return (const void *)st_gemv_kernel<kStBf16, 2, 8, false>; }
 
 }  // namespace dm
 

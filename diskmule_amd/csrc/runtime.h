@@ -104,10 +104,6 @@ struct dmhip_ctx {
     dm::Scratch attn;                        // attention chunk partials
     dm::Scratch attn_tickets;                // attention combine counters, zero between calls
     size_t attn_ticket_count = 0;            // counters in attn_tickets already zeroed
-    // Device memory an allocation-free call lends the fp16 matvec (K-split
-    // partial sums) in place of `aux` for its duration (null otherwise).
-    void *aux_lent = nullptr;
-    size_t aux_lent_bytes = 0;
     dm::ArgmaxState *argmax_state = nullptr;  // device
     uint32_t *router_tickets = nullptr;       // device, kRouterTickets counters, zero between launches
     uint32_t router_mark = 0;                 // mark of the pending device router calls (BadFlag), never 0 once set

@@ -338,7 +338,7 @@ int dmhip_ffn_device(dmhip_ctx *ctx, size_t batch, size_t hidden, size_t ffn,
    scratch comes from a fixed array in the library's code object of
    dmhip_ffn_noalloc_scratch_bytes() bytes (8 MiB) per device, resolved when
    a context is created on that device; a shape whose workspace (and, for
-   batches above 2, activation fragments) exceed it is rejected
+   batches above 2, the activations as fp16 pairs) exceed it is rejected
    (InvalidArgument) before any work.  Nothing is allocated: no hipMalloc,
    no growth of the context's scratch.  Every call on one device shares that
    device's array, so calls that overlap on one device (two contexts, or two

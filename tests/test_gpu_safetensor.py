@@ -178,6 +178,18 @@ def test_seeded_parity(ctx, fmt, rows, cols, group):
     assert (diff <= b).all(), f"{fmt}: worst {float((diff / b).max()):.3f}x the bound"
 
 
+@pytest.mark.parametrize("fmt,rows,cols,group", [
+    ("BF16", 8193, 2048, 0), ("BF16", 9, 2056, 0), ("F8_E4M3", 16391, 16, 0), ("F8_E4M3", 40, 4096, 0),
+    ("I8", 16385, 48, 0), ("I8", 40, 4112, 0), ("I4", 16399, 32, 16), ("I4", 40, 2048, 32), ("I4", 40, 2080, 32),
+])
+def test_pipelined_rows_edges(ctx, fmt, rows, cols, group):
+    """The longest rows of the pipelined form and the first past them, row
+    counts one past a workgroup's 8, and workgroups of two and three steps
+    (8193 to 16399 rows on 1024 workgroups), the last ones partly or wholly past the
+    end.  Bound: the one of the seeded cases."""
+    test_seeded_parity(ctx, fmt, rows, cols, group)
+
+
 def test_device_entry_point_matches_the_host_one(ctx):
     rng = np.random.default_rng(5)
     for fmt, rows, cols, group in (("F8_E4M3", 1024, 2048, 0), ("I4", 1024, 2048, 32), ("I8", 513, 2048, 0),
