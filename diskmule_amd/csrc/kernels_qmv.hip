@@ -27,8 +27,8 @@
 //
 // Data movement: see qmv_kernel.
 #include "dm_device.h"
+#include "dm_plan.h"
 #include "dm_qmv.h"
-
 
 namespace dm {
 
@@ -909,7 +909,7 @@ qmv_kernel(const QmvArgs p) {
 // which experts are selected and takes its share of one of them: with n
 // (expert, 8 tokens) entries, gridDim.x / n workgroups each.  The grid is two
 // 8-wave workgroups per CU, so one's prologue runs beside the other's
-// stream.
+// stream, and at least one per pair (experts_grid).
 template <uint32_t TYPE, int MODE, int KB, uint32_t W>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(KB > 2 ? 2 : 4, KB > 2 ? 2 : 4)))
 qmv_experts_kernel(const QmvArgs args, const QmvExperts ex) {
@@ -944,7 +944,7 @@ qmv_experts_kernel(const QmvArgs args, const QmvExperts ex) {
             if ((int)tid >= d) upto += v;
         }
         const uint32_t total = __shfl(upto, 63, 64);
-        const uint32_t share = gridDim.x / total ? gridDim.x / total : 1u;
+        const uint32_t share = experts_share(gridDim.x, total);
         const uint32_t entry = blockIdx.x / share;
         if (entry < total) {
             uint32_t base = upto - sum, mine = ~0u, from = 0;
@@ -1133,12 +1133,13 @@ hipError_t dispatch_experts(dmhip_ctx *ctx, uint32_t rows, uint32_t columns, con
     const uint32_t waves = 8 / wave_k * wave_k;
     const uint32_t cus = ctx->compute_units > 0 ? (uint32_t)ctx->compute_units : 256u;
     const QmvArgs a{nullptr, nullptr, x, y, nullptr, rows, columns, blocks * StageQ<TYPE>::bytes, 0, wave_k, 1, 1, 1, 0, 0.0f};
+    const uint32_t grid = experts_grid(cus, ex.pairs);
     // (rows of 3 or 6 blocks keep 6 waves busy, whose ring has room for
     // another slot each)
-    if (waves == 6 && kb == 1) return run_experts<TYPE, MODE, 1, 6>(ctx, a, ex, waves, 2 * cus);
-    if (kb == 1) return run_experts<TYPE, MODE, 1, 8>(ctx, a, ex, waves, 2 * cus);
-    if (kb == 2) return run_experts<TYPE, MODE, 2, 8>(ctx, a, ex, waves, 2 * cus);
-    return run_experts<TYPE, MODE, 3, 8>(ctx, a, ex, waves, 2 * cus);
+    if (waves == 6 && kb == 1) return run_experts<TYPE, MODE, 1, 6>(ctx, a, ex, waves, grid);
+    if (kb == 1) return run_experts<TYPE, MODE, 1, 8>(ctx, a, ex, waves, grid);
+    if (kb == 2) return run_experts<TYPE, MODE, 2, 8>(ctx, a, ex, waves, grid);
+    return run_experts<TYPE, MODE, 3, 8>(ctx, a, ex, waves, grid);
 }
 
 }  // namespace
