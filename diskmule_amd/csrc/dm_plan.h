@@ -17,4 +17,76 @@ constexpr uint32_t experts_grid(uint32_t cus, uint32_t pairs) { return 2 * cus >
 // Workgroups per entry; workgroup b works on entry b / share, if there is one.
 constexpr uint32_t experts_share(uint32_t grid, uint32_t entries) { return grid > entries ? grid / entries : 1u; }
 
+// ---- the fp16 matvec (kernels_qmv.hip) ----
+struct QmvPlan {
+    uint32_t kb, waves, wave_k, k_parts, row_groups, phases;
+};
+
+// The K split.  A workgroup of 16 waves of up to 128 registers holds the
+// fragments of 8 tokens of up to 32 blocks (2 per wave; a gate/up pair, which
+// needs more registers besides, 16), one of 8 waves of 256 those of 16
+// tokens of 16 blocks, or of 8 tokens of a pair's 24.  Longer rows, and
+// matrices with fewer tiles than CUs, are split over k_parts workgroups;
+// gate/up pairs, whose epilogue needs whole sums, go through longer rows in
+// phases instead.  The split minimises the largest workgroup's share of the
+// weights; within it, the most waves share K.
+constexpr QmvPlan qmv_split(uint32_t parts, uint32_t tiles, uint32_t blocks, uint32_t batch, int mode, uint32_t cus) {
+    QmvPlan p{};
+    p.k_parts = parts;
+    const uint32_t part_blocks = (blocks + parts - 1) / parts;
+    p.phases = 1;
+    if (batch <= 8 && part_blocks <= (mode == 2 ? 16u : 32u)) {
+        p.waves = 16;
+    } else {
+        p.waves = 8;
+        if (part_blocks > (batch <= 8 ? 24u : 16u)) p.phases = (part_blocks + 15) / 16;
+    }
+    p.row_groups = cus / parts < tiles ? cus / parts : tiles;
+    const uint32_t phase_blocks = (part_blocks + p.phases - 1) / p.phases;
+    p.kb = (phase_blocks + p.waves - 1) / p.waves;
+    p.wave_k = (phase_blocks + p.kb - 1) / p.kb;
+    return p;
+}
+
+constexpr QmvPlan qmv_plan(uint32_t rows, uint32_t blocks, uint32_t batch, int mode, uint32_t cus, uint32_t meet_words) {
+    const uint32_t tiles = (rows + 15) / 16;
+    QmvPlan best{};
+    double best_cost = 0.0;
+    for (uint32_t parts = 1; parts <= 8 && parts <= blocks && parts <= cus; parts *= 2) {
+        if (parts > 1 &&
+            (mode == 2 || (uint64_t)tiles * (parts - 1) * ((batch + 1) / 2) * 16 > meet_words))
+            break;
+        const QmvPlan p = qmv_split(parts, tiles, blocks, batch, mode, cus);
+        const uint32_t part_blocks = (blocks + parts - 1) / parts;
+        const uint32_t per = (tiles + p.row_groups - 1) / p.row_groups;
+        // tile blocks the busiest workgroup streams, plus the cost of a
+        // meeting (a round trip of an atomic, as long as about ten tile
+        // blocks) and of rebuilding the fragments of every pass
+        const double cost =
+            (double)per * part_blocks + (parts > 1 ? 10.0 : 0.0) + (p.phases > 1 ? 8.0 * p.phases * per : 0.0);
+        if (best.k_parts == 0 || cost < best_cost) {
+            best = p;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+// First block of run u of `units` (a run is one wave's blocks in one phase of
+// one part; u = units: the end).  In 32 bits: the kernels work it out in their
+// loops, where a wider division, or a second one for the remainder, costs 3 to
+// 16% of a call.
+constexpr uint32_t run_begin(uint32_t u, uint32_t units, uint32_t blocks) { return u * blocks / units; }
+// Whether that product stays within 32 bits whatever split the plan takes.  A
+// wave holds at most 3 blocks, so every split has more than blocks / 3 runs, and
+// rows from 92682 blocks (23.7 million columns) on do not fit; shorter ones from
+// 65536 blocks on are looked at split by split.
+constexpr bool qmv_runs_fit(uint32_t blocks, uint32_t batch, int mode) {
+    for (uint32_t parts = 1; parts <= (mode == 2 ? 1u : 8u); parts *= 2) {
+        const QmvPlan p = qmv_split(parts, 1, blocks, batch, mode, parts);
+        if ((uint64_t)p.wave_k * p.k_parts * p.phases * blocks > 0xffffffffull) return false;
+    }
+    return true;
+}
+
 }  // namespace dm

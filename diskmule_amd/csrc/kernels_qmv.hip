@@ -587,8 +587,8 @@ __device__ __forceinline__ void qmv_body(const QmvArgs &p, uint32_t part, uint32
         }
         q.tile0 += pass_step;
     };
-    auto k_begin = [&](uint32_t phase) { return ((part * phases + phase) * wk + kw) * blocks / units; };
-    auto k_end = [&](uint32_t phase) { return ((part * phases + phase) * wk + kw + 1) * blocks / units; };
+    auto k_begin = [&](uint32_t phase) { return run_begin((part * phases + phase) * wk + kw, units, blocks); };
+    auto k_end = [&](uint32_t phase) { return run_begin((part * phases + phase) * wk + kw + 1, units, blocks); };
 
     // Chunk j * 64 + lane of a block of a tile: offset from the wave's first
     // block of the tile's first row (16 c is a multiple of the 4 bytes the
@@ -1016,6 +1016,10 @@ bool qmv_supported(uint32_t type, size_t rows, size_t columns, const void *w, si
     // Offsets are 32-bit: the matrix plus two rows of slack must fit.
     if (rows == 0 || row_bytes * (rows + 2) + 1024 >= 0xffffffffull) return false;
     if ((uint64_t)batch * columns * 4 >= 0xffffffffull) return false;
+    // (both forms: a gate/up pair asks through here too)
+    if (columns / 256 > 0xffff && !(qmv_runs_fit((uint32_t)(columns / 256), (uint32_t)batch, 0) &&
+                                    qmv_runs_fit((uint32_t)(columns / 256), (uint32_t)batch, 2)))
+        return false;
     const uintptr_t a = (uintptr_t)w;
     if (type == kQ4_K ? (a & 15u) : (a & 3u)) return false;
     return true;
@@ -1023,56 +1027,8 @@ bool qmv_supported(uint32_t type, size_t rows, size_t columns, const void *w, si
 
 namespace {
 
-struct Plan {
-    uint32_t kb, waves, wave_k, k_parts, row_groups, phases;
-};
-
-// The K split.  A workgroup of 16 waves of up to 128 registers holds the
-// fragments of 8 tokens of up to 32 blocks (2 per wave; a gate/up pair, which
-// needs more registers besides, 16), one of 8 waves of 256 those of 16
-// tokens of 16 blocks, or of 8 tokens of a pair's 24.  Longer rows, and
-// matrices with fewer tiles than CUs, are split over k_parts workgroups;
-// gate/up pairs, whose epilogue needs whole sums, go through longer rows in
-// phases instead.  The split minimises the largest workgroup's share of the
-// weights; within it, the most waves share K.
-Plan choose_plan(uint32_t rows, uint32_t blocks, uint32_t batch, int mode, uint32_t cus) {
-    const uint32_t tiles = (rows + 15) / 16;
-    Plan best{};
-    double best_cost = 0.0;
-    for (uint32_t parts = 1; parts <= 8 && parts <= blocks && parts <= cus; parts *= 2) {
-        if (parts > 1 &&
-            (mode == 2 || (uint64_t)tiles * (parts - 1) * ((batch + 1) / 2) * 16 > kQmvMeetWords))
-            break;
-        Plan p;
-        p.k_parts = parts;
-        const uint32_t part_blocks = (blocks + parts - 1) / parts;
-        p.phases = 1;
-        if (batch <= 8 && part_blocks <= (mode == 2 ? 16u : 32u)) {
-            p.waves = 16;
-        } else {
-            p.waves = 8;
-            if (part_blocks > (batch <= 8 ? 24u : 16u)) p.phases = (part_blocks + 15) / 16;
-        }
-        p.row_groups = cus / parts < tiles ? cus / parts : tiles;
-        const uint32_t phase_blocks = (part_blocks + p.phases - 1) / p.phases;
-        p.kb = (phase_blocks + p.waves - 1) / p.waves;
-        p.wave_k = (phase_blocks + p.kb - 1) / p.kb;
-        const uint32_t per = (tiles + p.row_groups - 1) / p.row_groups;
-        // tile blocks the busiest workgroup streams, plus the cost of a
-        // meeting (a round trip of an atomic, as long as about ten tile
-        // blocks) and of rebuilding the fragments of every pass
-        const double cost =
-            (double)per * part_blocks + (parts > 1 ? 10.0 : 0.0) + (p.phases > 1 ? 8.0 * p.phases * per : 0.0);
-        if (best.k_parts == 0 || cost < best_cost) {
-            best = p;
-            best_cost = cost;
-        }
-    }
-    return best;
-}
-
 template <uint32_t TYPE, int NT, int MODE, int KB, uint32_t W, bool PHASED = false>
-hipError_t run(dmhip_ctx *ctx, const Plan &p, QmvArgs &a) {
+hipError_t run(dmhip_ctx *ctx, const QmvPlan &p, QmvArgs &a) {
     // no more wave groups than a workgroup has tiles
     const uint32_t tiles = (a.rows + 15) / 16, per = (tiles + p.row_groups - 1) / p.row_groups;
     const uint32_t groups = W / p.wave_k, waves = (groups < per ? groups : per) * p.wave_k;
@@ -1089,7 +1045,7 @@ hipError_t dispatch(dmhip_ctx *ctx, uint32_t rows, uint32_t columns, const void 
                     const float *x, int normalize, float epsilon, float *y) {
     const uint32_t blocks = columns / 256;
     const uint32_t cus = ctx->compute_units > 0 ? (uint32_t)ctx->compute_units : 256u;
-    const Plan p = choose_plan(rows, blocks, batch, MODE, cus);
+    const QmvPlan p = qmv_plan(rows, blocks, batch, MODE, cus, kQmvMeetWords);
     QmvArgs a{(const uint8_t *)w, (const uint8_t *)w2, x, y, ctx->qmv_meet, rows, columns,
               blocks * StageQ<TYPE>::bytes, batch, p.wave_k, p.k_parts, p.row_groups, p.phases, normalize, epsilon};
     if (p.phases > 1)

@@ -14,6 +14,22 @@ SHIM = r"""
 extern "C" {
 uint32_t experts_grid(uint32_t cus, uint32_t pairs) { return dm::experts_grid(cus, pairs); }
 uint32_t experts_share(uint32_t grid, uint32_t entries) { return dm::experts_share(grid, entries); }
+void qmv_plan(uint32_t rows, uint32_t blocks, uint32_t batch, int mode, uint32_t cus, uint32_t *out) {
+    const dm::QmvPlan p = dm::qmv_plan(rows, blocks, batch, mode, cus, 512 * 1024);
+    const uint32_t v[6] = {p.kb, p.waves, p.wave_k, p.k_parts, p.row_groups, p.phases};
+    for (int i = 0; i < 6; i++) out[i] = v[i];
+}
+int qmv_runs_fit(uint32_t blocks, uint32_t batch, int mode) { return dm::qmv_runs_fit(blocks, batch, mode); }
+// Whether the runs are consecutive, cover all blocks and hold at most `most` each.
+int runs_cover(uint32_t units, uint32_t blocks, uint32_t most) {
+    uint64_t at = 0;
+    for (uint32_t u = 0; u < units; u++) {
+        const uint64_t lo = dm::run_begin(u, units, blocks), hi = dm::run_begin(u + 1, units, blocks);
+        if (lo != at || hi < lo || hi - lo > most) return 0;
+        at = hi;
+    }
+    return at == blocks;
+}
 }
 """
 
@@ -44,3 +60,38 @@ def test_every_grouped_expert_entry_has_workgroups(plan):
                 share = plan.experts_share(grid, entries)
                 assert share >= 1 and (entries - 1) * share + share - 1 < grid, (cus, pairs, entries)
     assert all(plan.experts_grid(256, pairs) == 512 for pairs in range(1, 129))
+
+
+BLOCKS = [*range(1, 70), 95, 96, 97, 112, 127, 128, 129, 208, 256, 257, 512, 1000, 4096, 65535, 65536, 92681, 92682,
+          131072, 1000003, (1 << 24) - 1]
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+def test_fp16_matvec_plans_give_every_block_to_a_wave(plan, mode):
+    """Every plan of the fp16 matvec: it is one of the compiled forms, and the
+    runs of its waves, parts and phases are consecutive, cover all blocks of
+    K and are no longer than the blocks a wave holds fragments for; the rows
+    of so many blocks that a run's start passes 32 bits are not taken."""
+    assert all(plan.qmv_runs_fit(blocks, batch, mode) for batch in (1, 16) for blocks in range(1, 65536, 7))
+    assert not any(plan.qmv_runs_fit(blocks, batch, mode) for batch in (1, 16) for blocks in range(92682, 1 << 24, 9973))
+    out = (ctypes.c_uint32 * 6)()
+    for cus in (32, 256):
+        for rows in (1, 16, 17, 300, 4096, 20000, 151936):
+            for batch in (1, 2, 8, 9, 16):
+                for blocks in BLOCKS:
+                    plan.qmv_plan(rows, blocks, batch, mode, cus, out)
+                    kb, waves, wave_k, parts, row_groups, phases = out
+                    case = (cus, rows, batch, blocks, list(out))
+                    assert 1 <= wave_k <= waves and parts * row_groups <= cus and (parts == 1 or mode == 0), case
+                    tiles = -(-rows // 16)
+                    assert parts == 1 or tiles * (parts - 1) * ((batch + 1) // 2) * 16 <= 512 * 1024, case
+                    if phases > 1 or batch > 8:
+                        assert waves == 8 and 1 <= kb <= 2, case
+                    elif waves == 8:
+                        assert mode == 2 and kb == 3, case
+                    else:
+                        assert waves == 16 and 1 <= kb <= (2 if mode == 0 else 1), case
+                    if plan.qmv_runs_fit(blocks, batch, mode):
+                        assert plan.runs_cover(wave_k * parts * phases, blocks, kb), case
+                    else:
+                        assert blocks > 0xffff, case
