@@ -89,4 +89,23 @@ constexpr bool qmv_runs_fit(uint32_t blocks, uint32_t batch, int mode) {
     return true;
 }
 
+// ---- the prefill GEMM (kernels_gemm.hip) ----
+constexpr uint32_t kGemmRows = 128;   // tile height, to which the workspace rows are padded
+constexpr uint32_t kGemmWaves = 4;    // waves of a workgroup, each with a quarter of K
+constexpr uint64_t gemm_padded_rows(uint64_t m) { return (m + kGemmRows - 1) / kGemmRows * kGemmRows; }
+// LDS of the A preparation: 8 rows of the largest quarter's columns as bf16.
+constexpr uint64_t gemm_prep_lds(uint64_t k) {
+    const uint64_t blocks = k / 256, quarter = (blocks + kGemmWaves - 1) / kGemmWaves;
+    return 8 * (quarter * 128 + 4) * 4;
+}
+// Whether the MFMA path takes a product of m x k activations with n encoded
+// rows of w_bytes in all: more than 16 tokens (fewer stream W faster through
+// the decode matvec), whole 256-column blocks, offsets that fit the 31-bit
+// buffer range, and a quarter of K that the preparation can stage in the 160
+// KiB of LDS (up to 39936 columns; longer rows go to the decode matvec, 16 tokens at a time).
+constexpr bool gemm_fits_mfma(uint64_t m, uint64_t n, uint64_t k, uint64_t w_bytes) {
+    return m > 16 && k % 256 == 0 && gemm_prep_lds(k) <= 160 * 1024 && w_bytes + 1024 < 0x7fffffffull &&
+           gemm_padded_rows(m) * k * 2 < 0x7fffffffull && m * n * 4 < 0x7fffffffull;
+}
+
 }  // namespace dm

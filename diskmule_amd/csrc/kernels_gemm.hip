@@ -56,6 +56,7 @@
 // both, measured within 2% of this form; 8 waves with an eighth of K each,
 // 10-20% slower (a longer final sum with nothing beside it).
 #include "dm_device.h"
+#include "dm_plan.h"
 #include "dm_qmv.h"
 #include "runtime.h"
 
@@ -65,8 +66,7 @@ namespace {
 
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));  // 16-byte aligned
 
-constexpr uint32_t kBM = 128, kBN = 64, kWaves = 4;
-constexpr uint32_t kPadRows = 128;  // workspace rows are padded to the tile height
+constexpr uint32_t kBM = kGemmRows, kBN = 64, kWaves = kGemmWaves;
 // MFMA steps between the load of an A fragment and its use.
 constexpr uint32_t kADist = 2;
 static_assert(16 % kADist == 0, "the A ring repeats every block");
@@ -600,11 +600,9 @@ __global__ void bf16_to_f32_kernel(const uint16_t *__restrict__ a, size_t count,
 
 namespace {
 
-size_t padded_rows(size_t m) { return (m + kPadRows - 1) / kPadRows * kPadRows; }
-
 // Workspace of the MFMA path: a16 | rowscale (4 quarters).
 size_t mfma_workspace(size_t m, size_t k) {
-    const size_t mp = padded_rows(m);
+    const size_t mp = gemm_padded_rows(m);
     return mp * k * 2 + 4 * mp * 4 + 2 * 256;
 }
 
@@ -626,14 +624,11 @@ int launch_gemm(dmhip_ctx *ctx, size_t mp, size_t m, size_t n, size_t k, const h
 template <class F>
 int run_gemm(dmhip_ctx *ctx, size_t m, size_t n, size_t k, const uint16_t *a_bf16, const void *weights,
              uint64_t w_bytes, float *c, void *workspace) {
-    const size_t mp = padded_rows(m);
+    const size_t mp = gemm_padded_rows(m);
     char *ws = (char *)(((uintptr_t)workspace + 255) & ~(uintptr_t)255);
     half8 *a16 = (half8 *)ws;
     float *rowscale = (float *)(ws + ((mp * k * 2 + 255) & ~(size_t)255));
-    const uint32_t blocks = (uint32_t)(k / 256);
-    // the largest quarter's columns staged per row (bf16 pairs), 8 rows
-    const uint32_t qmax = (blocks + kWaves - 1) / kWaves;
-    const uint32_t prep_lds = 8 * (qmax * 128 + 4) * 4;
+    const uint32_t prep_lds = (uint32_t)gemm_prep_lds(k);
     static LdsLimit prep_limit;
     DM_HIP(prep_limit.ensure((const void *)gemm_prep_kernel<F>, prep_lds));
     hipLaunchKernelGGL(gemm_prep_kernel<F>, dim3((uint32_t)(mp / 8), kWaves), dim3(256), prep_lds, ctx->stream,
@@ -677,14 +672,9 @@ int dmhip_gemm_device(dmhip_ctx *ctx, uint32_t type, size_t m, size_t n, size_t 
         return fail(DMHIP_ERR_VECTOR_TOO_LARGE, "HIP vector length exceeds the 32-bit kernel limit");
     DM_CHECK_STATUS(set_device(ctx));
 
-    // The MFMA path: more than 16 tokens (fewer stream W faster through the
-    // decode GEMV), whole 256-column blocks, offsets that fit the 31-bit
-    // buffer range, 16-byte aligned operands.
+    // The MFMA path, for 16-byte aligned operands (and see gemm_fits_mfma).
     const uint64_t w_bytes = rb * n;
-    const size_t mp = padded_rows(m);
-    const bool mfma = m > 16 && k % 256 == 0 && (type == kQ4_K || type == kQ6_K || type == kQ8_0) &&
-                      w_bytes + 1024 < 0x7fffffffull && (uint64_t)mp * k * 2 < 0x7fffffffull &&
-                      (uint64_t)m * n * 4 < 0x7fffffffull &&
+    const bool mfma = (type == kQ4_K || type == kQ6_K || type == kQ8_0) && gemm_fits_mfma(m, n, k, w_bytes) &&
                       ((uintptr_t)weights & 15u) == 0 && ((uintptr_t)a_bf16 & 15u) == 0 && ((uintptr_t)c & 15u) == 0;
     if (mfma) {
         if (type == kQ4_K) return run_gemm<FormatQ4K>(ctx, m, n, k, a_bf16, weights, w_bytes, c, workspace);

@@ -1593,6 +1593,24 @@ def test_prefill_gemm_tile_edges(ctx, kind, m, n, k):
     assert_channel_close(got, exact, scale, CHANNEL_TOL_GEMM, f"type {kind}")
 
 
+@pytest.mark.parametrize("kind", [Q4_K, Q6_K, Q8_0])
+@pytest.mark.parametrize("k", [39936, 40192])
+def test_prefill_gemm_longest_rows(ctx, kind, k):
+    """The longest rows whose quarter the A preparation can stage in LDS, and
+    the first past them, which go to the decode matvec: the per-channel bound of the
+    prefill products."""
+    m, n = 18, 5
+    print(f"longest rows: type {kind} m={m} n={n} k={k}", flush=True)
+    a = synth.to_bf16_bits(synth.normal(synth.activation_seed(9, kind), m * k))
+    w = synth.quantized_matrix(kind, n, k, synth.weight_seed(9, kind))
+    ab, wb, cb = dev(ctx, a), dev(ctx, w), dev_out(ctx, m * n * 4)
+    ws = dev_out(ctx, ctx.gemm_workspace_bytes(m, k))
+    ctx.gemm_device(kind, m, n, k, ab.device_ptr, wb.device_ptr, cb.device_ptr, ws.device_ptr, len(ws))
+    got = cb.read(0, m * n * 4, np.float32).reshape(m, n)
+    exact, scale = exact_products(kind, n, k, w, synth.bf16_bits_to_f32(a).reshape(m, k))
+    assert_channel_close(got, exact, scale, CHANNEL_TOL_GEMM, f"type {kind} k {k}")
+
+
 def test_objects_outliving_their_context_exit_cleanly():
     """Regression: device buffers and caches freed after their context was
     closed (the order Python's collector may pick at exit)."""

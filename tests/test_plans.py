@@ -19,6 +19,8 @@ void qmv_plan(uint32_t rows, uint32_t blocks, uint32_t batch, int mode, uint32_t
     const uint32_t v[6] = {p.kb, p.waves, p.wave_k, p.k_parts, p.row_groups, p.phases};
     for (int i = 0; i < 6; i++) out[i] = v[i];
 }
+uint64_t gemm_prep_lds(uint64_t k) { return dm::gemm_prep_lds(k); }
+int gemm_fits_mfma(uint64_t m, uint64_t n, uint64_t k, uint64_t w_bytes) { return dm::gemm_fits_mfma(m, n, k, w_bytes); }
 int qmv_runs_fit(uint32_t blocks, uint32_t batch, int mode) { return dm::qmv_runs_fit(blocks, batch, mode); }
 // Whether the runs are consecutive, cover all blocks and hold at most `most` each.
 int runs_cover(uint32_t units, uint32_t blocks, uint32_t most) {
@@ -44,6 +46,9 @@ def plan(tmp_path_factory):
     lib = ctypes.CDLL(str(d / "shim.so"))
     for name in ("experts_grid", "experts_share"):
         getattr(lib, name).restype = ctypes.c_uint32
+    lib.gemm_prep_lds.restype = ctypes.c_uint64
+    lib.gemm_prep_lds.argtypes = [ctypes.c_uint64]
+    lib.gemm_fits_mfma.argtypes = [ctypes.c_uint64] * 4
     return lib
 
 
@@ -95,3 +100,11 @@ def test_fp16_matvec_plans_give_every_block_to_a_wave(plan, mode):
                         assert plan.runs_cover(wave_k * parts * phases, blocks, kb), case
                     else:
                         assert blocks > 0xffff, case
+
+
+def test_prefill_gemm_stages_a_quarter_of_k_in_lds(plan):
+    """The preparation's LDS never passes a workgroup's 160 KiB on a shape that
+    the MFMA path takes; 39936 columns are its last."""
+    for k in range(256, 200000, 256):
+        taken = plan.gemm_fits_mfma(17, 64, k, 64 * (k // 256) * 210)
+        assert bool(taken) == (k <= 39936) and (not taken or plan.gemm_prep_lds(k) <= 160 * 1024), k
