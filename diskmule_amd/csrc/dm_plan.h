@@ -102,10 +102,14 @@ constexpr uint64_t gemm_prep_lds(uint64_t k) {
 // rows of w_bytes in all: more than 16 tokens (fewer stream W faster through
 // the decode matvec), whole 256-column blocks, offsets that fit the 31-bit
 // buffer range, and a quarter of K that the preparation can stage in the 160
-// KiB of LDS (up to 39936 columns; longer rows go to the decode matvec, 16 tokens at a time).
+// KiB of LDS (up to 39936 columns; longer rows go to the decode matvec, 16
+// tokens at a time).  The stores of the rows past m in the last tile rely on
+// their offsets lying past the end of C, so those offsets may not wrap at 32
+// bits: at 17 rows (padded to 128) n stops at 8388608.
 constexpr bool gemm_fits_mfma(uint64_t m, uint64_t n, uint64_t k, uint64_t w_bytes) {
     return m > 16 && k % 256 == 0 && gemm_prep_lds(k) <= 160 * 1024 && w_bytes + 1024 < 0x7fffffffull &&
-           gemm_padded_rows(m) * k * 2 < 0x7fffffffull && m * n * 4 < 0x7fffffffull;
+           gemm_padded_rows(m) * k * 2 < 0x7fffffffull && m * n * 4 < 0x7fffffffull &&
+           gemm_padded_rows(m) * n * 4 <= 0x100000000ull;
 }
 
 }  // namespace dm

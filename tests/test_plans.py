@@ -108,3 +108,16 @@ def test_prefill_gemm_stages_a_quarter_of_k_in_lds(plan):
     for k in range(256, 200000, 256):
         taken = plan.gemm_fits_mfma(17, 64, k, 64 * (k // 256) * 210)
         assert bool(taken) == (k <= 39936) and (not taken or plan.gemm_prep_lds(k) <= 160 * 1024), k
+
+
+def test_prefill_gemm_stores_of_padding_rows_stay_past_the_end(plan):
+    """No store of a row past m reaches C: the 32-bit offset of every padding
+    row's columns is past C's end, also at the most columns that fit."""
+    for m in (17, 40, 127, 129, 200, 1000, 2049):
+        padded = -(-m // 128) * 128
+        edge = (1 << 32) // (4 * padded)  # the last n whose padded rows end within 2^32 bytes
+        for n in sorted({64, 5000, edge - 1, edge, edge + 1, 2 * edge, ((1 << 31) - 4) // (4 * m)}):
+            if not plan.gemm_fits_mfma(m, n, 256, 144 * n):
+                assert n > edge or 144 * n + 1024 >= 0x7fffffff or m * n * 4 >= 0x7fffffff, (m, n)
+                continue
+            assert ((padded - 1) * n + n - 1) * 4 < 1 << 32, (m, n)  # (they start at m * n * 4, C's end)
