@@ -952,22 +952,17 @@ __global__ void __launch_bounds__(64 * (S > 8 ? S : 8))
                         const uint32_t *__restrict__ go, uint32_t go_count, Combine8 cb) {
     // Jobs whose matrices a kernel earlier on the stream looked up: their
     // addresses come from dev_w, and the launch does nothing unless each of
-    // the go_count (up to 64) tokens' go words is 1.  The address and every
-    // go word are asked for before the first is looked at: one round trip to
-    // memory before the weights.  Whole calls of a resident layer, in us, the
-    // words one after another and then the address / the words at once and
-    // then the address / this form: 2048 x 768, 128 experts top 8, 1 token
-    // 40.1 / 40.9 / 39.9, 4 tokens 63.1 / 64.3 / 61.6; top 4, 8 tokens
-    // 64.1 / 65.0 / 63.2.
-    uint64_t looked_up = 0;
-    if (dev_w) {
-        const uint32_t t = min(threadIdx.x & 63u, go_count - 1);
-        looked_up = __hip_atomic_load(&dev_w[blockIdx.y], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t set = __hip_atomic_load(&go[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (__builtin_amdgcn_ballot_w64(set == 0)) return;
-    }
+    // the go_count tokens' go words is 1.  (Uniform reads through the scalar
+    // cache.  One vector load for all words made every resident call 0.7 to
+    // 1 us longer: 2048 x 768, 128 experts top 8, 1 token 40.1 -> 40.9 us.
+    // The address asked for together with the words, also by vector loads,
+    // gained 1 to 2 us at 4 to 8 tokens but changed the registers of the rest:
+    // one token of 6144 x 2048, 16 experts top 8, 71.1 -> 75.0 us.)
+    if (go)
+        for (uint32_t t = 0; t < go_count; t++)
+            if (go[t] == 0) return;
     const Job8 j = jobs.job[blockIdx.y];
-    const uint8_t *w = (const uint8_t *)(dev_w ? looked_up : (uint64_t)j.w);
+    const uint8_t *w = (const uint8_t *)(dev_w ? dev_w[blockIdx.y] : j.w);
     constexpr uint32_t WAVES = S > 8 ? S : 8;
     qmv8_body<TYPE, S, MODE, TOK, G, WAVES, false, PUB>(w, w + w2_offset, rows, columns, row_bytes, total_bytes,
                                                         x + j.x_off, j.x_stride, 0, 0.0f, glm, y + j.y_off,
@@ -1339,7 +1334,6 @@ hipError_t launch_qmv8_grouped(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uin
                                const uint64_t *dev_w, const uint32_t *go, const QmvCombine *combine,
                                uint32_t go_count) {
     const uint32_t mats = gate_up ? 2u : 1u;
-    if (dev_w && (!go || go_count < 1 || go_count > 64)) return hipErrorInvalidValue;
     // device-side addresses (and the fused combine): one launch of one-token
     // jobs, in order
     if (dev_w || combine) {
