@@ -17,6 +17,33 @@ constexpr uint32_t experts_grid(uint32_t cus, uint32_t pairs) { return 2 * cus >
 // Workgroups per entry; workgroup b works on entry b / share, if there is one.
 constexpr uint32_t experts_share(uint32_t grid, uint32_t entries) { return grid > entries ? grid / entries : 1u; }
 
+// Whether a resident layer call's tokens are grouped by expert on the device
+// (each selected expert streamed once for all its tokens by the fp16 kernel)
+// rather than run as one int8 job per pair of token and selection.
+//  * One token shares nothing: never.
+//  * More than 8 tokens or max_jobs pairs: always (else the host forms the
+//    launches after a round trip: 10 tokens of 1024 x 512, 60 experts top 2,
+//    47 against 61 us).
+//  * Otherwise where the pairs' experts come to 140 MB and grouping is expected
+//    to save 20 MB of them (selections spread evenly over the experts).  In us,
+//    per pair / grouped, with the MB saved:
+//      4096 x 1536, 32 experts top 4: 2 tokens 51 / 63 (6), 3 65 / 69 (18),
+//      4 75 / 75 (34), 5 90 / 78 (54);
+//      4096 x 1536, 64 experts top 2: 7 tokens 69 / 74 (15), 8 78 / 77 (21);
+//      2048 x 768, 128 experts top 8: 4 tokens 63 / 64 (9), 6 78 / 73 (21);
+//      4096 x 1024, 64 experts top 8: 2 tokens 61 / 67 (8), 3 80 / 76 (24);
+//      6144 x 2048, 16 experts top 8: 1 token 71 / 84 (0), 2 107 / 105 (98),
+//      3 143 / 115; 1024 x 512, 32 experts top 8 (65 MB in all): 8 47 / 48 (35).
+constexpr bool moe_groups_by_expert(uint64_t batch, uint64_t k, uint64_t experts, uint64_t expert_bytes, uint64_t max_jobs) {
+    if (batch < 2) return false;
+    const uint64_t pairs = batch * k;
+    if (batch > 8 || pairs > max_jobs) return true;
+    double none = 1.0;  // chance that no token selects a given expert
+    for (uint64_t t = 0; t < batch; t++) none *= 1.0 - (double)k / (double)experts;
+    const double shared = (double)pairs - (double)experts * (1.0 - none);
+    return (double)pairs * (double)expert_bytes >= 140.0 * (1 << 20) && shared * (double)expert_bytes >= 20e6;
+}
+
 // ---- the fp16 matvec (kernels_qmv.hip) ----
 struct QmvPlan {
     uint32_t kb, waves, wave_k, k_parts, row_groups, phases;

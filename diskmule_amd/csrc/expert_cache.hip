@@ -29,6 +29,7 @@
 #include <thread>
 #include <vector>
 
+#include "dm_plan.h"
 #include "dm_qmv.h"
 
 namespace dm {
@@ -196,14 +197,6 @@ namespace {
 constexpr size_t kSelectionPairs = 16 * dm::kMaxTopK;  // batch <= 16
 constexpr size_t kSelectionBytes = kSelectionPairs * 8 + 16 * 4 + 16 * 4;  // ids, probabilities, per-token flags, go
 constexpr size_t kReleaseEvents = 64;
-// Layer calls whose selected experts' bytes, counted per pair, reach this
-// group the tokens by expert on the device (launch_qmv_experts).  Measured on
-// MI355X, one job per pair against grouped: 2048 x 768, 128 experts top 8
-// (24.5 MB a token) 2 / 4 / 6 / 8 tokens 46 / 62 / 77 / 87 against
-// 52 / 63 / 75 / 83 us; 4096 x 1536, 32 experts top 4 (49 MB a token) 2 / 4 / 8
-// tokens 52 / 77 / 109 against 61 / 77 / 98 us; 1024 x 512, 60 experts top 2 8
-// tokens (12 MB in all) 37 against 46 us.
-constexpr size_t kExpertGroupBytes = 140u << 20;
 constexpr size_t kCombineTickets = 4096;  // row-tile workgroups of a fused down + combine launch
 constexpr size_t kStagingEntries = 4;  // file source: experts in flight from storage
 // Memory source: uploads whose timing is kept until it is read.  The ring is
@@ -765,19 +758,16 @@ int dmhip_moe_layer(dmhip_ctx *ctx, dmhip_expert_cache *c, size_t layer, size_t 
     // Up to kMaxLookupTokens tokens whose experts are likely resident: each
     // token's last router workgroup looks its selected experts up in the
     // layer's residency table, and the expert launches (one job per token
-    // and selection) and the combine are queued right behind the router,
-    // reading the slot addresses it found; when a slot is missing (or a
-    // token's logits are not finite) they do nothing and the host takes the
-    // path below with the selection in hand.  Every earlier upload is
+    // and selection, or per expert) and the combine are queued right behind
+    // the router, reading the slot addresses it found; when a slot is missing
+    // (or a token's logits are not finite) they do nothing and the host takes
+    // the path below with the selection in hand.  Every earlier upload is
     // already waited for on the compute stream, before the table copy and
     // the router.
-    // Grouping streams each expert once for all its tokens; its launches cost
-    // about 8 us more than those of one job per pair, whose bytes grow with
-    // the pairs.
-    const bool by_expert = (batch > 8 || pairs > kMaxGroupedJobs ||
-                            pairs * (L.gate_up_bytes + L.down_bytes) >= kExpertGroupBytes) &&
-                           qmv_experts_supported(gate_up_type, width, hidden, experts, pairs, batch) &&
-                           qmv_experts_supported(down_type, hidden, width, experts, pairs, pairs);
+    const bool by_expert =
+        moe_groups_by_expert(batch, k, experts, L.gate_up_bytes + L.down_bytes, kMaxGroupedJobs) &&
+        qmv_experts_supported(gate_up_type, width, hidden, experts, pairs, batch) &&
+        qmv_experts_supported(down_type, hidden, width, experts, pairs, pairs);
     const bool lookup = Lay.try_lookup && grouped && (by_expert || (batch <= 8 && pairs <= kMaxGroupedJobs)) &&
                         router_takes_lookup((uint32_t)hidden, (uint32_t)experts, (uint32_t)batch, router_bf16, x);
     if (lookup) {
@@ -805,27 +795,27 @@ int dmhip_moe_layer(dmhip_ctx *ctx, dmhip_expert_cache *c, size_t layer, size_t 
                                c->lookup_go);
             DM_HIP(hipGetLastError());
         } else {
-        // job p: selection p % k of token p / k
-        std::vector<QmvJob> gu_jobs(pairs), dn_jobs(pairs);
-        for (size_t p = 0; p < pairs; p++) {
-            gu_jobs[p] = QmvJob{nullptr, 1u, (uint32_t)(p / k * hidden), (uint32_t)(p * width), 0, 0};
-            dn_jobs[p] = QmvJob{nullptr, 1u, (uint32_t)(p * width), (uint32_t)(p * hidden), 0, 0};
-        }
-        DM_HIP(launch_qmv8_grouped(ctx, gate_up_type, (uint32_t)width, (uint32_t)hidden, 1, up_offset,
-                                   gu_jobs.data(), pairs, x, d_act, c->lookup_gate_up, c->lookup_go, nullptr, tokens));
-        // the down launch also makes the ordered combine when its split
-        // allows (every workgroup holds whole row tiles of every expert)
-        const QmvCombine cmb{c->combine_tickets, kCombineTickets, d_probs, y, (uint32_t)k, (uint32_t)hidden};
-        if (launch_qmv8_grouped(ctx, down_type, (uint32_t)hidden, (uint32_t)width, 0, 0, dn_jobs.data(), pairs,
-                                d_act, d_eo, c->lookup_down, c->lookup_go, &cmb, tokens) != hipSuccess) {
-            (void)hipGetLastError();
-            DM_HIP(launch_qmv8_grouped(ctx, down_type, (uint32_t)hidden, (uint32_t)width, 0, 0, dn_jobs.data(), pairs,
-                                       d_act, d_eo, c->lookup_down, c->lookup_go, nullptr, tokens));
-            hipLaunchKernelGGL(moe_combine_pos_kernel, dim3((uint32_t)((batch * hidden + 255) / 256)), dim3(256), 0,
-                               ctx->stream, d_eo, nullptr, d_probs, tokens, (uint32_t)k, (uint32_t)hidden, y,
-                               c->lookup_go);
-            DM_HIP(hipGetLastError());
-        }
+            // job p: selection p % k of token p / k
+            std::vector<QmvJob> gu_jobs(pairs), dn_jobs(pairs);
+            for (size_t p = 0; p < pairs; p++) {
+                gu_jobs[p] = QmvJob{nullptr, 1u, (uint32_t)(p / k * hidden), (uint32_t)(p * width), 0, 0};
+                dn_jobs[p] = QmvJob{nullptr, 1u, (uint32_t)(p * width), (uint32_t)(p * hidden), 0, 0};
+            }
+            DM_HIP(launch_qmv8_grouped(ctx, gate_up_type, (uint32_t)width, (uint32_t)hidden, 1, up_offset,
+                                       gu_jobs.data(), pairs, x, d_act, c->lookup_gate_up, c->lookup_go, nullptr, tokens));
+            // the down launch also makes the ordered combine when its split
+            // allows (every workgroup holds whole row tiles of every expert)
+            const QmvCombine cmb{c->combine_tickets, kCombineTickets, d_probs, y, (uint32_t)k, (uint32_t)hidden};
+            if (launch_qmv8_grouped(ctx, down_type, (uint32_t)hidden, (uint32_t)width, 0, 0, dn_jobs.data(), pairs,
+                                    d_act, d_eo, c->lookup_down, c->lookup_go, &cmb, tokens) != hipSuccess) {
+                (void)hipGetLastError();
+                DM_HIP(launch_qmv8_grouped(ctx, down_type, (uint32_t)hidden, (uint32_t)width, 0, 0, dn_jobs.data(), pairs,
+                                           d_act, d_eo, c->lookup_down, c->lookup_go, nullptr, tokens));
+                hipLaunchKernelGGL(moe_combine_pos_kernel, dim3((uint32_t)((batch * hidden + 255) / 256)), dim3(256), 0,
+                                   ctx->stream, d_eo, nullptr, d_probs, tokens, (uint32_t)k, (uint32_t)hidden, y,
+                                   c->lookup_go);
+                DM_HIP(hipGetLastError());
+            }
         }
     } else {
         DM_HIP(launch_router_top_k(ctx->stream, router_bf16, (uint32_t)hidden, (uint32_t)experts,

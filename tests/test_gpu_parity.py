@@ -1333,6 +1333,37 @@ def test_moe_layer_groups_tokens_by_expert(ctx, hidden, width, experts, k, batch
     src.free()
 
 
+def test_moe_layer_one_token_of_large_experts(ctx):
+    """One token whose 8 experts come to 147 MB: its experts are shared with no
+    other token, so the resident calls (third and later: the layer looks
+    experts up again after a call that found all of them) run the same kernels
+    as the first, host-path ones, bit for bit."""
+    hidden, width, experts, k = 4096, 2304, 8, 8
+    router = synth.to_bf16_bits(synth.normal(synth.weight_seed(53, 0), experts * hidden) * np.float32(0.02))
+    gu_bytes, dn_bytes = 2 * width * synth.row_bytes(Q4_K, hidden), hidden * synth.row_bytes(Q6_K, width)
+    assert k * (gu_bytes + dn_bytes) > 140 << 20
+    gu = synth.quantized_matrix(Q4_K, experts * 2 * width, hidden, synth.weight_seed(53, 1))
+    dn = synth.quantized_matrix(Q6_K, experts * hidden, width, synth.weight_seed(53, 2))
+    src = PinnedHostBuffer(gu.size + dn.size)
+    src.array[:gu.size] = gu
+    src.array[gu.size:] = dn
+    cache = ExpertCache(ctx, src, [ExpertLayerLayout(experts, 0, gu_bytes, gu.size, dn_bytes)], experts)
+    x = synth.normal(synth.activation_seed(53, 0), hidden).reshape(1, hidden)
+    sel, wts, out = capi.moe_layer(1, hidden, width, experts, k, router, Q4_K, gu, Q6_K, dn, x)
+    rb, yb, xb = dev(ctx, router), dev_out(ctx, hidden * 4), dev(ctx, x)
+    runs = []
+    for call in range(5):
+        ids, probs = ctx.moe_layer(cache, 0, 1, hidden, width, experts, k, rb.device_ptr, Q4_K, Q6_K,
+                                   xb.device_ptr, yb.device_ptr)
+        assert np.array_equal(ids, sel) and np.allclose(probs, wts, rtol=1e-5, atol=1e-7)
+        runs.append(yb.read(0, hidden * 4, np.float32).copy())
+        assert_close(runs[-1], out[0], f"call {call}")
+        assert cache.stats()["misses"] == experts
+    assert all(np.array_equal(bits(r), bits(runs[0])) for r in runs[1:])
+    cache.free()
+    src.free()
+
+
 def test_moe_layer_lookup_wide_router(ctx):
     """Two tokens over a router wider than 8192 columns (the exact fold's
     expert-parallel kernel, which writes the device-side lookup itself):

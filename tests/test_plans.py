@@ -19,6 +19,9 @@ void qmv_plan(uint32_t rows, uint32_t blocks, uint32_t batch, int mode, uint32_t
     const uint32_t v[6] = {p.kb, p.waves, p.wave_k, p.k_parts, p.row_groups, p.phases};
     for (int i = 0; i < 6; i++) out[i] = v[i];
 }
+int moe_groups_by_expert(uint64_t batch, uint64_t k, uint64_t experts, uint64_t bytes) {
+    return dm::moe_groups_by_expert(batch, k, experts, bytes, 64);
+}
 uint64_t gemm_prep_lds(uint64_t k) { return dm::gemm_prep_lds(k); }
 int gemm_fits_mfma(uint64_t m, uint64_t n, uint64_t k, uint64_t w_bytes) { return dm::gemm_fits_mfma(m, n, k, w_bytes); }
 int qmv_runs_fit(uint32_t blocks, uint32_t batch, int mode) { return dm::qmv_runs_fit(blocks, batch, mode); }
@@ -48,6 +51,7 @@ def plan(tmp_path_factory):
         getattr(lib, name).restype = ctypes.c_uint32
     lib.gemm_prep_lds.restype = ctypes.c_uint64
     lib.gemm_prep_lds.argtypes = [ctypes.c_uint64]
+    lib.moe_groups_by_expert.argtypes = [ctypes.c_uint64] * 4
     lib.gemm_fits_mfma.argtypes = [ctypes.c_uint64] * 4
     return lib
 
@@ -65,6 +69,24 @@ def test_every_grouped_expert_entry_has_workgroups(plan):
                 share = plan.experts_share(grid, entries)
                 assert share >= 1 and (entries - 1) * share + share - 1 < grid, (cus, pairs, entries)
     assert all(plan.experts_grid(256, pairs) == 512 for pairs in range(1, 129))
+
+
+def test_tokens_are_grouped_by_expert_only_where_they_share(plan):
+    """One token, or tokens that can hardly share an expert, never; calls that
+    the one-job-per-pair launches do not take, always; between them only
+    where enough bytes are saved (the measured calls on either side)."""
+    mb = 1 << 20
+    for k, experts in ((1, 1), (8, 8), (8, 16), (8, 128), (64, 64), (100, 128)):
+        assert not plan.moe_groups_by_expert(1, k, experts, 1000 * mb)
+        assert plan.moe_groups_by_expert(9, k, experts, mb) and plan.moe_groups_by_expert(16, k, experts, mb)
+    assert plan.moe_groups_by_expert(2, 33, 128, mb)  # 66 pairs
+    size = {(2048, 768): 3059712, (4096, 1536): 12238848, (4096, 1024): 8159232, (6144, 2048): 24477696, (1024, 512): 1019904}
+    for shape, experts, k, batch, grouped in (
+            ((2048, 768), 128, 8, 4, False), ((2048, 768), 128, 8, 6, True), ((4096, 1536), 32, 4, 3, False),
+            ((4096, 1536), 32, 4, 5, True), ((4096, 1536), 64, 2, 7, False), ((4096, 1024), 64, 8, 2, False),
+            ((4096, 1024), 64, 8, 3, True), ((6144, 2048), 16, 8, 1, False), ((6144, 2048), 16, 8, 3, True),
+            ((1024, 512), 32, 8, 8, False)):
+        assert bool(plan.moe_groups_by_expert(batch, k, experts, size[shape])) == grouped, (shape, experts, k, batch)
 
 
 BLOCKS = [*range(1, 70), 95, 96, 97, 112, 127, 128, 129, 208, 256, 257, 512, 1000, 4096, 65535, 65536, 92681, 92682,
