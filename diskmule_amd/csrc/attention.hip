@@ -17,7 +17,8 @@
 // them in the reference's order (d ascending, one lane per position; the keys
 // reach the lanes through LDS so that every HBM read is a coalesced row
 // segment), attn_stream_kernel as 8-term chains added in a tree, whose error
-// is smaller.
+// is smaller; it goes back to the reference's order for rows whose partial sums
+// could pass the largest float, so both find the same scores non-finite.
 #include "dm_device.h"
 #include "runtime.h"
 
@@ -336,11 +337,12 @@ attn_chunk_kernel(const float *__restrict__ query, const float *__restrict__ key
 // where 8 rows and the heads' sums do not fit 256 registers): no staging and
 // no barrier until the end, 16 or 32 KiB of keys and values in flight per
 // wave.  Scores are 8-term fma chains per lane added in a fixed tree over the
-// lanes; the sums of R rows and of the heads are reduced together (each
-// exchange halves the values a lane keeps), which leaves one row and head with
-// each lane, so the softmax costs two exponentials per block of rows, not two
-// per head.  It is the online one (earlier sums rescaled when a larger maximum
-// arrives); the waves meet in LDS at the chunk's end.
+// lanes (in the reference's order where a partial sum could overflow); the
+// sums of R rows and of the heads are reduced together (each exchange halves
+// the values a lane keeps), which leaves one row and head with each lane, so
+// the softmax costs two exponentials per block of rows, not two per head.  It
+// is the online one (earlier sums rescaled when a larger maximum arrives); the
+// waves meet in LDS at the chunk's end.
 //
 // Large windows are bound by the reads of the keys and values: 16 query on 2
 // KV heads of 512 dims at 32768 positions, 52.8 us for 268 MB (5.1 TB/s); the
@@ -350,7 +352,10 @@ attn_chunk_kernel(const float *__restrict__ query, const float *__restrict__ key
 // 19.7 / 58.3; 16 on 8 x 256: 13.9 / 15.2 / 22.2 / 105.9 against 9.4 / 11.1 /
 // 18.7 / 92.6; 32 on 8 x 128: 14.7 / 15.5 / 22.4 / 85.3 against 9.8 / 11.1 /
 // 16.7 / 56.9; 8 on 8 x 128: 13.5 / 14.5 / 20.1 / 76.5 against 9.3 / 10.1 /
-// 14.2 / 55.0.  With the scores reduced over the lanes head by head and an
+// 14.2 / 55.0.  The watch for partial sums that could overflow (largest |query|
+// of the workgroup, largest |key| of each lane's rows) costs about 0.2 us of a
+// short call (16 on 8 x 256, 300 positions: 9.4 -> 9.6) and nothing at 32768
+// (16 on 2 x 512: 53.1 -> 52.4).  With the scores reduced over the lanes head by head and an
 // exponential per head in every lane: 60.3 and 54.5 in the kernel at 2 x 512.
 // ---------------------------------------------------------------------------
 template <int CTRL>
@@ -421,6 +426,7 @@ attn_stream_kernel(const float *__restrict__ query, const float *__restrict__ ke
     constexpr int RB = R == 8 ? 3 : 2, HB0 = GT == 8 ? 3 : GT == 4 ? 2 : GT == 2 ? 1 : 0;
     constexpr int HB = HB0 < TOP + 1 - RB ? HB0 : TOP + 1 - RB, NV = GT >> HB, LOW = TOP + 1 - RB - HB;
     extern __shared__ __attribute__((aligned(16))) float lds[];
+    __shared__ float s_q[kStreamWaves];  // largest |query| of each wave's share
     const uint32_t t = threadIdx.x, lane = t & 63u, waves = blockDim.x >> 6;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const uint32_t l = lane % LPR, lg = lane / LPR;              // lane in its group, group
@@ -459,6 +465,7 @@ attn_stream_kernel(const float *__restrict__ query, const float *__restrict__ ke
     const uint32_t units = gz * (HD / 4);
     const floatx4 *q4 = (const floatx4 *)(query + qbase * HD);
     floatx4 qv[4];
+    float q_max = 0.0f;
     auto ask = [&](uint32_t i0) {
 #pragma unroll
         for (uint32_t k = 0; k < 4; k++) qv[k] = q4[min(i0 + k * blockDim.x, units - 1)];
@@ -468,6 +475,8 @@ attn_stream_kernel(const float *__restrict__ query, const float *__restrict__ ke
         for (uint32_t k = 0; k < 4; k++) {
             const uint32_t i = i0 + k * blockDim.x;
             if (i < GT * HD / 4) ((floatx4 *)qs)[i] = qv[k];  // (heads past the last: scored, then dropped)
+#pragma unroll
+            for (int e = 0; e < 4; e++) q_max = fmaxf(q_max, fabsf(qv[k][e]));
         }
     };
     ask(t);
@@ -480,9 +489,20 @@ attn_stream_kernel(const float *__restrict__ query, const float *__restrict__ ke
         ask(i);
         put(i);
     }
+    const auto big = [](float a, float b) { return fmaxf(a, b); };
+    q_max = attn_across<3>(attn_across<4>(attn_across<5>(q_max, big), big), big);
+    q_max = attn_across<0>(attn_across<1>(attn_across<2>(q_max, big), big), big);
+    if (lane == 0) s_q[wave] = q_max;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+
+    // Products of at most 2^127 / HD leave every partial sum of a score, in
+    // any order, at 2^127 or less.
+    constexpr float kProductLimit = 0x1p127f / HD;
+    q_max = 0.0f;
+#pragma unroll
+    for (uint32_t k = 0; k < kStreamWaves; k++) q_max = fmaxf(q_max, s_q[k < waves ? k : 0]);
 
     float o[GT][8], m[NV], ls[NV];
 #pragma unroll
@@ -493,10 +513,17 @@ attn_stream_kernel(const float *__restrict__ query, const float *__restrict__ ke
     for (int i = 0; i < NV; i++) m[i] = -INFINITY, ls[i] = 0.0f;
     bool flag = false;
     const auto add = [](float a, float b) { return a + b; };
-    const auto big = [](float a, float b) { return fmaxf(a, b); };
     for (; j0 < n; j0 += step) {
         const bool mine = j0 + R * lg + my_row < n;
         float s[GT];
+        float key_max = 0.0f;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            float mx = 0.0f;
+#pragma unroll
+            for (int d = 0; d < 8; d++) mx = fmaxf(mx, fabsf(kr[r][d / 4][d % 4]));
+            key_max = fmaxf(key_max, mx);
+        }
 #pragma unroll
         for (int h = 0; h < GT; h++) {
             const floatx4 q0 = *(const floatx4 *)&qs[h * HD + 4 * l], q1 = *(const floatx4 *)&qs[h * HD + HD / 2 + 4 * l];
@@ -542,6 +569,31 @@ attn_stream_kernel(const float *__restrict__ query, const float *__restrict__ ke
             if constexpr (LOW >= 3) v = attn_across<2>(v, add);
             if constexpr (LOW >= 2) v = attn_across<1>(v, add);
             if constexpr (LOW >= 1) v = attn_across<0>(v, add);
+            s[i] = v;
+        }
+        if (__builtin_amdgcn_ballot_w64(key_max * q_max > kProductLimit)) {
+            // A partial sum of some score may pass the largest float in one
+            // order and not in another: these rows' scores are taken in the
+            // reference's order, so that the same ones are non-finite.
+            uint64_t slot = slot0 + min(j0 + R * lg + my_row, n - 1);
+            if (slot >= capacity) slot -= capacity;
+            const floatx4 *k4 = (const floatx4 *)(keys + (uint64_t)kh * HD + slot * width);
+#pragma unroll
+            for (int i = 0; i < NV; i++) {
+                const floatx4 *h4 = (const floatx4 *)(qs + (my_head + i) * HD);
+                float v = 0.0f;
+#pragma clang loop unroll(disable)
+                for (uint32_t d = 0; d < HD / 4; d++) {
+                    const floatx4 q = h4[d], k = k4[d];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v = __builtin_fmaf(q[e], k[e], v);
+                }
+                s[i] = v;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const float v = s[i];
             if (mine && my_head + i < gz) flag |= __builtin_isnan(v) || v == INFINITY;
             s[i] = mine ? v : -INFINITY;
         }

@@ -475,11 +475,12 @@ int dmhip_append_kv_device(dmhip_ctx *ctx, dmhip_kv_layer *layer, size_t positio
 /* MetalContext::attention_cached (src/metal.rs:1270-1323): one query token
    ([query_heads][head_dimension]) against the layer's last min(position,
    capacity) positions; query head h reads KV head h / (query_heads /
-   kv_heads).  Scores are unscaled fp32 fma sums (for head dimensions
+   kv_heads).  Scores are unscaled fp32 fma sums: for head dimensions
    128, 256 and 512 with up to 8 query heads per KV head in chains of 8 dims
-   added in a tree, else the sequential fma of the reference's fold: a score
-   whose partial sums pass the largest float may be finite in one order
-   only), softmax over the window, output [query_heads][head_dimension].
+   added in a tree, else, and wherever a partial sum could pass the largest
+   float, the sequential fma of the reference's fold; so the same scores are
+   non-finite as there.  Softmax over the window, output
+   [query_heads][head_dimension].
    Checks, in order: InvalidAttentionShape (heads), Overflow, InvalidAttention-
    Shape (query/output lengths), KvWidth (layer width != kv_heads *
    head_dimension), EmptyInput "attention" (position 0).  A non-finite score

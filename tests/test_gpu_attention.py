@@ -314,6 +314,51 @@ def test_non_finite_scores_are_rejected(ctx):
         b.free()
 
 
+@pytest.mark.parametrize("hd", [128, 256, 512])
+@pytest.mark.parametrize("group", [1, 2, 3, 8])
+def test_partial_sums_past_the_largest_float(ctx, hd, group):
+    """Scores whose partial sums overflow in one order of the dims and not in
+    another: accepted or refused, and weighted, as the reference's fold in
+    order of the dims has them, whatever kernel the shape takes.  Every finite
+    score here is a small whole number in every order, and the outputs are
+    whole numbers, so they are compared bit for bit."""
+    kvh, rows = 2, 9
+    width, qh, big = kvh * hd, kvh * group, np.float32(2.0 ** 125)
+    dims = np.arange(hd)
+    # +big on the first 16 dims, -big on the 16 from hd / 2 on: the fold
+    # reaches +inf (and stays), sums over both halves of a lane's dims cancel
+    first_half = np.where(dims < 16, big, np.where((dims >= hd // 2) & (dims < hd // 2 + 16), -big, 0)).astype(np.float32)
+    # +big, -big alternating every 4 dims, the same again from hd / 2 on: the
+    # fold stays at 2^127 or less, a lane's 8 dims alone pass the largest float
+    alternating = np.where(dims % (hd // 2) < 16, np.where(dims // 4 % 2 == 0, big, -big), 0).astype(np.float32)
+    edge = np.zeros(hd, np.float32)  # in front of the limit: largest products that cannot overflow
+    edge[:] = np.float32(2.0 ** 127 / hd)
+    q = np.ones(qh * hd, np.float32)
+    values = np.tile(np.arange(1, rows + 1, dtype=np.float32)[:, None], (1, width))
+    values[4] = 14  # the mean is 6 with this row, 5 without it
+    for name, row, fold in (("first half", first_half, np.inf), ("its negative", -first_half, -np.inf),
+                            ("alternating", alternating, 0.0), ("edge", edge * np.where(dims % 2, -1, 1), 0.0)):
+        print(f"hd={hd} group={group} {name}", flush=True)
+        keys = np.zeros((rows, width), np.float32)
+        keys[4, hd:] = row  # KV head 1 only
+        with np.errstate(over="ignore"):
+            acc = np.float32(0)
+            for v in row.astype(np.float32):
+                acc = np.float32(acc + v)
+        assert acc == np.float32(fold)
+        layer = ctx.new_kv_layer(width, rows, None)
+        fill_layer(ctx, layer, keys, values)
+        out = np.zeros(qh * hd, np.float32)
+        if fold == np.inf:
+            expect_error("NonFinite", ctx.attention_cached, q, layer, qh, kvh, hd, out)
+        else:
+            ctx.attention_cached(q, layer, qh, kvh, hd, out)
+            got = out.reshape(kvh, -1)
+            assert np.all(got[0] == 6.0)
+            assert np.all(got[1] == (6.0 if fold == 0.0 else 5.0)), got[1, :4]
+        layer.free()
+
+
 # ---- validation, in src/metal.rs's order ---------------------------------------------
 
 def test_new_kv_layer_checks(ctx):
