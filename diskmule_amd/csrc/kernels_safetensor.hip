@@ -72,7 +72,7 @@ __device__ __forceinline__ void st_barrier() {
 // INT8 [rows], INT4 [rows][sc] with `group` columns per scale.
 // R rows per wave step, C chunks of each row in flight per lane.
 template <uint32_t FMT, uint32_t kStRows, uint32_t kStChunks, bool PIPE>
-__global__ void __launch_bounds__(64 * kStWaves)
+__global__ void __launch_bounds__(64 * kStWaves) __attribute__((amdgpu_waves_per_eu(PIPE ? 4 : 1)))
 st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, size_t row_bytes,
                const float *__restrict__ scales, uint32_t scale_columns, uint32_t group, const float *__restrict__ x,
                float *__restrict__ y) {
@@ -81,7 +81,8 @@ st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, s
     // so a 16-byte read of 16 lanes touches all 64 banks once.  INT4: then a
     // sum per 16 columns.
     extern __shared__ __attribute__((aligned(16))) float xs[];
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = PIPE ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const uint32_t chunks = columns / E;
     // One step: kStChunks chunks of a lane in each of kStRows rows.  The
     // chunks' weights and their block / group scales are all in flight before
@@ -96,15 +97,18 @@ st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, s
         for (uint32_t r = 0; r < kStRows; r++)
 #pragma unroll
             for (uint32_t j = 0; j < kStChunks; j++) {
-                const uint32_t c = c0 + 64 * j + lane;
-                const bool ok = r0 + r < rows && c < chunks;
-                st.v[r][j] = ok ? *(const u32x4 *)(w + (size_t)(r0 + r) * row_bytes + (size_t)c * 16)
-                                : u32x4{0, 0, 0, 0};
+                // PIPE: rows and chunks past the end read the last one (and are
+                // not used), so that no load is behind a branch and the waits
+                // count them exactly; else nothing is read there.
+                uint32_t c = c0 + 64 * j + lane, row = r0 + r;
+                const bool ok = PIPE || (row < rows && c < chunks);
+                if constexpr (PIPE) c = min(c, chunks - 1), row = min(row, rows - 1);
+                st.v[r][j] = ok ? *(const u32x4 *)(w + (size_t)row * row_bytes + (size_t)c * 16) : u32x4{0, 0, 0, 0};
                 if constexpr (FMT == kStF8) {
                     // the chunk's 16 columns lie in one 128-column block
-                    st.sv[r][j][0] = ok ? scales[((r0 + r) / 128) * scale_columns + c / 8] : 0.0f;
+                    st.sv[r][j][0] = ok ? scales[(row / 128) * scale_columns + c / 8] : 0.0f;
                 } else if constexpr (FMT == kStI4) {
-                    const float *srow = scales + (size_t)(r0 + r) * scale_columns;
+                    const float *srow = scales + (size_t)row * scale_columns;
                     // group 16: a scale per half chunk; else one per chunk
                     st.sv[r][j][0] = ok ? srow[group == 16 ? 2 * c : (32 * c) / group] : 0.0f;
                     st.sv[r][j][1] = ok && group == 16 ? srow[2 * c + 1] : 0.0f;
@@ -120,13 +124,16 @@ st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, s
         // every load of a thread in flight before the first store (columns <= 16384;
         // measured at 12288 x 6144: F8 16.6 -> 15.9 us, INT8 16.3 -> 15.5 us, BF16
         // 26.2 -> 25.6 us per launch against one load in flight at a time)
-        constexpr uint32_t kXU = PIPE ? E * kStChunks / 16 : 16;
+        constexpr uint32_t kXU = PIPE ? (E * kStChunks + 15) / 16 : 16;
         const uint32_t n4 = columns / 4;
         floatx4 t[kXU];
 #pragma unroll
         for (uint32_t j = 0; j < kXU; j++) {
             const uint32_t i = j * 64 * kStWaves + threadIdx.x;
-            t[j] = i < n4 ? ((const floatx4 *)x)[i] : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            if constexpr (PIPE)
+                t[j] = ((const floatx4 *)x)[min(i, n4 - 1)];
+            else
+                t[j] = i < n4 ? ((const floatx4 *)x)[i] : floatx4{0.0f, 0.0f, 0.0f, 0.0f};
         }
         if constexpr (PIPE) {
             __builtin_amdgcn_sched_barrier(0);
@@ -228,17 +235,24 @@ st_gemv_kernel(const uint8_t *__restrict__ w, uint32_t rows, uint32_t columns, s
         }
     };
     if constexpr (PIPE) {
-        Step next;
-        for (; r0 < rows; r0 += 2 * step) {
+        // (The branches are on the wave's own row, in scalar registers, and
+        // none lies between a load and the sum before it.)
+        auto sum = [&](const Step &st) {
             float acc[kStRows] = {};
-            load(next, r0 + step, 0);
-            add(cur, 0, acc);
+            add(st, 0, acc);
             finish(r0, acc);
-            if (r0 + step >= rows) break;
-            float acc2[kStRows] = {};
-            load(cur, r0 + 2 * step, 0);
-            add(next, 0, acc2);
-            finish(r0 + step, acc2);
+        };
+        if (r0 >= rows) return;
+        Step next;
+        for (;;) {
+            if (r0 + step >= rows) return sum(cur);
+            load(next, r0 + step, 0);
+            sum(cur);
+            r0 += step;
+            if (r0 + step >= rows) return sum(next);
+            load(cur, r0 + step, 0);
+            sum(next);
+            r0 += step;
         }
     } else {
         for (; r0 < rows; r0 += step) {
@@ -311,13 +325,22 @@ hipError_t launch_st_t(hipStream_t s, int cus, const uint8_t *w, uint32_t rows, 
     // F8 18.7 against 17.0 us)
     // Rows of at most 4 chunks a lane run pipelined (a step's weights asked for
     // before the step before it is summed, the first before x is staged, every
-    // workgroup the same number of steps).  In us, without / with: 16384 x 1024
-    // F8 8.5 / 5.3, INT8 6.7 / 5.9, BF16 7.6 / 7.1; 6144 x 4096 equal (F8 7.2 /
-    // 7.3, INT8 7.4 / 7.2).  INT4 up to one chunk a lane only: 16384 x 1024
-    // 10.8 / 9.5, but 6144 x 4096 7.0 / 9.7 and 12288 x 6144 14.3 / 17.3 (174
-    // registers leave two workgroups on a CU).
-    if (columns / kStPerChunk<FMT> <= (FMT == kStI4 ? 64 : 64 * 4))
-        return launch_st_rc<FMT, 2, 4, true>(s, cus, w, rows, columns, row_bytes, scales, scale_columns, group, x, y);
+    // workgroup the same number of steps), compiled for 1, 2 and 4 chunks so
+    // that no register is held for a chunk that is never read.  In us, without
+    // / with: 16384 x 1024 F8 9.9 / 5.6, INT8 7.6 / 5.7, BF16 8.8 / 7.9; 6144 x
+    // 4096 F8 7.7 / 7.2, INT8 7.7 / 7.4; 2048 x 4096 F8 5.6 / 5.1.  INT4 up to
+    // one chunk a lane only: 16384 x 1024 11.4 / 6.3, 6144 x 2048 5.6 / 5.0;
+    // with 4 chunks its 174 registers left two workgroups on a CU, and 6144 x
+    // 4096 took 9.7 against 7.0, 12288 x 6144 17.3 against 14.3.
+    const uint32_t chunks = columns / kStPerChunk<FMT>;
+    if (chunks <= 64)
+        return launch_st_rc<FMT, 2, 1, true>(s, cus, w, rows, columns, row_bytes, scales, scale_columns, group, x, y);
+    if constexpr (FMT != kStI4) {
+        if (chunks <= 128)
+            return launch_st_rc<FMT, 2, 2, true>(s, cus, w, rows, columns, row_bytes, scales, scale_columns, group, x, y);
+        if (chunks <= 256)
+            return launch_st_rc<FMT, 2, 4, true>(s, cus, w, rows, columns, row_bytes, scales, scale_columns, group, x, y);
+    }
     return launch_st_rc<FMT, 2, 8, false>(s, cus, w, rows, columns, row_bytes, scales, scale_columns, group, x, y);
 }
 

@@ -190,6 +190,16 @@ def test_pipelined_rows_edges(ctx, fmt, rows, cols, group):
     test_seeded_parity(ctx, fmt, rows, cols, group)
 
 
+@pytest.mark.parametrize("fmt,per", [("BF16", 8), ("F8_E4M3", 16), ("I8", 16)])
+@pytest.mark.parametrize("chunks", [64, 65, 128, 129, 256])
+def test_pipelined_rows_chunk_counts(ctx, fmt, per, chunks):
+    """Rows at the edges of the forms for 1, 2 and 4 chunks a lane (`per`
+    columns a chunk): an odd row count on one step, and one past two steps of
+    1024 workgroups.  Bound: the one of the seeded cases."""
+    for rows in (13, 8193):
+        test_seeded_parity(ctx, fmt, rows, chunks * per, 0)
+
+
 def test_device_entry_point_matches_the_host_one(ctx):
     rng = np.random.default_rng(5)
     for fmt, rows, cols, group in (("F8_E4M3", 1024, 2048, 0), ("I4", 1024, 2048, 32), ("I8", 513, 2048, 0),
