@@ -44,6 +44,56 @@ constexpr bool moe_groups_by_expert(uint64_t batch, uint64_t k, uint64_t experts
     return (double)pairs * (double)expert_bytes >= 140.0 * (1 << 20) && shared * (double)expert_bytes >= 20e6;
 }
 
+// ---- decode matvecs of Q4_K and Q6_K: the int8 kernel or the fp16 one ----
+// The int8 kernel (kernels_qmv8.hip) takes each token's records through the
+// matrix cores apart and lets every wave build those of its columns, so its
+// work per block grows with the tokens and its prologue with the columns; it
+// splits K so that a launch has at least 4096 waves, 16 per CU, and a launch
+// of more than that and less than twice as many leaves part of its second
+// round empty.  The fp16 kernel (kernels_qmv.hip) costs as much for 1 token as
+// for 8, and its prologue about 2 us more.  One token: always int8; four or
+// more, and three of Q6_K: always fp16.  Between them, int8 / fp16 in us over
+// rotating matrices:
+//   Q4_K, 2 tokens
+//     up to 4096 rows, by columns: 1024 x 5120 6.1 / 6.3, x 6144 6.5 / 6.4,
+//     x 8192 8.2 / 6.5; 1536 x 7168 7.5 / 7.8, x 8192 8.3 / 7.8; 2048 x 7168
+//     7.5 / 7.9, x 8192 8.3 / 7.9; 4096 x 8192 9.3 / 11.2, x 10240 10.1 / 11.1,
+//     x 12288 12.3 / 11.6
+//     above, short rows: 12288 x 2048 6.9 / 8.5, 40960 x 1024 8.8 / 9.6, 65536
+//     x 2048 16.2 / 16.8, 6144 x 3072 7.0 / 7.6; 10240 x 3072 9.3 / 8.7
+//     4096 waves: 8192 x 5120 10.0 / 10.8, x 6144 11.9 / 11.0; 16384 x 4096
+//     10.8 / 11.4; 32768 x 6144 26.1 / 26.6, x 8192 40.1 / 33.7; beside them
+//     7168 x 5120 11.3 / 10.7, 12288 x 4096 11.4 / 10.2, 20480 x 4096 15.5 / 12.8
+//     persistent waves (above 65536 rows): 98304 x 5120 59.0 / 60.6, 151936 x
+//     6144 98.3 / 109.7, x 8192 140 / 135
+//   Q6_K, 2 tokens
+//     up to 4096 rows: 1024 x 3072 6.5 / 6.8, x 4096 7.0 / 5.7; 2048 x 5120
+//     7.9 / 9.2, x 6144 8.5 / 7.7; 4096 x 7168 10.6 / 11.5, x 8192 12.1 / 11.6,
+//     1024 x 16384 93.8 / 8.9
+//     above: 8192 x 2048 7.3 / 8.0, 12288 x 2048 9.7 / 9.8, 24576 x 1024 9.0 /
+//     9.7, 7168 x 3072 9.3 / 8.4; 28672 x 1024 11.1 / 9.6, 14336 x 2048 11.8 /
+//     9.9; of 4096 waves 16384 x 2048 9.4 / 9.9, 32768 x 1024 9.4 / 9.8, 32768
+//     x 2048 14.5 / 14.2
+//     heads: 98304 x 4096 70.5 / 69.5, 151936 x 4096 107 / 109, x 5120 131 / 137
+//   Q4_K, 3 tokens: 1024 x 2048 5.1 / 5.5, 1536 x 4096 6.9 / 7.4, x 3072 7.0 /
+//     6.4, x 1536 5.9 / 5.5, 1024 x 4096 6.9 / 5.9; 2048 x 5120 7.5 / 8.8, x 6144
+//     8.3 / 7.2; 4096 x 6144 9.1 / 9.6, x 8192 11.6 / 11.1; 8192 x 2048 7.2 / 7.3,
+//     10240 x 2048 9.5 / 8.5, 8192 x 3072 9.2 / 7.7
+constexpr bool qmv8_faster(bool q6_k, uint64_t rows, uint64_t columns, uint64_t batch) {
+    if (batch == 1) return true;
+    if (batch > 3 || (batch == 3 && q6_k)) return false;
+    // (three tokens of few rows: only where the split leaves each wave one block)
+    if (batch == 3 && rows < 2048) return (columns == 2048 && rows >= 1024) || (columns == 4096 && rows >= 1536);
+    const bool q4_pair = !q6_k && batch == 2;
+    if (rows <= 4096) return q4_pair ? columns < 4608 + 7 * rows / 4 : columns < 8192 && columns < 2304 + 7 * rows / 4;
+    const uint64_t tiles = (rows + 15) / 16, weights = rows * columns, m = 1u << 20;
+    const bool whole = tiles > 4096 || 4096 % tiles == 0;  // whole rounds of waves
+    if (q4_pair)
+        return columns <= 2048 || (columns <= 3072 && rows <= 8192) || (whole && columns <= (rows > 16384 ? 6144 : 5120));
+    if (batch == 3) return columns <= 2048 && weights <= 16 * m;
+    return (columns <= 2048 && weights <= (whole ? 32 : 24) * m) || (columns <= 8192 && weights > 300 * m);
+}
+
 // ---- the fp16 matvec (kernels_qmv.hip) ----
 struct QmvPlan {
     uint32_t kb, waves, wave_k, k_parts, row_groups, phases;

@@ -32,6 +32,7 @@
 // go through a per-wave LDS staging area so that the global loads are fully
 // coalesced.
 #include "dm_device.h"
+#include "dm_plan.h"
 #include "dm_qmv.h"
 
 
@@ -1270,24 +1271,8 @@ hipError_t launch8(dmhip_ctx *ctx, uint32_t batch, int mode, const Args8 &a) {
 bool qmv8_supported(uint32_t type, size_t rows, size_t columns, size_t batch) {
     if (type != kQ4_K && type != kQ6_K && type != kQ8_0) return false;
     if (batch < 1 || batch > kMaxTokens8 || columns % 256 || columns == 0) return false;
-    // Q4_K / Q6_K of several tokens: the int8 kernel against the fp16 one,
-    // measured per launch on MI355X.  The int8 kernel takes each token's
-    // records through the matrix cores apart, so its work per block grows with
-    // the tokens; the fp16 one costs as much for 1 token as for 8, and its
-    // prologue about 2 us more.
-    //  2 tokens: Q4_K 4096 x 5120 6.5 against 9.1 us, 6144 x 4096 9.6 against
-    //    8.5, 20000 x 4096 15.3 against 12.7, 32768 x 4096 16.0 against 16.7;
-    //    Q6_K 4096 x 5120 8.5 against 9.5, 8192 x 4096 11.8 against 9.7,
-    //    32768 x 4096 29.8 against 25.9, 151936 x 4096 103 against 112.
-    //  3 tokens: Q4_K 4096 x 4096 6.8 against 7.1, 1024 x 4096 6.6 against
-    //    5.2; Q6_K 4096 x 4096 8.7 against 7.5.
-    // From 4 tokens on the fp16 kernel is faster throughout.
-    if (type != kQ8_0) {
-        const uint64_t weights = (uint64_t)rows * columns, m = 1u << 20;
-        if (batch > 3) return false;
-        if (batch == 3 && (type == kQ6_K || rows < 2048 || weights > 20 * m)) return false;
-        if (batch == 2 && weights > 22 * m && weights <= (type == kQ4_K ? 100 * m : 300 * m)) return false;
-    }
+    // (Q8_0 has only this kernel)
+    if (type != kQ8_0 && !qmv8_faster(type == kQ6_K, rows, columns, batch)) return false;
     return plan8(type, (uint32_t)rows, (uint32_t)columns, (uint32_t)batch, 1).s != 0;
 }
 

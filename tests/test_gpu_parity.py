@@ -264,6 +264,18 @@ def test_batched_gemv_plans(ctx, kind, rows, cols, batch):
     assert_channel_close(got[:, pick], exact, scale, CHANNEL_TOL_GEMV, f"type {kind} {rows}x{cols} batch {batch}")
 
 
+@pytest.mark.parametrize("kind,rows,cols,batch", [
+    (Q4_K, 4090, 10240, 2), (Q4_K, 12300, 2048, 2), (Q4_K, 8192, 5120, 2),  # int8: long rows, short rows, whole rounds
+    (Q6_K, 16384, 2048, 2), (Q4_K, 4096, 6144, 3),
+    (Q4_K, 1000, 6144, 2), (Q6_K, 1000, 4096, 2), (Q6_K, 500, 16384, 2), (Q4_K, 2050, 6144, 3),  # fp16: small, long rows
+    (Q4_K, 6200, 4096, 2), (Q6_K, 7000, 3072, 2)])
+def test_two_and_three_token_matvecs_at_the_rule_between_the_kernels(ctx, kind, rows, cols, batch):
+    """Both sides of the lines between the int8 and the fp16 kernel at 2 and 3
+    tokens: the checks of the fp16 matvec's plans."""
+    print(f"type={kind} {rows}x{cols} batch={batch}", flush=True)
+    test_batched_gemv_plans(ctx, kind, rows, cols, batch)
+
+
 @pytest.mark.parametrize("hidden,ffn,batch", [(2048, 530, 3), (5120, 300, 8), (7168, 200, 4), (4096, 2100, 16),
                                               (5120, 700, 12)])
 def test_batched_ffn_plans(ctx, hidden, ffn, batch):

@@ -22,6 +22,9 @@ void qmv_plan(uint32_t rows, uint32_t blocks, uint32_t batch, int mode, uint32_t
 int moe_groups_by_expert(uint64_t batch, uint64_t k, uint64_t experts, uint64_t bytes) {
     return dm::moe_groups_by_expert(batch, k, experts, bytes, 64);
 }
+int qmv8_faster(int q6_k, uint64_t rows, uint64_t columns, uint64_t batch) {
+    return dm::qmv8_faster(q6_k, rows, columns, batch);
+}
 uint64_t gemm_prep_lds(uint64_t k) { return dm::gemm_prep_lds(k); }
 int gemm_fits_mfma(uint64_t m, uint64_t n, uint64_t k, uint64_t w_bytes) { return dm::gemm_fits_mfma(m, n, k, w_bytes); }
 int qmv_runs_fit(uint32_t blocks, uint32_t batch, int mode) { return dm::qmv_runs_fit(blocks, batch, mode); }
@@ -49,6 +52,7 @@ def plan(tmp_path_factory):
     lib = ctypes.CDLL(str(d / "shim.so"))
     for name in ("experts_grid", "experts_share"):
         getattr(lib, name).restype = ctypes.c_uint32
+    lib.qmv8_faster.argtypes = [ctypes.c_int] + [ctypes.c_uint64] * 3
     lib.gemm_prep_lds.restype = ctypes.c_uint64
     lib.gemm_prep_lds.argtypes = [ctypes.c_uint64]
     lib.moe_groups_by_expert.argtypes = [ctypes.c_uint64] * 4
@@ -87,6 +91,26 @@ def test_tokens_are_grouped_by_expert_only_where_they_share(plan):
             ((4096, 1024), 64, 8, 3, True), ((6144, 2048), 16, 8, 1, False), ((6144, 2048), 16, 8, 3, True),
             ((1024, 512), 32, 8, 8, False)):
         assert bool(plan.moe_groups_by_expert(batch, k, experts, size[shape])) == grouped, (shape, experts, k, batch)
+
+
+def test_matvecs_of_two_and_three_tokens_take_the_faster_kernel(plan):
+    """Shapes measured on both kernels, on either side of every line of the
+    rule: long rows leave the int8 kernel also where the matrix is small, short
+    rows keep it also where it is large."""
+    q4, q6 = 0, 1
+    int8 = [(q4, 1024, 5120, 2), (q4, 1536, 7168, 2), (q4, 2048, 7168, 2), (q4, 4096, 8192, 2),
+            (q4, 12288, 2048, 2), (q4, 32768, 1024, 2), (q4, 6144, 3072, 2), (q4, 8192, 5120, 2), (q4, 32768, 6144, 2), (q4, 151936, 4096, 2),
+            (q6, 1024, 3072, 2), (q6, 2048, 5120, 2), (q6, 4096, 7168, 2), (q6, 24576, 1024, 2), (q6, 16384, 2048, 2),
+            (q6, 151936, 5120, 2), (q4, 1024, 2048, 3), (q4, 1536, 4096, 3),
+            (q4, 2048, 5120, 3), (q4, 4096, 6144, 3), (q4, 8192, 2048, 3)]
+    fp16 = [(q4, 1024, 8192, 2), (q4, 2048, 8192, 2), (q4, 4096, 12288, 2), (q4, 6144, 4096, 2), (q4, 12288, 4096, 2),
+            (q4, 8192, 8192, 2), (q4, 32768, 8192, 2), (q6, 1024, 4096, 2), (q6, 4096, 8192, 2), (q6, 1024, 16384, 2),
+            (q6, 7168, 3072, 2), (q6, 32768, 2048, 2), (q6, 32768, 16384, 2), (q4, 1024, 4096, 3), (q4, 1536, 3072, 3),
+            (q4, 4096, 8192, 3), (q4, 8192, 3072, 3), (q6, 4096, 4096, 3), (q4, 4096, 4096, 4), (q6, 4096, 4096, 4)]
+    assert all(plan.qmv8_faster(*case) for case in int8), [c for c in int8 if not plan.qmv8_faster(*c)]
+    assert not any(plan.qmv8_faster(*case) for case in fp16), [c for c in fp16 if plan.qmv8_faster(*c)]
+    assert all(plan.qmv8_faster(q, rows, columns, 1) for q in (q4, q6) for rows in (1, 16, 5000, 151936)
+               for columns in (256, 4096, 65536))
 
 
 BLOCKS = [*range(1, 70), 95, 96, 97, 112, 127, 128, 129, 208, 256, 257, 512, 1000, 4096, 65535, 65536, 92681, 92682,
