@@ -76,8 +76,9 @@ int enqueue_matvec(dmhip_ctx *ctx, uint32_t type, size_t rows, size_t columns, c
 int enqueue_matvec_argmax(dmhip_ctx *ctx, uint32_t type, size_t rows, size_t columns,
                           const void *w, const float *x, float *y, uint32_t *index_device) {
     if (qmv_supported(type, rows, columns, w, 1)) {
-        // Two launches: the activation pass resets the argmax state and the
-        // matvec folds the argmax into its epilogue and publishes the index.
+        // One launch: the int8 kernel folds the argmax into its epilogue and
+        // its last workgroup publishes the index.  (Rows too long for its
+        // LDS: the fp16 kernel, then the argmax launches.)
         DM_HIP(launch_qmv(ctx, type, (uint32_t)rows, (uint32_t)columns, w, 1, x, y,
                           ctx->argmax_state, index_device));
         return DMHIP_OK;
@@ -118,14 +119,15 @@ int dmhip_ffn_device_noalloc(dmhip_ctx *ctx, size_t batch, size_t hidden, size_t
         return fail(DMHIP_ERR_INVALID_ARGUMENT, "batch %zu is outside 1..=16", batch);
     const size_t ws = dmhip_ffn_workspace_bytes(batch, hidden, ffn);
     // batches above 2 are accepted up to the scratch that their activations as
-    // fp16 pairs take: h (gate and up, whose types may differ) or the
-    // activation rows (down), the largest of the three
+    // fp16 pairs would take beside the workspace: h (gate and up, whose types
+    // may differ) or the activation rows (down), the largest of the three.  A
+    // limit only: nothing is stored there
     size_t lend = 0;
     if (batch > 2) {
         const uint32_t types[3] = {gate_type, up_type, down_type};
         const size_t cols[3] = {hidden, hidden, ffn};
         for (int i = 0; i < 3; i++) {
-            const size_t b = qmv_prepare_bytes(types[i], cols[i], batch);
+            const size_t b = qmv_noalloc_bytes(types[i], cols[i], batch);
             lend = b > lend ? b : lend;
         }
     }

@@ -25,9 +25,10 @@ struct ArgmaxFinish {
     unsigned long long *best;
 };
 
-// True when the int8-MFMA matvec (decode batches of 1-4 tokens, Q4_K/Q6_K/
-// Q8_0, whose activation records fit the workgroup's LDS) takes this shape;
-// the caller has already checked qmv_supported.
+// True when the int8-MFMA matvec takes this shape: 1-4 tokens of Q8_0, 1 token
+// of Q4_K and Q6_K and 2-3 where it is the faster kernel (qmv8_faster), whose
+// activation records fit the workgroup's LDS; the caller has already checked
+// qmv_supported.
 bool qmv8_supported(uint32_t type, size_t rows, size_t columns, size_t batch);
 
 // y[b][r] = W[r] . x[b] with the int8-MFMA kernels.  With `partials` the
@@ -63,9 +64,6 @@ struct QmvJob {
 // Q4_K) and hold whole rows.
 bool qmv8_grouped_supported(uint32_t type, size_t rows, size_t columns, uint32_t mats);
 
-// All jobs in one or a few launches.  gate_up == 0: y = W x.  gate_up == 1:
-// y = (g / (1 + exp(-g))) * u with g = gate . x, u = up . x, the routed-expert
-// activation of src/glm52/expert.rs:260-267.
 // The ordered combine of each token's experts fused into their down launch:
 // jobs t * k .. t * k + k - 1 are token t's selections, and
 // y_final[t * y_stride + r] = sum over them in order of
@@ -79,6 +77,9 @@ struct QmvCombine {
     uint32_t k, y_stride;
 };
 
+// All jobs in one or a few launches.  gate_up == 0: y = W x.  gate_up == 1:
+// y = (g / (1 + exp(-g))) * u with g = gate . x, u = up . x, the routed-expert
+// activation of src/glm52/expert.rs:260-267.
 // With dev_w (one-token jobs, at most 64, one launch) the job addresses are
 // read on the device from dev_w[job] and the launch does nothing unless
 // go[0 .. go_count) are all 1: both written by a kernel earlier on the
@@ -92,7 +93,8 @@ hipError_t launch_qmv8_grouped(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uin
 // True when the MFMA matvec takes this shape: Q4_K or Q6_K rows of whole
 // 256-value blocks, a weight base address aligned to 4 bytes (16 for Q4_K),
 // and fewer than 4 GiB of weights (one buffer descriptor); or Q8_0 rows of
-// whole 256-value super-blocks at a 16-byte aligned base, batch 1-2.
+// whole 256-value super-blocks at a 16-byte aligned base, 1-4 tokens whose
+// records fit.
 bool qmv_supported(uint32_t type, size_t rows, size_t columns, const void *w, size_t batch);
 
 // The routed experts of a layer call on the fp16 kernel, their tokens grouped
@@ -108,7 +110,7 @@ hipError_t launch_qmv_experts(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uint
 
 // The scratch that the allocation-free entry point reckons per batch above 2 of
 // rows of `columns` values when it accepts or rejects a shape.
-size_t qmv_prepare_bytes(uint32_t type, size_t columns, size_t batch);
+size_t qmv_noalloc_bytes(uint32_t type, size_t columns, size_t batch);
 
 // y[b][r] = W[r] . x[b]; when `argmax` is non-null (batch 1) the kernels
 // also reset `argmax`, fold a greedy argmax over the rows into it and write

@@ -101,8 +101,8 @@ __device__ __forceinline__ half2_t magic_hi(uint32_t v) {
     return __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u));
 }
 
-// Workgroup barrier ordering LDS only: the wave's global loads in flight
-// (the next tile's W and A) are not waited for, as __syncthreads() would.
+// Workgroup barrier ordering LDS only: global loads and stores in flight are
+// not waited for, as __syncthreads() would.
 __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();

@@ -107,7 +107,6 @@ template <uint32_t TYPE> constexpr uint32_t quad_half(uint32_t r, uint32_t c) {
     return TYPE == kQ4_K ? r >> 1 : c & 1u;
 }
 
-typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // x may be 4-byte aligned
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 template <int CTRL>
@@ -1051,8 +1050,10 @@ hipError_t dispatch(dmhip_ctx *ctx, uint32_t rows, uint32_t columns, const void 
     if (p.phases > 1)
         return batch <= 8 ? run<TYPE, 1, MODE, 2, 8, true>(ctx, p, a) : run<TYPE, 2, MODE, 2, 8, true>(ctx, p, a);
     if (batch > 8) return p.kb == 1 ? run<TYPE, 2, MODE, 1, 8>(ctx, p, a) : run<TYPE, 2, MODE, 2, 8>(ctx, p, a);
-    if (p.waves == 8) return run<TYPE, 1, MODE, 3, 8>(ctx, p, a);
-    if constexpr (MODE == 0) {
+    // (16 waves; a gate/up pair, which holds a block per wave there, has 8 of 3 blocks besides)
+    if constexpr (MODE == 2) {
+        if (p.waves == 8) return run<TYPE, 1, MODE, 3, 8>(ctx, p, a);
+    } else {
         if (p.kb == 2) return run<TYPE, 1, MODE, 2, 16>(ctx, p, a);
     }
     return run<TYPE, 1, MODE, 1, 16>(ctx, p, a);
@@ -1112,9 +1113,11 @@ hipError_t launch_qmv_experts(dmhip_ctx *ctx, uint32_t type, uint32_t rows, uint
                          : dispatch_experts<kQ6_K, 0>(ctx, rows, columns, x, y, ex);
 }
 
-// What an allocation-free call sets aside for a matrix (the activation
-// fragments of the documented limit; the K-split partials use it).
-size_t qmv_prepare_bytes(uint32_t type, size_t columns, size_t batch) {
+// The activations of a batch as fp16 fragments in memory.  No launch stores
+// them there (they are built in registers, and the K-split partials go to
+// ctx->qmv_meet): it is the allocation-free entry point's limit on a shape,
+// kept so that it accepts and rejects the same ones.
+size_t qmv_noalloc_bytes(uint32_t type, size_t columns, size_t batch) {
     const size_t spb = type == kQ4_K ? 9 : 8;
     const size_t xp_bytes = (columns / 256) * spb * 4 * 2 * batch * 8 * sizeof(_Float16);
     return ((xp_bytes + 255) & ~(size_t)255) + 64 * sizeof(float);
