@@ -74,6 +74,24 @@ CHANNEL_TOL_GEMV = 1e-4
 CHANNEL_TOL_GEMM = 2e-3
 
 
+# Chains of products (a gated FFN, a routed-expert layer) have no S_i of their
+# own: their bar is the relative 2-norm of a token's output against the
+# oracle's sequential fp32 fold.  Random roundings: the fold of n terms is off
+# by about 2^-24 sqrt(n / 2) of its result (4.7e-6 at 12288), rounding an
+# activation at 2^-22 of a block's or token's largest (about 4 times its rms)
+# by 2^-22 * 4 / sqrt(12) = 3e-7, a fp32 sigmoid or norm by less; two products
+# in a row and a factor of two above their sum: 2e-5.  Losing the low half of
+# the fp16 pairs (2^-12) or a scale's low bits shows at 1e-4 and more.
+NORM_TOL = 2e-5
+
+
+def assert_norm_close(a, r, what=""):
+    a, r = np.asarray(a, dtype=np.float64), np.asarray(r, dtype=np.float64)
+    e = float(np.linalg.norm(a - r) / np.linalg.norm(r))
+    assert e <= NORM_TOL, f"{what}: 2-norm error {e:.3e} (bar {NORM_TOL:.1e})"
+    return e
+
+
 def dense_rows(kind, rows, cols, w, first=0, count=None):
     """float64 [count][cols] dequantization of rows first.. of an encoded
     matrix (the oracle's decoders, bit-exact with the reference's)."""
