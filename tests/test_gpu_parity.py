@@ -189,8 +189,8 @@ def test_decode_gemv_matches_oracle(ctx, kind, rows, cols, cfg):
 
 @pytest.mark.parametrize("batch", [2, 3, 4, 8, 9, 16])
 def test_batched_gemv_matches_oracle(ctx, batch):
-    """Batches 1-4 take the int8 kernel at this size (records of every token
-    in LDS), larger ones the fp16 kernel."""
+    """Two tokens take the int8 kernel at this size (records of every token in
+    LDS), larger batches the fp16 kernel."""
     rows, cols = 1000, 2048
     for kind in (Q4_K, Q6_K):
         w = synth.quantized_matrix(kind, rows, cols, synth.weight_seed(40 + batch))
@@ -210,16 +210,18 @@ def test_batched_gemv_matches_oracle(ctx, batch):
     (Q6_K, 2048, 768, 4),    # 630-byte rows (every other row 2 bytes off a dword), odd block count
     (Q6_K, 300, 12288, 8),   # short and wide: K split over 8 waves, partial last tile
     (Q4_K, 100, 12288, 12),  # two token groups, partial tile
-    (Q4_K, 4096, 12288, 3),  # fp16: above the size the int8 kernel takes 3-4 tokens for
-    (Q4_K, 1000, 12288, 3),  # int8: three tokens' records of 48 blocks (117 KB of LDS)
+    (Q4_K, 4096, 12288, 3),  # fp16: rows too long for the int8 kernel at three tokens
+    (Q4_K, 1000, 12288, 3),
+    (Q4_K, 3001, 7424, 3),   # int8: three tokens' records of 29 blocks, partial last tile
     (Q6_K, 1000, 2560, 5),   # 10 blocks: partial last pair of a split
-    (Q6_K, 300, 12288, 4),   # records too large for LDS: the fp16 kernel at 4 tokens
-    (Q4_K, 70, 4096, 4),     # int8, 4 tokens, partial last tile
+    (Q6_K, 300, 12288, 4),   # short and wide at 4 tokens
+    (Q4_K, 70, 4096, 4),     # 4 tokens, partial last tile
+    (Q4_K, 1038, 2048, 3),   # int8: a wave per block, partial last tile
 ])
 def test_batched_gemv_short_and_misaligned_shapes(ctx, kind, rows, cols, batch):
-    """Batches above 2 on the int8 kernel (1-4 tokens whose records fit the
-    LDS: misaligned 630-byte Q6_K rows, wide rows) and on the fp16 kernel's
-    wide K split and partial block pairs."""
+    """Batches above 2 on the fp16 kernel (misaligned 630-byte Q6_K rows, wide K
+    splits, partial block pairs) and, for three tokens of Q4_K whose rows are
+    not too long, on the int8 kernel."""
     print(f"batched gemv type={kind} {rows}x{cols} batch={batch}", flush=True)
     w = synth.quantized_matrix(kind, rows, cols, synth.weight_seed(90 + batch))
     x = synth.normal(synth.activation_seed(90 + batch), batch * cols).reshape(batch, cols)
@@ -361,16 +363,16 @@ def _int8_record_bound(kind, rows, cols, w, x):
 
 
 def _fp16_pair_bound(kind, rows, cols, w, x):
-    """The fp16 path's worst-case error per output row (batches 3-16): the
-    token is scaled by one power of two so max|x| 2^-e lies in [2^14, 2^15)
-    and split into fp16 hi + lo, so |x~ - x| <= 2^-22 |x| (two roundings of
-    half an fp16 ulp) + 2^-39 max|x| (lo below fp16's normal range).  Q4_K's
-    dmin m sum(x) term takes 32-column sums in fp32 (at most 31 roundings,
-    2^-19 of sum|x|) before the same split, and dmin m <= 63 dmin bounds its
-    factor.  The fp32 noise term is the one of the int8 bound."""
+    """The fp16 path's worst-case error per output row (batches 3-16): each
+    256-value block is scaled by a power of two so max|x| 2^-e lies in [2^14,
+    2^15) and split into fp16 hi + lo, so |x~ - x| <= 2^-22 |x| (two roundings
+    of half an fp16 ulp) + 2^-39 of the block's max|x| (lo below fp16's normal
+    range).  Q4_K's dmin m sum(x) term takes 32-column sums in fp32 (at most 31
+    roundings, 2^-19 of sum|x|) before the same split, and dmin m <= 63 dmin
+    bounds its factor.  The fp32 noise term is the one of the int8 bound."""
     dense = capi.dequantize(kind, w, rows * cols).reshape(rows, cols).astype(np.float64)
     ax = np.abs(x.astype(np.float64))
-    per_x = 2.0 ** -22 * ax + 2.0 ** -39 * ax.max()
+    per_x = 2.0 ** -22 * ax + 2.0 ** -39 * np.repeat(ax.reshape(-1, 256).max(axis=1), 256)
     bound = np.abs(dense) @ per_x
     if kind == Q4_K:
         blocks = w.reshape(rows, cols // 256, 144)
@@ -387,9 +389,9 @@ def _fp16_pair_bound(kind, rows, cols, w, x):
                                                  (Q4_K, 4096, 12288, 6)])
 def test_in_block_outliers_stay_within_the_bound(ctx, kind, rows, cols, batch):
     """One element 10^4 times its neighbours inside each 256-value block, and
-    blocks 10^4 smaller than the rest: batches of 1-4 tokens take the int8
-    records (22 bits per block), batches 6 and 8 the fp16 path (22 bits per
-    token); each is checked against the bound derived for its path, and the
+    blocks 10^4 smaller than the rest: batches of 1 and 2 tokens take the int8
+    records, batches of 4 and more the fp16 pairs (22 bits per block, both);
+    each is checked against the bound derived for its path, and the
     tolerance."""
     print(f"outliers type={kind} {rows}x{cols} batch={batch}", flush=True)
     w = synth.quantized_matrix(kind, rows, cols, synth.weight_seed(130, kind))
@@ -400,7 +402,7 @@ def test_in_block_outliers_stay_within_the_bound(ctx, kind, rows, cols, batch):
     got = yb.read(0, batch * rows * 4, np.float32).reshape(batch, rows)
     for b in range(batch):
         e, _ = assert_close(got[b], want[b], f"outliers type {kind} token {b}")
-        if batch <= 4:
+        if batch <= 2:
             bound = _int8_record_bound(kind, rows, cols, w, x[b])
         else:
             bound = _fp16_pair_bound(kind, rows, cols, w, x[b])
@@ -482,8 +484,9 @@ def _small_scale_matrix(kind, rows, cols, seed):
 @pytest.mark.parametrize("batch", [1, 2, 4, 8])
 def test_small_scale_blocks_gemv(ctx, kind, batch):
     """Super-block scales in fp16's subnormal range beside ordinary rows: the
-    int8 records (batch 1-4) and the fp16 pairs (batch 8) keep every output
-    channel within the per-channel bar, not only the vector-wide one."""
+    int8 records (batches 1 and 2; every batch of Q8_0) and the fp16 pairs
+    (batches 4 and 8) keep every output channel within the
+    per-channel bar, not only the vector-wide one."""
     rows, cols = 4096, 4096
     w = _small_scale_matrix(kind, rows, cols, synth.weight_seed(150, kind))
     x = synth.normal(synth.activation_seed(150, batch), batch * cols).reshape(batch, cols)
@@ -754,7 +757,7 @@ def test_argmax_top_k_rms_norm_silu(ctx, golden):
 def test_dense_ffn_matches_oracle(ctx, batch):
     """Config 3.  Batch 1-2 runs the int8 gate/up kernel with RMSNorm folded
     into its activation scale, batches 3-8 the fp16 one; the down projection
-    (12288 columns) is int8 for 1-2 tokens and fp16 above."""
+    (12288 columns) is int8 for 1 token and fp16 above."""
     hidden, ffn = 4096, 12288
     print(f"C3 batch={batch}", flush=True)
     g = synth.quantized_matrix(Q4_K, ffn, hidden, synth.weight_seed(3, 0))
