@@ -470,7 +470,7 @@ def bench_c5(ctx, synth, steps, warmup):
     """C5: 512-token prefill GEMM at K = 4096, N = 4096 and 12288, for Q4_K
     (the headline) and the other two quantized types of the path.  `ms` is
     the whole call (A preparation + GEMM); the GEMM kernel alone is in the
-    kernel trace of profiles/c5_gemm_kernel_stats.md."""
+    kernel trace of profiles/c5_prefill_gemm_kernel_stats.md."""
     m, k = 512, 4096
     a = synth.to_bf16_bits(synth.normal(synth.activation_seed(5), m * k))
     ab = upload(ctx, a)
